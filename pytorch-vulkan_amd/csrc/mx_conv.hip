@@ -580,20 +580,24 @@ int select_algo_heuristic(const mx_conv2d_desc& d, int phase, int requested, int
   }
 }
 
-// Per-tile figures for the planners: rows, columns, workgroups resident per
-// CU, and the CU's MFMA throughput with a full set of such tiles, relative to
-// 85% of its FP32 peak.  The rates (and the constants of plan_cost) were
-// fitted to measured times of every (tile, split) plan on the 53 ResNet-50
-// layers (forward, dInput, dWeight) on MI355X: the fitted planner's choices
-// cost 1.5% more in total than the best measured plan per layer.
-struct TileInfo {
-  int bm, bn, per_cu;
+// Per-tile figures for the planners: rows, columns, and per phase kind
+// (forward / dInput, dWeight) the workgroups resident per CU and the CU's
+// throughput with a full set of such tiles, relative to 85% of its FP32 MFMA
+// peak (the split bf16 product passes 1).  Fitted with the constants of
+// plan_cost to measured times of every (tile, split) plan on MI355X.
+struct TileRate {
+  int per_cu;
   double rate;
+};
+struct TileInfo {
+  int bm, bn;
+  TileRate fwd, dw;
   const char* name;
 };
 constexpr TileInfo kTileInfo[conv::NTILES] = {
-    {256, 128, 2, 1.20, "256x128x16"}, {128, 256, 2, 1.22, "128x256x16"}, {128, 128, 2, 1.15, "128x128x16"},
-    {64, 256, 2, 0.68, "64x256x16"},   {256, 64, 2, 0.76, "256x64x16"},   {64, 64, 4, 1.10, "64x64x32"}};
+    {256, 128, {2, 1.81}, {2, 1.60}, "256x128x16"}, {128, 256, {2, 1.60}, {2, 1.60}, "128x256x16"},
+    {128, 128, {2, 1.60}, {2, 1.50}, "128x128x16"}, {64, 256, {2, 1.07}, {2, 1.40}, "64x256x16"},
+    {256, 64, {2, 1.00}, {2, 1.45}, "256x64x16"},   {64, 64, {5, 1.26}, {3, 1.13}, "64x64x32"}};
 
 // Kernel tag of a tile for a phase: forward and dInput compile the small tile
 // with 16-deep slabs (conv::TileSmallShallow).
@@ -603,24 +607,26 @@ const char* tile_name(int tile, int phase) {
 
 // Estimated time of one implicit GEMM (per group M x Ncols x K, G groups)
 // with tile `ti` and K split `splits` ways of kps each, plus the finalize pass
-// that sums the partial outputs.  A CU holding n tiles runs at
-// rate * occ(n) of its share of 85% of the FP32 MFMA peak, occ rising from
-// 0.75 with one resident tile to 1 with per_cu; tiles beyond that queue.  The
-// finalize moves (splits + 1) outputs' bytes at an effective 3.1 TB/s.  The
-// two constants were fitted on MI355X to every (tile, split) plan of 83
-// layer phases (C3's implicit-GEMM layers and the small C1 / C4 layers, each
-// plan forced and timed): the planner's picks sum to 0.1-0.4% above the
-// best plan per layer on C3 and 1.5-1.6% on the small layers, against 0.5%
-// and 8.9% with the earlier 0.56 and 8 TB/s.
-double plan_cost(const TileInfo& ti, int64_t M, int64_t Ncols, int64_t G, int64_t splits, int64_t kps,
+// that sums the partial outputs.  A CU holding n tiles runs at rate * occ(n)
+// of its share of 85% of the FP32 MFMA peak, occ rising from 0.71 with one
+// resident tile to 1 with per_cu; tiles beyond that queue.  A tile's first
+// loads and its stores cost it as much as 41 more k.  The finalize moves
+// (splits + 1) outputs' bytes at an effective 3.6 TB/s.  The constants were
+// fitted on MI355X to every (tile, split) plan of 110 layer phases (the
+// 53 ResNet-50 layers at batch 64, small U-Net layers, odd sizes), each plan
+// forced and timed: the planner's picks sum to 0.7% above the best plan per
+// phase on phases over 40 us and 0.9% on the shorter ones, where the figures
+// that fitted the FP32 products were 10.2% and 1.5% above.
+double plan_cost(const TileInfo& ti, bool dweight, int64_t M, int64_t Ncols, int64_t G, int64_t splits, int64_t kps,
                  int64_t out_elems) {
+  const TileRate& tr = dweight ? ti.dw : ti.fwd;
   const double cu = cu_count();
   const double cu_flops = 0.85 * 157.3e12 / 256.0;
   const int64_t tiles = ((M + ti.bm - 1) / ti.bm) * ((Ncols + ti.bn - 1) / ti.bn) * G;
   const int64_t per_cu = (tiles * splits + int64_t(cu) - 1) / int64_t(cu);
-  const double occ = std::min(1.0, 0.75 + 0.25 * double(per_cu - 1) / double(ti.per_cu - 1));
-  double t = double(per_cu) * 2.0 * ti.bm * ti.bn * double(kps) / (cu_flops * ti.rate * occ) + 2e-6;
-  if (splits > 1) t += double(splits + 1) * double(out_elems) * 4.0 / 3.1e12 + 3e-6;
+  const double occ = std::min(1.0, 0.71 + 0.29 * double(per_cu - 1) / double(tr.per_cu - 1));
+  double t = double(per_cu) * 2.0 * ti.bm * ti.bn * (double(kps) + 41.0) / (cu_flops * tr.rate * occ) + 2e-6;
+  if (splits > 1) t += double(splits + 1) * double(out_elems) * 4.0 / 3.6e12 + 3e-6;
   return t;
 }
 
@@ -642,7 +648,7 @@ struct GemmPlan {
 // diagnosis); a forced split for which the budget holds no split at all is an
 // error, as a forced algorithm beyond the budget is in
 // csrc/ops/convolution.cpp:472-473.
-int plan_gemm(int64_t M, int64_t Ncols, int64_t K, int64_t G, unsigned tiles, int64_t max_splits,
+int plan_gemm(bool dweight, int64_t M, int64_t Ncols, int64_t K, int64_t G, unsigned tiles, int64_t max_splits,
               int64_t out_elems, int64_t ws_per_split, int64_t ws_limit, GemmPlan* out) {
   int force_tile = -1, force_splits = 0;
   if (const char* e = std::getenv("MX_CONV_PLAN")) {
@@ -666,7 +672,7 @@ int plan_gemm(int64_t M, int64_t Ncols, int64_t K, int64_t G, unsigned tiles, in
         budget_stop = true;
         break;
       }
-      const double cost = plan_cost(kTileInfo[t], M, Ncols, G, splits, kps, out_elems);
+      const double cost = plan_cost(kTileInfo[t], dweight, M, Ncols, G, splits, kps, out_elems);
       if (force_tile >= 0 || best_t < 0 || cost < best_t) {  // forced: the largest split that fits
         best_t = cost;
         best.tile = t;
@@ -725,7 +731,7 @@ int plan_forward(const mx_conv2d_desc& d, const float* x, const float* w, const 
   f->padded = !f->packed && (p.K % 4 != 0 || !aligned16(w));
   f->bmode = (unpadded_1x1(p) && p.HW % 4 == 0 && aligned16(x)) ? conv::B_VEC : conv::B_GATHER;
   p.out_elems = int64_t(p.N) * p.Cout * p.OHOW;
-  MX_TRY(plan_gemm(p.Cout_g, int64_t(p.N) * p.OHOW, int64_t(p.Cin_g) * p.KK, p.G, knob_tiles(d, kSinglePassTiles), 512,
+  MX_TRY(plan_gemm(false, p.Cout_g, int64_t(p.N) * p.OHOW, int64_t(p.Cin_g) * p.KK, p.G, knob_tiles(d, kSinglePassTiles), 512,
                    p.out_elems, p.out_elems * 4, ws_limit, &f->gp));
   p.splits = f->gp.splits;
   p.kps = f->gp.kps;
@@ -828,7 +834,7 @@ int plan_dinput(const mx_conv2d_desc& d, const float* dy, const float* w, float*
     }
   }
   f->out_elems = int64_t(p.N) * p.Cin * p.HW;
-  MX_TRY(plan_gemm(bm, bn, std::max<int64_t>(bk, 1), p.G, knob_tiles(d, kSinglePassTiles), f->any_zero ? 1 : 512,
+  MX_TRY(plan_gemm(false, bm, bn, std::max<int64_t>(bk, 1), p.G, knob_tiles(d, kSinglePassTiles), f->any_zero ? 1 : 512,
                    f->out_elems, f->out_elems * 4, ws_limit, &f->gp));
   // A 1x1 kernel is already [g][co][ci]; larger kernels are packed per phase.
   f->packed = p.KK > 1;
@@ -892,8 +898,8 @@ struct DwPlan {
 // writes one full-size partial dW (and a dBias partial) that the finalize
 // re-reads.  The x operand is the column gather unless the kernel is an
 // unpadded 1x1 stride-1 one with 4-aligned planes; dy is read as scalar rows
-// when OH*OW % 4 != 0.  Gathers over 256 columns (and a 256-wide tile with
-// both gathers) are not built.
+// when OH*OW % 4 != 0.  Column gathers run on tiles up to 128x128 and 256x64,
+// scalar dy rows on all but the 256x128 and 128x256 tiles.
 int plan_dweight(const mx_conv2d_desc& d, const float* x, const float* dy, float* dw, float* db, int64_t ws_limit,
                  DwPlan* f) {
   ConvArgs& p = f->p;
@@ -912,10 +918,10 @@ int plan_dweight(const mx_conv2d_desc& d, const float* x, const float* dy, float
   p.cols_blocked = f->bmode == conv::B_GATHER && conv::blocked_channels(p.Cin_g) ? 1 : 0;
   const int64_t out = int64_t(p.G) * p.Cout_g * p.Ncols;
   unsigned tiles = kAllTiles;
-  if (f->bmode == conv::B_GATHER) tiles &= ~((1u << conv::WIDE) | (1u << conv::FLAT));
-  if (f->bmode == conv::B_GATHER && f->amode == conv::B_GATHER) tiles &= ~(1u << conv::TALL);
+  if (f->bmode == conv::B_GATHER) tiles &= ~((1u << conv::TALL) | (1u << conv::WIDE) | (1u << conv::FLAT));
+  if (f->amode == conv::B_GATHER) tiles &= ~((1u << conv::TALL) | (1u << conv::WIDE));
   const int64_t per_split = out * 4 + (with_db ? int64_t(p.Cout) * 4 : 0);
-  MX_TRY(plan_gemm(p.M, p.Ncols, p.K, p.G, knob_tiles(d, tiles), 65535, out, per_split, ws_limit, &f->gp));
+  MX_TRY(plan_gemm(true, p.M, p.Ncols, p.K, p.G, knob_tiles(d, tiles), 65535, out, per_split, ws_limit, &f->gp));
   p.splits = f->gp.splits;
   p.kps = f->gp.kps;
   if (f->gp.splits > 1) {

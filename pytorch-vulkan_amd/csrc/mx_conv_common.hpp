@@ -103,7 +103,6 @@ __device__ __forceinline__ int wave_uniform(int v) { return __builtin_amdgcn_rea
 template <int ROWS, int BK, bool BLOCKED>
 struct Im2colLoader {
   static constexpr bool KMAJOR = false;
-  int kstep = BK;  // k advance per load(); the main loop may set 2 * BK
   static constexpr int EPT = ROWS * BK / kThreads;
   static_assert(ROWS % 64 == 0 && ROWS <= kThreads && EPT >= 1 && BK % EPT == 0 && kChanBlock % EPT == 0,
                 "Im2colLoader tiling");
@@ -121,9 +120,9 @@ struct Im2colLoader {
     const int pos = col0 + r;
     ok = pos < p.Ncols;
     const int pp = ok ? pos : 0;
-    const int img = pp / p.OHOW;
+    const int img = int(fdiv(uint32_t(pp), p.f_ohow));
     const int q = pp - img * p.OHOW;
-    const int oh = q / p.OW;
+    const int oh = int(fdiv(uint32_t(q), p.f_ow));
     const int ow = q - oh * p.OW;
     ih0 = ok ? oh * p.sh - p.ph : INT_MIN / 2;  // fails every bounds test
     iw0 = ow * p.sw - p.pw;
@@ -179,20 +178,12 @@ struct Im2colLoader {
         v[e] = bload(rs, valid ? xoff + uint32_t(ih * W + iw) * 4u : kOffNone, uint32_t(ci) * uint32_t(HW) * 4u);
       }
     }
-    k += kstep;
+    skip();
   }
-  __device__ __forceinline__ void store(float* lds) const {
-    constexpr int LDK = BK + 4;
-    const int tid = threadIdx.x;
-    float* dst = lds + (tid % ROWS) * LDK + ks;
-    if constexpr (EPT % 4 == 0) {
-#pragma unroll
-      for (int e = 0; e < EPT; e += 4)
-        *reinterpret_cast<f32x4*>(dst + e) = f32x4{v[e], v[e + 1], v[e + 2], v[e + 3]};
-    } else {
-#pragma unroll
-      for (int e = 0; e < EPT; ++e) dst[e] = v[e];
-    }
+  __device__ __forceinline__ void skip() { k += BK; }
+  template <class S>
+  __device__ __forceinline__ void store(S st) const {
+    st.template run<EPT>(threadIdx.x % ROWS, ks, v);
   }
 };
 
@@ -204,7 +195,6 @@ struct Im2colLoader {
 template <int ROWS, int BK, bool DY>
 struct PosQuadLoader {
   static constexpr bool KMAJOR = true;
-  int kstep = BK;  // k advance per load(); the main loop may set 2 * BK
   static constexpr int TPK = ROWS / 4;        // threads per k
   static constexpr int KPP = kThreads / TPK;  // k per pass
   static constexpr int PASSES = BK / KPP;
@@ -223,7 +213,7 @@ struct PosQuadLoader {
     const int pos = col0 + 4 * (tid % TPK);
     const bool ok = pos < p.Ncols;
     const int pp = ok ? pos : 0;
-    const int img = pp / hw;
+    const int img = int(fdiv(uint32_t(pp), DY ? p.f_ohow : p.f_hw));
     voff = ok ? uint32_t((gbase + int64_t(img) * cs + (pp - img * hw) + int64_t(kk) * hw) * 4) : kOffNone;
     hw4 = uint32_t(hw) * 4u;
     k = k0;
@@ -235,14 +225,13 @@ struct PosQuadLoader {
       const int kx = k + kk + q * KPP;
       v[q] = bload4(rs, kx < kmax ? voff : kOffNone, uint32_t(k + q * KPP) * hw4);
     }
-    k += kstep;
+    skip();
   }
-  __device__ __forceinline__ void store(float* lds) const {
-    constexpr int LDR = ROWS + 4;
-    const int tid = threadIdx.x;
+  __device__ __forceinline__ void skip() { k += BK; }
+  template <class S>
+  __device__ __forceinline__ void store(S st) const {
 #pragma unroll
-    for (int q = 0; q < PASSES; ++q)
-      *reinterpret_cast<f32x4*>(lds + (kk + q * KPP) * LDR + 4 * (tid % TPK)) = v[q];
+    for (int q = 0; q < PASSES; ++q) st.col4(kk + q * KPP, 4 * (threadIdx.x % TPK), v[q]);
   }
 };
 
@@ -253,7 +242,6 @@ struct PosQuadLoader {
 template <int ROWS, int BK, bool BLOCKED>
 struct PhaseGatherLoader {
   static constexpr bool KMAJOR = false;
-  int kstep = BK;  // k advance per load(); the main loop may set 2 * BK
   static constexpr int EPT = ROWS * BK / kThreads;
   static_assert(ROWS % 64 == 0 && ROWS <= kThreads && EPT >= 1 && BK % EPT == 0 && kChanBlock % EPT == 0,
                 "PhaseGatherLoader tiling");
@@ -326,20 +314,12 @@ struct PhaseGatherLoader {
         v[e] = bload(rs, valid ? doff + uint32_t(oh * OW + ow) * 4u : kOffNone, uint32_t(co) * uint32_t(OHOW) * 4u);
       }
     }
-    k += kstep;
+    skip();
   }
-  __device__ __forceinline__ void store(float* lds) const {
-    constexpr int LDK = BK + 4;
-    const int tid = threadIdx.x;
-    float* dst = lds + (tid % ROWS) * LDK + ks;
-    if constexpr (EPT % 4 == 0) {
-#pragma unroll
-      for (int e = 0; e < EPT; e += 4)
-        *reinterpret_cast<f32x4*>(dst + e) = f32x4{v[e], v[e + 1], v[e + 2], v[e + 3]};
-    } else {
-#pragma unroll
-      for (int e = 0; e < EPT; ++e) dst[e] = v[e];
-    }
+  __device__ __forceinline__ void skip() { k += BK; }
+  template <class S>
+  __device__ __forceinline__ void store(S st) const {
+    st.template run<EPT>(threadIdx.x % ROWS, ks, v);
   }
 };
 
@@ -351,7 +331,6 @@ struct PhaseGatherLoader {
 template <int ROWS, int BK>
 struct DyRowsLoader {
   static constexpr bool KMAJOR = false;
-  int kstep = BK;  // k advance per load(); the main loop may set 2 * BK
   static constexpr int LPR = BK;  // lanes per row
   static constexpr int RPP = kThreads / BK;
   static constexpr int PASSES = ROWS / RPP;
@@ -387,16 +366,14 @@ struct DyRowsLoader {
     const uint32_t base = kin ? img * cohow4 + roff + (uint32_t(kx) - img * uint32_t(OHOW)) * 4u : kOffNone;
 #pragma unroll
     for (int q = 0; q < PASSES; ++q) v[q] = bload(rs, rok[q] ? base : kOffNone, uint32_t(q) * pass4);
-    k += kstep;
+    skip();
   }
-  __device__ __forceinline__ void store(float* lds) const {
-    constexpr int LDK = BK + 4;
-    const int tid = threadIdx.x;
+  __device__ __forceinline__ void skip() { k += BK; }
+  template <class S>
+  __device__ __forceinline__ void store(S st) const {
+    st.template rows1<PASSES>(threadIdx.x / BK, RPP, kk, v);
 #pragma unroll
-    for (int q = 0; q < PASSES; ++q) {
-      lds[(tid / BK + q * RPP) * LDK + kk] = v[q];
-      bsum[q] += v[q];
-    }
+    for (int q = 0; q < PASSES; ++q) bsum[q] += v[q];
   }
 };
 
@@ -407,7 +384,6 @@ struct DyRowsLoader {
 template <int ROWS, int BK, bool DY>
 struct PosKLoader {
   static constexpr bool KMAJOR = false;
-  int kstep = BK;  // k advance per load(); the main loop may set 2 * BK
   static constexpr int LPR = BK / 4;  // lanes per row
   static constexpr int RPP = kThreads / LPR;
   static constexpr int PASSES = ROWS / RPP;
@@ -446,14 +422,14 @@ struct PosKLoader {
     const uint32_t base = kin ? img * cs4 + roff + (uint32_t(kx) - img * uint32_t(hw)) * 4u : kOffNone;
 #pragma unroll
     for (int q = 0; q < PASSES; ++q) v[q] = bload4(rs, rok[q] ? base : kOffNone, uint32_t(q) * pass4);
-    k += kstep;
+    skip();
   }
-  __device__ __forceinline__ void store(float* lds) const {
-    constexpr int LDK = BK + 4;
-    const int tid = threadIdx.x;
+  __device__ __forceinline__ void skip() { k += BK; }
+  template <class S>
+  __device__ __forceinline__ void store(S st) const {
 #pragma unroll
     for (int q = 0; q < PASSES; ++q) {
-      *reinterpret_cast<f32x4*>(lds + (tid / LPR + q * RPP) * LDK + 4 * kq) = v[q];
+      st.row4(threadIdx.x / LPR + q * RPP, 4 * kq, v[q]);
       if constexpr (DY) bsum[q] += (v[q][0] + v[q][1]) + (v[q][2] + v[q][3]);
     }
   }
@@ -470,9 +446,6 @@ struct PosKLoader {
 template <int ROWS, int BK, bool BLOCKED>
 struct XColsLoader {
   static constexpr bool KMAJOR = false;
-  // Per-row offsets of the plain order leave room for one register set only.
-  static constexpr bool DEEP = BLOCKED;
-  int kstep = BK;  // k advance per load(); the main loop may set 2 * BK
   static constexpr int RPP = kThreads / BK;
   static constexpr int PASSES = ROWS / RPP;
   static constexpr int NR = BLOCKED ? 1 : PASSES;  // rows with their own tap / channel
@@ -550,13 +523,12 @@ struct XColsLoader {
         v[q] = bload(rs, valid ? ibase + coff[q] + uint32_t(ih * W + iw) * 4u : kOffNone, 0u);
       }
     }
-    k += kstep;
+    skip();
   }
-  __device__ __forceinline__ void store(float* lds) const {
-    constexpr int LDK = BK + 4;
-    const int tid = threadIdx.x;
-#pragma unroll
-    for (int q = 0; q < PASSES; ++q) lds[((tid / BK) * PASSES + q) * LDK + kk] = v[q];
+  __device__ __forceinline__ void skip() { k += BK; }
+  template <class S>
+  __device__ __forceinline__ void store(S st) const {
+    st.template rows1<PASSES>((threadIdx.x / BK) * PASSES, 1, kk, v);
   }
 };
 
@@ -565,9 +537,10 @@ struct XColsLoader {
 using TileTall = Cfg<256, 128, 16, 2, 2>;   // 4 waves of 128 x 64
 using TileWide = Cfg<128, 256, 16, 2, 2>;   // 4 waves of 64 x 128
 using TileSq = Cfg<128, 128, 16, 2, 2>;     // 4 waves of 64 x 64
+using TileSqDeep = Cfg<128, 128, 16, 2, 2, true, true>;  // forward and dInput: two register sets
 using TileFlat = Cfg<64, 256, 16, 1, 2>;    // 4 waves of 64 x 64 in a row
 using TileNarrow = Cfg<256, 64, 16, 4, 2>;  // 4 waves of 64 x 64 in a column
-using TileSmall = Cfg<64, 64, 32, 2, 4>;    // 4 waves of 32 x 32, 32-deep slabs (dWeight)
+using TileSmall = Cfg<64, 64, 32, 2, 3>;    // 4 waves of 32 x 32, 32-deep slabs (dWeight)
 // Forward and dInput run the small tile with 16-deep slabs: half the LDS and
 // load registers, so five workgroups fit a CU instead of four (measured on
 // the ResNet-50 layers: 1x1 forwards and input gradients 2-15% faster; the

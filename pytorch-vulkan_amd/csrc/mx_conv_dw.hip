@@ -1,4 +1,4 @@
-// Conv2D dWeight (+ fused dBias) as a split-K implicit GEMM on FP32 MFMA (gfx950).
+// Conv2D dWeight (+ fused dBias) as a split-K implicit GEMM on MFMA (gfx950, FP32).
 //
 // Reference behaviour followed: conv2d_backward_weight_tiled_body.glsl:1-71
 // (dW[co, (ci,kh,kw)] = sum over positions of dy[co, pos] * im2col(x)[pos, (ci,kh,kw)]),
@@ -43,11 +43,12 @@ MX_TILE_KERNEL(C) void conv_dw_kernel(ConvArgs p) {
   const int k_begin = split * p.kps;
   const int k_end = min(p.K, k_begin + p.kps);
   LA la;
-  la.init(p, row0, g, k_begin, k_end);
   LB lb;
-  lb.init(p, col0, g, k_begin, k_end);
   Acc<C> acc;
-  mainloop<C>(acc, la, lb, (k_end - k_begin + C::BK - 1) / C::BK, smem);
+  tile_product<C>(acc, la, lb, (k_end - k_begin + C::BK - 1) / C::BK, smem, [&](auto& a, auto& b) {
+    a.init(p, row0, g, k_begin, k_end);
+    b.init(p, col0, g, k_begin, k_end);
+  });
 
   const int64_t dw_elems = int64_t(p.G) * p.Cout_g * p.Ncols;
   float* dst = (p.splits == 1 ? p.out : p.ws + split * dw_elems) + int64_t(g) * p.Cout_g * p.Ncols;
@@ -70,14 +71,7 @@ MX_TILE_KERNEL(C) void conv_dw_kernel(ConvArgs p) {
     }
     ccol[j] = n < p.Ncols ? uint32_t(c) * 4u : kOffNone;
   }
-  for_each_acc_row<C>([&](int r, int i, int v) {
-    const int co = row0 + r;
-    const bool rok = co < p.M;
-    const uint32_t roff = uint32_t(co * p.Ncols) * 4u;
-#pragma unroll
-    for (int j = 0; j < C::FN; ++j)
-      bstore(acc.v[i][j][v], ro, (rok && ccol[j] != kOffNone) ? roff + ccol[j] : kOffNone, 0);
-  });
+  store_tile<C>(ro, ccol, uint32_t(p.Ncols) * 4u, row0, p.M, [&](int i, int j, int v) { return acc.v[i][j][v]; });
   if (p.db != nullptr && tn == 0) {
     float* dbd = (p.splits == 1 ? p.db : p.ws_db + int64_t(split) * p.Cout) + g * p.Cout_g;
     const int tid = threadIdx.x;
@@ -197,22 +191,23 @@ int launch_b(ConvArgs p, int bmode, hipStream_t s) {
   p.tiles_m = (p.M + C::BM - 1) / C::BM;
   p.tiles_n = (p.Ncols + C::BN - 1) / C::BN;
   const dim3 grid(p.tiles_m * p.tiles_n, p.splits, p.G);
+  // Not built, for their registers (the planner never picks them): scalar dy
+  // rows on the 256x128 / 128x256 tiles, the x-column gather over 256 columns
+  // or on a 256x128 tile.
+  constexpr bool large = C::BM * C::BN > 128 * 128;
+  constexpr bool dy_rows = std::is_same_v<LA, DyRowsLoader<C::BM, C::BK>>;
   if (bmode == B_VEC) {
-    hipLaunchKernelGGL((conv_dw_kernel<C, LA, PosKLoader<C::BN, C::BK, false>>), grid, dim3(kThreads), 0, s, p);
+    if constexpr (!(large && dy_rows))
+      hipLaunchKernelGGL((conv_dw_kernel<C, LA, PosKLoader<C::BN, C::BK, false>>), grid, dim3(kThreads), 0, s, p);
+    else
+      return set_error(MX_ERR_INVALID, "conv2d dweight: tile too large for scalar dy rows");
+  } else if constexpr (C::BN <= 128 && !large) {
+    if (p.cols_blocked)
+      hipLaunchKernelGGL((conv_dw_kernel<C, LA, XColsLoader<C::BN, C::BK, true>>), grid, dim3(kThreads), 0, s, p);
+    else
+      hipLaunchKernelGGL((conv_dw_kernel<C, LA, XColsLoader<C::BN, C::BK, false>>), grid, dim3(kThreads), 0, s, p);
   } else {
-    // The x-column gather over 256 columns, or paired with the scalar dy rows
-    // on a 256-wide tile, does not fit the register budget; the planner never
-    // picks those.
-    constexpr bool dy_rows = std::is_same_v<LA, DyRowsLoader<C::BM, C::BK>>;
-    constexpr bool fits = C::BN <= 128 && (C::BM * C::BN <= 128 * 128 || !dy_rows);
-    if constexpr (fits) {
-      if (p.cols_blocked)
-        hipLaunchKernelGGL((conv_dw_kernel<C, LA, XColsLoader<C::BN, C::BK, true>>), grid, dim3(kThreads), 0, s, p);
-      else
-        hipLaunchKernelGGL((conv_dw_kernel<C, LA, XColsLoader<C::BN, C::BK, false>>), grid, dim3(kThreads), 0, s, p);
-    } else {
-      return set_error(MX_ERR_INVALID, "conv2d dweight: tile too large for two gathered operands");
-    }
+    return set_error(MX_ERR_INVALID, "conv2d dweight: tile too large for the x-column gather");
   }
   MX_HIP(hipGetLastError());
   return MX_OK;
@@ -221,7 +216,10 @@ int launch_b(ConvArgs p, int bmode, hipStream_t s) {
 template <class C>
 int launch_a(const ConvArgs& p, int amode, int bmode, hipStream_t s) {
   if (amode == B_VEC) return launch_b<C, PosKLoader<C::BM, C::BK, true>>(p, bmode, s);
-  return launch_b<C, DyRowsLoader<C::BM, C::BK>>(p, bmode, s);
+  // Scalar dy rows leave the larger tiles no registers for the second
+  // accumulator set.
+  constexpr bool dual = C::BM * C::BN <= 64 * 64;
+  return launch_b<Cfg<C::BM, C::BN, C::BK, C::WAVES_M, C::OCC, dual>, DyRowsLoader<C::BM, C::BK>>(p, bmode, s);
 }
 
 }  // namespace

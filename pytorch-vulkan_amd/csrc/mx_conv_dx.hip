@@ -1,4 +1,4 @@
-// Conv2D dInput as one implicit GEMM per stride phase on FP32 MFMA (gfx950).
+// Conv2D dInput as one implicit GEMM per stride phase on MFMA (gfx950, FP32).
 //
 // Reference behaviour followed: csrc/shaders/conv2d_backward_input_tiled_body.glsl:1-95
 // (dInput implicit GEMM: dx[ci, ipos] = sum over (co, kh, kw) of
@@ -75,11 +75,12 @@ __device__ __forceinline__ void dx_tile(const ConvArgs& p, int g, int lin, int s
   const int row0 = tm * C::BM, col0 = tn * C::BN;
   const int k0 = split * p.kps, k1 = min(p.K, k0 + p.kps);
   BufStridedLoader<C::BM, C::BK, MA> la;  // element (ci, k) = wt[g][k][ci]
-  la.init(p.wt + int64_t(g) * p.K * p.Cin_g, int64_t(p.K) * p.Cin_g * 4, 1, p.Cin_g, row0, p.M, k0, k1);
   LB lb;
-  lb.init(p, col0, g, k0, k1);
   Acc<C> acc;
-  mainloop<C>(acc, la, lb, (k1 - k0 + C::BK - 1) / C::BK, smem);
+  tile_product<C>(acc, la, lb, (k1 - k0 + C::BK - 1) / C::BK, smem, [&](auto& a, auto& b) {
+    a.init(p.wt + int64_t(g) * p.K * p.Cin_g, int64_t(p.K) * p.Cin_g * 4, 1, p.Cin_g, row0, p.M, k0, k1);
+    b.init(p, col0, g, k0, k1);
+  });
   float* const out = p.splits == 1 ? p.out : p.ws + split * p.out_elems;
   // (Not built for the 256-wide tiles, whose registers it would spill; the
   // host does not request it for them.)
@@ -112,13 +113,12 @@ __device__ __forceinline__ void dx_tile(const ConvArgs& p, int g, int lin, int s
     });
     return;
   }
-  // The output (one launch's dx, or one split's partial, below 2^31 bytes)
-  // as a buffer resource: stores outside the tile's valid rows / columns go
-  // to kOffNone and are dropped, so the stores run straight through without
-  // a branch or a 64-bit address per element.  Byte offset of each fragment
-  // column (img * Cin * HW + phase position), once.
+  // The output (one launch's dx, or one split's partial, below 2^31 bytes) as
+  // a buffer resource: stores outside the tile's valid rows / columns are
+  // dropped.  Byte offset of each fragment column (img * Cin * HW + phase
+  // position), once.
   const i32x4 ro = buffer_rsrc(out, p.out_elems * 4);
-  uint32_t cbase[C::FN];
+  uint32_t col[C::FN];
 #pragma unroll
   for (int j = 0; j < C::FN; ++j) {
     const int pos = col0 + acc_col<C>(j);
@@ -127,17 +127,10 @@ __device__ __forceinline__ void dx_tile(const ConvArgs& p, int g, int lin, int s
     const int img = pp / p.HpWp;
     const int q = pp - img * p.HpWp;
     const int i = q / p.Wp;
-    cbase[j] = cok ? uint32_t(img * p.Cin * p.HW + (p.pa + p.sh * i) * p.W + p.pb + p.sw * (q - i * p.Wp)) * 4u
-                   : kOffNone;
+    col[j] = cok ? uint32_t((img * p.Cin + g * p.Cin_g) * p.HW + (p.pa + p.sh * i) * p.W + p.pb + p.sw * (q - i * p.Wp)) * 4u
+                 : kOffNone;
   }
-  for_each_acc_row<C>([&](int r, int i, int v) {
-    const int ci = row0 + r;
-    const bool rok = ci < p.M;
-    const uint32_t roff = uint32_t((g * p.Cin_g + ci) * p.HW) * 4u;
-#pragma unroll
-    for (int j = 0; j < C::FN; ++j)
-      bstore(acc.v[i][j][v], ro, (rok && cbase[j] != kOffNone) ? roff + cbase[j] : kOffNone, 0);
-  });
+  store_tile<C>(ro, col, uint32_t(p.HW) * 4u, row0, p.M, [&](int i, int j, int v) { return acc.v[i][j][v]; });
 }
 
 template <class C, Mode MA, class LB>
@@ -233,7 +226,7 @@ int conv_dx_launch_set(const DxPhaseSet& set, int tile, Mode ma, int bmode, hipS
   switch (tile) {
     case TALL: return launch_set_a<TileTall>(set, ma, bmode, s);
     case WIDE: return launch_set_a<TileWide>(set, ma, bmode, s);
-    case SQ: return launch_set_a<TileSq>(set, ma, bmode, s);
+    case SQ: return launch_set_a<TileSqDeep>(set, ma, bmode, s);
     case FLAT: return launch_set_a<TileFlat>(set, ma, bmode, s);
     default: return launch_set_a<TileSmallShallow>(set, ma, bmode, s);
   }
@@ -243,7 +236,7 @@ int conv_dx_launch(const ConvArgs& p, int tile, Mode ma, int bmode, hipStream_t 
   switch (tile) {
     case TALL: return launch_a<TileTall>(p, ma, bmode, s);
     case WIDE: return launch_a<TileWide>(p, ma, bmode, s);
-    case SQ: return launch_a<TileSq>(p, ma, bmode, s);
+    case SQ: return launch_a<TileSqDeep>(p, ma, bmode, s);
     case FLAT: return launch_a<TileFlat>(p, ma, bmode, s);
     default: return launch_a<TileSmallShallow>(p, ma, bmode, s);
   }

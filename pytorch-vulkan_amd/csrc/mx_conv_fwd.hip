@@ -1,4 +1,4 @@
-// Conv2D forward as an implicit GEMM on FP32 MFMA (gfx950).
+// Conv2D forward (FP32) as an implicit GEMM on MFMA (gfx950).
 //
 // Reference behaviour followed: csrc/shaders/conv2d_tiled_body.glsl:1-87
 // (implicit-GEMM forward, bias in the store) and
@@ -25,48 +25,42 @@ MX_TILE_KERNEL(C) void conv_fwd_kernel(ConvArgs p) {
   const int split = blockIdx.y;
   const int k0 = split * p.kps, k1 = min(p.K, k0 + p.kps);
   BufStridedLoader<C::BM, C::BK, MA> la;
-  la.init(p.wt + int64_t(g) * p.Cout_g * p.ldw, int64_t(p.Cout_g) * p.ldw * 4, p.ldw, 1, row0, p.M, k0, k1);
   LB lb;
-  lb.init(p, col0, g, k0, k1);
   Acc<C> acc;
-  mainloop<C>(acc, la, lb, (k1 - k0 + C::BK - 1) / C::BK, smem);
+  tile_product<C>(acc, la, lb, (k1 - k0 + C::BK - 1) / C::BK, smem, [&](auto& a, auto& b) {
+    a.init(p.wt + int64_t(g) * p.Cout_g * p.ldw, int64_t(p.Cout_g) * p.ldw * 4, p.ldw, 1, row0, p.M, k0, k1);
+    b.init(p, col0, g, k0, k1);
+  });
   // With split-K the tile goes to this split's partial output (bias added by
   // the finalize).
   float* const out = p.splits == 1 ? p.out : p.ws + split * p.out_elems;
   const float* const bias = p.splits == 1 ? p.bias : nullptr;
-  // The output (one launch's, below 2^31 bytes) as a buffer resource: a
-  // store outside the tile's valid rows / columns goes to kOffNone and is
-  // dropped, so the epilogue has no branches.  Stores count in the same
-  // vector-memory counter as loads, so the bias values of a fragment row
-  // block are all loaded before its first store: a load between stores would
-  // make every later store wait for the earlier ones to complete.
+  // The output (one launch's, below 2^31 bytes) as a buffer resource: stores
+  // outside the tile's valid rows / columns are dropped.  Stores count in the
+  // same vector-memory counter as loads, so the bias values of the lane's rows
+  // (four at a time, rows 8q + 4h .. + 3) are all loaded before the first
+  // store: a load between stores would make every later store wait for the
+  // earlier ones to complete.
   const i32x4 ro = buffer_rsrc(out, p.out_elems * 4);
+  f32x4 b[C::FM][4] = {};
+  if (bias) {
+    const i32x4 rb = buffer_rsrc(bias + g * p.Cout_g, int64_t(p.Cout_g) * 4);
+    const uint32_t first = uint32_t(row0 + wave_row0<C>() + lane_row()) * 4u;
+#pragma unroll
+    for (int i = 0; i < C::FM; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) b[i][q] = bload4(rb, first + uint32_t(block_row(i, 4 * q)) * 4u, 0);
+  }
   // Output byte offset of each fragment column (img * Cout * OHOW + q), once.
-  uint32_t cbase[C::FN];
+  uint32_t col[C::FN];
 #pragma unroll
   for (int j = 0; j < C::FN; ++j) {
-    const int pos = col0 + acc_col<C>(j);
-    const int img = (pos < p.Ncols ? pos : 0) / p.OHOW;
-    cbase[j] = pos < p.Ncols ? uint32_t(img * p.Cout * p.OHOW + (pos - img * p.OHOW)) * 4u : kOffNone;
+    const uint32_t pos = col0 + acc_col<C>(j);
+    const uint32_t img = fdiv(pos, p.f_ohow);
+    col[j] = pos < uint32_t(p.Ncols) ? ((img * p.Cout + g * p.Cout_g) * p.OHOW + (pos - img * p.OHOW)) * 4u : kOffNone;
   }
-#pragma unroll
-  for (int i = 0; i < C::FM; ++i) {
-    float b[16];
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int co = row0 + acc_row<C>(i, v);
-      b[v] = (bias && co < p.M) ? bias[g * p.Cout_g + co] : 0.f;
-    }
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int co = row0 + acc_row<C>(i, v);
-      const bool rok = co < p.M;
-      const uint32_t roff = uint32_t((g * p.Cout_g + co) * p.OHOW) * 4u;
-#pragma unroll
-      for (int j = 0; j < C::FN; ++j)
-        bstore(acc.v[i][j][v] + b[v], ro, (rok && cbase[j] != kOffNone) ? roff + cbase[j] : kOffNone, 0);
-    }
-  }
+  store_tile<C>(ro, col, uint32_t(p.OHOW) * 4u, row0, p.M,
+                [&](int i, int j, int v) { return acc.v[i][j][v] + b[i][v >> 2][v & 3]; });
 }
 
 // Wp[g][co][k] = w[g*Cout_g + co][ci][kh][kw] with k the blocked gathered
@@ -148,7 +142,7 @@ int conv_fwd_launch(const ConvArgs& p, int tile, Mode ma, int bmode, hipStream_t
   switch (tile) {
     case TALL: return launch_a<TileTall>(p, ma, bmode, s);
     case WIDE: return launch_a<TileWide>(p, ma, bmode, s);
-    case SQ: return launch_a<TileSq>(p, ma, bmode, s);
+    case SQ: return launch_a<TileSqDeep>(p, ma, bmode, s);
     case FLAT: return launch_a<TileFlat>(p, ma, bmode, s);
     default: return launch_a<TileSmallShallow>(p, ma, bmode, s);
   }

@@ -1,5 +1,5 @@
 // FP32 strided / batched GEMM with fused alpha, beta*bias epilogue on gfx950
-// MFMA (v_mfma_f32_32x32x2f32).
+// MFMA (FP32 operands as three bf16 pieces, mfma_core.hpp).
 //
 // Covers the reference's matmul_strided{,_reg}{,_bias}.comp and
 // bmm_strided.comp (mm_impl csrc/ops/mm.cpp:244-343, addmm_bias_vulkan
@@ -13,6 +13,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <string>
+#include <type_traits>
 
 #include "mfma_core.hpp"
 #include "mx_internal.hpp"
@@ -46,10 +47,11 @@ MX_TILE_KERNEL(C) void gemm_kernel(GemmArgs p) {
   const int64_t bz = int64_t(p.batch0) + blockIdx.z;
   StridedLoader<C::BM, C::BK, MA> la;
   StridedLoader<C::BN, C::BK, MB> lb;
-  la.init(p.a + bz * p.a_sb, p.a_sm, p.a_sk, row0, p.M, 0, p.K);
-  lb.init(p.b + bz * p.b_sb, p.b_sn, p.b_sk, col0, p.N, 0, p.K);
   Acc<C> acc;
-  mainloop<C>(acc, la, lb, (p.K + C::BK - 1) / C::BK, smem);
+  tile_product<C>(acc, la, lb, (p.K + C::BK - 1) / C::BK, smem, [&](auto& a, auto& b) {
+    a.init(p.a + bz * p.a_sb, p.a_sm, p.a_sk, row0, p.M, 0, p.K);
+    b.init(p.b + bz * p.b_sb, p.b_sn, p.b_sk, col0, p.N, 0, p.K);
+  });
   float* __restrict__ cb = p.c + bz * p.c_sb;
   const float* __restrict__ bias = p.bias ? p.bias + bz * p.bias_sb : nullptr;
   const float alpha = p.alpha, beta = p.beta;
@@ -75,6 +77,15 @@ MX_TILE_KERNEL(C) void gemm_kernel(GemmArgs p) {
       for (int j = 0; j < C::FN; ++j)
         if (ccol[j] < p.N) crow[ccol[j]] = alpha * acc.v[i][j][v] + beta * brow[int64_t(ccol[j]) * p.bias_sn];
     });
+    return;
+  }
+  if (p.ldc >= 0 && p.ldc <= kVecStrideMax) {
+    // Offsets from the tile's corner, below 2^31 bytes at this row stride.
+    uint32_t col[C::FN];
+#pragma unroll
+    for (int j = 0; j < C::FN; ++j) col[j] = ccol[j] < p.N ? uint32_t(ccol[j] - col0) * 4u : kOffNone;
+    store_tile<C>(buffer_rsrc(cb + int64_t(row0) * p.ldc + col0, kBufMaxBytes), col, uint32_t(p.ldc) * 4u, 0,
+                  p.M - row0, [&](int i, int j, int v) { return alpha * acc.v[i][j][v] + bcol[j]; });
     return;
   }
   for_each_acc_row<C>([&](int r, int i, int v) {
@@ -113,8 +124,9 @@ bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u
 Mode pick_mode(const float* base, int64_t s_row, int64_t s_k, int64_t s_batch, int64_t batch, int64_t R,
                int64_t K) {
   const bool batch_ok = batch <= 1 || s_batch % 4 == 0;
-  if (s_k == 1 && aligned16(base) && s_row % 4 == 0 && batch_ok && K % 4 == 0) return Mode::KVEC;
-  if (s_row == 1 && aligned16(base) && s_k % 4 == 0 && batch_ok && R % 4 == 0) return Mode::RVEC;
+  const auto vec_stride = [](int64_t s) { return s >= 0 && s <= kVecStrideMax && s % 4 == 0; };
+  if (s_k == 1 && aligned16(base) && vec_stride(s_row) && batch_ok && K % 4 == 0) return Mode::KVEC;
+  if (s_row == 1 && aligned16(base) && vec_stride(s_k) && batch_ok && R % 4 == 0) return Mode::RVEC;
   if (s_k == 1) return Mode::KSCALAR;
   if (s_row == 1) return Mode::RSCALAR;
   return std::llabs(s_k) <= std::llabs(s_row) ? Mode::KSCALAR : Mode::RSCALAR;
@@ -122,11 +134,18 @@ Mode pick_mode(const float* base, int64_t s_row, int64_t s_k, int64_t s_batch, i
 
 template <class C, Mode MA, Mode MB>
 int launch3(GemmArgs p, hipStream_t s) {
+  // A 128x128 tile has the registers for two slabs of each operand in flight
+  // when both are read 16 bytes at a time, and for the second accumulator set
+  // unless both are row-scalar.
+  constexpr bool sq = C::BM * C::BN == 128 * 128;
+  constexpr bool vec = (MA == Mode::KVEC || MA == Mode::RVEC) && (MB == Mode::KVEC || MB == Mode::RVEC);
+  constexpr bool dual = !(sq && MA == Mode::RSCALAR && MB == Mode::RSCALAR);
+  using D = std::conditional_t<sq, Cfg<C::BM, C::BN, C::BK, C::WAVES_M, C::OCC, dual, vec>, C>;
   const int ntiles = p.tiles_m * p.tiles_n;
   for (int b0 = 0; b0 < p.batch; b0 += 65535) {
     p.batch0 = b0;
     const dim3 grid(ntiles, 1, std::min(p.batch - b0, 65535));
-    hipLaunchKernelGGL((gemm_kernel<C, MA, MB>), grid, dim3(kThreads), 0, s, p);
+    hipLaunchKernelGGL((gemm_kernel<D, MA, MB>), grid, dim3(kThreads), 0, s, p);
     MX_HIP(hipGetLastError());
   }
   return MX_OK;
@@ -178,7 +197,7 @@ struct TileChoice {
   int bm, bn, per_cu;
   double rate;  // throughput of a CU full of such tiles, relative to 256 x 128
 };
-constexpr TileChoice kTiles[] = {{256, 128, 2, 1.0}, {128, 256, 2, 1.0}, {128, 128, 2, 0.94}, {64, 64, 4, 0.6}};
+constexpr TileChoice kTiles[] = {{256, 128, 2, 1.0}, {128, 256, 2, 0.98}, {128, 128, 2, 0.94}, {64, 64, 4, 0.77}};
 
 // Cheapest tile by a wave-quantised cost model: rounds of resident tiles
 // times the time of one round (per_cu tiles per CU at the relative rate).

@@ -1,0 +1,139 @@
+"""The split product of the GEMM and convolution tiles: every FP32 operand as
+three bf16 pieces, six piece products on the bf16 matrix instruction, FP32
+accumulators.
+
+Bound: the pieces restore an operand exactly and the dropped products are below
+2^-24 of a term, so what is left is FP32 accumulation, at most one rounding
+(2^-24 relative to the running sum, itself at most the sum of the terms'
+magnitudes) per 16 terms and product -- bounded here by (K / 16 + 8) * 2^-23 of
+the summed magnitudes.  Operands without pieces (infinite, above the largest
+bf16, below 2^-110) take the FP32 product, checked at K * 2^-24 of the
+magnitudes or by their pattern.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def mx():
+    import torch_vulkan  # noqa: F401
+    from torch_vulkan import mx as m
+    return m
+
+
+def gemm(mx, a, b, bias=None):
+    c = torch.full((*a.shape[:-1], b.shape[-1]), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    mx.gemm(a, b, c, bias=bias, beta=1.0 if bias is not None else 0.0,
+            stream=torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    return c
+
+
+def operands(layout, m, n, k, seed):
+    g = torch.Generator().manual_seed(seed)
+    a, b = torch.randn(m, k, generator=g), torch.randn(k, n, generator=g)
+    av = a.cuda() if layout[0] == "n" else a.t().contiguous().cuda().t()
+    bv = b.cuda() if layout[1] == "n" else b.t().contiguous().cuda().t()
+    return a, b, av, bv
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (63, 65, 15), (64, 64, 16), (65, 129, 17), (128, 128, 32), (129, 64, 33),
+                                   (257, 131, 48), (384, 256, 260), (8, 1000, 2048), (70, 90, 8190)])
+def test_split_product_sizes(mx, layout, m, n, k):
+    a, b, av, bv = operands(layout, m, n, k, m + n + k)
+    got = gemm(mx, av, bv).cpu().double()
+    ref, mag = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    assert ((got - ref).abs() <= (k / 16 + 8) * 2.0 ** -23 * mag).all()
+
+
+def test_split_product_is_more_exact_than_fp32_sums(mx):
+    """The relative error over K = 4096 stays below that of FP32 sums in one
+    sequence (2^-24 sqrt(K / 6): random roundings of a random walk)."""
+    a, b, av, bv = operands("nt", 256, 256, 4096, 3)
+    got, ref = gemm(mx, av, bv).cpu().double(), a.double() @ b.double()
+    assert ((got - ref).norm() / ref.norm()).item() < 2.0 ** -24 * (4096 / 6) ** 0.5
+
+
+@pytest.mark.parametrize("value", [float("inf"), -float("inf"), float("nan"), 3.4028234e38, -3.4e38])
+@pytest.mark.parametrize("m,n,k", [(70, 50, 40), (300, 300, 64)])
+def test_operands_without_pieces(mx, value, m, n, k):
+    """One such element: its row follows FP32 arithmetic (inf times the signs
+    of B's row), the other rows are untouched."""
+    a, b, av, bv = operands("nt", m, n, k, 7)
+    b[5] = torch.where(b[5].abs() < 0.05, torch.full_like(b[5], 0.05), b[5]) * 0.01
+    bv.copy_(b)
+    a[17] *= 0.01
+    a[17, 5] = value
+    av.copy_(a)
+    got, ref = gemm(mx, av, bv).cpu(), (a.double() @ b.double()).float()
+    assert torch.equal(torch.isnan(got), torch.isnan(ref))
+    assert torch.equal(torch.isinf(got), torch.isinf(ref)) and torch.equal(got[torch.isinf(ref)], ref[torch.isinf(ref)])
+    fine = torch.isfinite(ref)
+    mag = torch.nan_to_num(a).double().abs() @ b.double().abs()
+    assert ((got.double() - ref.double()).abs() <= k * 2.0 ** -23 * mag)[fine].all()
+
+
+@pytest.mark.parametrize("exp_a,exp_b", [(-60, 0), (-118, 0), (-118, 10), (-70, -50), (-128, 20)])
+def test_tiny_operands(mx, exp_a, exp_b):
+    """Operands whose pieces lose bits to bf16's smallest denormal (2^-133) get
+    the FP32 product.  (Operands below 2^-134, FP32 denormals themselves, have no
+    nonzero piece and count as zero.)"""
+    a, b, av, bv = operands("nt", 96, 80, 96, 11)
+    a, b = a.double().mul(2.0 ** exp_a).float(), b.mul(2.0 ** exp_b)
+    av.copy_(a), bv.copy_(b)
+    got = gemm(mx, av, bv).cpu().double()
+    ref, mag = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    assert ((got - ref).abs() <= 96 * (2.0 ** -23 * mag + 2.0 ** -149)).all()
+
+
+@pytest.mark.parametrize("case", ["inf", "tiny", "normal"])
+@pytest.mark.parametrize("geometry", [((2, 20, 9, 11), 24, 3, 1, 1), ((3, 32, 8, 8), 70, 1, 1, 0),
+                                      ((2, 3, 21, 17), 33, 7, 2, 3), ((4, 48, 7, 7), 130, 3, 2, 1)])
+def test_conv_phases(mx, case, geometry):
+    """Forward, both gradients and dBias of the implicit GEMM."""
+    xs, co, k, s, p = geometry
+    g = torch.Generator().manual_seed(co)
+    x, w = torch.randn(xs, generator=g), torch.randn(co, xs[1], k, k, generator=g) * 0.1
+    d = mx.conv_desc(xs, tuple(w.shape), (s, s), (p, p))
+    dy = torch.randn(xs[0], co, d.oh, d.ow, generator=g)
+    if case == "tiny":
+        dy, x = dy.double().mul(2.0 ** -118).float(), x.double().mul(2.0 ** -118).float()
+    if case == "inf":
+        dy[1, 2, 3, 1] = float("inf")
+        x[0, 1, 4, 5] = float("inf")
+    xc, wc, dyc = x.cuda(), w.cuda(), dy.cuda()
+    y, dx, dw, db = torch.empty_like(dyc), torch.empty_like(xc), torch.empty_like(wc), torch.empty(co, device="cuda")
+    st, algo = torch.cuda.current_stream().cuda_stream, mx.ALGO_IMPLICIT_GEMM
+    mx.conv2d_forward(d, xc, wc, None, y, algo, st)
+    mx.conv2d_backward_input(d, dyc, wc, dx, algo, st)
+    scale = 2.0 ** 118 if case == "tiny" else 1.0  # dW of two tiny operands underflows in any FP32 sum
+    dy_w = (dyc.double() * scale).float()
+    mx.conv2d_backward_weight(d, xc, dy_w, dw, db, algo, st)
+    torch.cuda.synchronize()
+
+    def check(got, f, *ops):
+        ref, mag = f(*(o.double() for o in ops)), f(*(torch.nan_to_num(o.double(), posinf=0).abs() for o in ops))
+        got, ref = got.cpu().double(), ref.cpu()
+        fine = torch.isfinite(ref)
+        assert torch.isfinite(got)[fine].all() and not torch.isfinite(got)[~fine].any()
+        terms = x.numel() / 4 if ops[0] is x else 9 * co
+        assert ((got - ref).abs() <= (terms / 16 + 64) * 2.0 ** -23 * mag + 2.0 ** -140)[fine].all()
+
+    def grads(which):
+        def f(a, b):
+            u, v = (torch.zeros(xs, dtype=torch.float64), a) if which == 0 else (a, torch.zeros_like(w).double())
+            u.requires_grad_(), v.requires_grad_()
+            return torch.autograd.grad(F.conv2d(u, v, None, s, p), (u, v)[which], b)[0]
+        return f
+
+    check(y, lambda a, b: F.conv2d(a, b, None, s, p), x, w)
+    check(dx, grads(0), w, dy)
+    check(dw, grads(1), x, dy_w.cpu())
+    check(db, lambda a: a.sum((0, 2, 3)), dy_w.cpu())
