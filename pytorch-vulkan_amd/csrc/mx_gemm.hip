@@ -36,6 +36,10 @@ struct GemmArgs {
   int tiles_m, tiles_n;
   float alpha, beta;
   int bias_kind;
+  // K split (splits > 1): split i takes k in [i * kps, (i + 1) * kps) and
+  // writes its partial product to ws[i][batch][M][N].
+  int splits, kps;
+  float* ws;
 };
 
 template <class C, Mode MA, Mode MB>
@@ -45,13 +49,27 @@ MX_TILE_KERNEL(C) void gemm_kernel(GemmArgs p) {
   tile_coords(xcd_remap(blockIdx.x, p.tiles_m * p.tiles_n), p.tiles_m, p.tiles_n, tm, tn);
   const int row0 = tm * C::BM, col0 = tn * C::BN;
   const int64_t bz = int64_t(p.batch0) + blockIdx.z;
+  const int split = blockIdx.y;
+  const int k0 = split * p.kps, k1 = min(p.K, k0 + p.kps);
   StridedLoader<C::BM, C::BK, MA> la;
   StridedLoader<C::BN, C::BK, MB> lb;
   Acc<C> acc;
-  tile_product<C>(acc, la, lb, (p.K + C::BK - 1) / C::BK, smem, [&](auto& a, auto& b) {
-    a.init(p.a + bz * p.a_sb, p.a_sm, p.a_sk, row0, p.M, 0, p.K);
-    b.init(p.b + bz * p.b_sb, p.b_sn, p.b_sk, col0, p.N, 0, p.K);
+  tile_product<C>(acc, la, lb, (k1 - k0 + C::BK - 1) / C::BK, smem, [&](auto& a, auto& b) {
+    a.init(p.a + bz * p.a_sb, p.a_sm, p.a_sk, row0, p.M, k0, k1);
+    b.init(p.b + bz * p.b_sb, p.b_sn, p.b_sk, col0, p.N, k0, k1);
   });
+  if (p.splits > 1) {
+    uint32_t col[C::FN];
+#pragma unroll
+    for (int j = 0; j < C::FN; ++j) {
+      const int n = acc_col<C>(j);
+      col[j] = col0 + n < p.N ? uint32_t(n) * 4u : kOffNone;
+    }
+    float* const part = p.ws + ((int64_t(split) * p.batch + bz) * p.M + row0) * p.N + col0;
+    store_tile<C>(buffer_rsrc(part, kBufMaxBytes), col, uint32_t(p.N) * 4u, 0, p.M - row0,
+                  [&](int i, int j, int v) { return acc.v[i][j][v]; });
+    return;
+  }
   float* __restrict__ cb = p.c + bz * p.c_sb;
   const float* __restrict__ bias = p.bias ? p.bias + bz * p.bias_sb : nullptr;
   const float alpha = p.alpha, beta = p.beta;
@@ -96,6 +114,42 @@ MX_TILE_KERNEL(C) void gemm_kernel(GemmArgs p) {
     for (int j = 0; j < C::FN; ++j)
       if (ccol[j] < p.N) crow[ccol[j]] = alpha * acc.v[i][j][v] + bcol[j];
   });
+}
+
+// C = alpha * (sum of the K splits' partial products, in split order) +
+// beta * bias.  VEC: four columns per thread (N and C's strides multiples of
+// four, C 16-byte aligned).
+template <bool VEC>
+__global__ __launch_bounds__(256) void gemm_sum_kernel(GemmArgs p) {
+  constexpr int W = VEC ? 4 : 1;
+  typedef float vec __attribute__((ext_vector_type(W)));
+  const int64_t plane = int64_t(p.M) * p.N, total = plane * p.batch;
+  const int kind = p.beta == 0.f ? int(MX_BIAS_NONE) : p.bias_kind;
+  for (int64_t i = (int64_t(blockIdx.x) * 256 + threadIdx.x) * W; i < total; i += int64_t(gridDim.x) * 256 * W) {
+    const float* src = p.ws + i;
+    vec s = *reinterpret_cast<const vec*>(src);
+#pragma unroll 8
+    for (int q = 1; q < p.splits; ++q) s += *reinterpret_cast<const vec*>(src + q * total);
+    const int64_t bz = i / plane;
+    const uint32_t at = uint32_t(i - bz * plane), row = at / uint32_t(p.N), n = at - row * uint32_t(p.N);
+    vec o;
+    if constexpr (VEC) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = p.alpha * s[e];
+    } else {
+      o = p.alpha * s;
+    }
+    if (kind != MX_BIAS_NONE) {
+      const float* b = p.bias + bz * p.bias_sb + n * p.bias_sn + (kind == MX_BIAS_COL ? 0 : row * p.bias_sm);
+      if constexpr (VEC) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] += p.beta * b[e * p.bias_sn];
+      } else {
+        o += p.beta * b[0];
+      }
+    }
+    *reinterpret_cast<vec*>(p.c + bz * p.c_sb + int64_t(row) * p.ldc + n) = o;
+  }
 }
 
 // k == 0: C = beta * bias (or zeros when beta == 0 / no bias).
@@ -144,7 +198,7 @@ int launch3(GemmArgs p, hipStream_t s) {
   const int ntiles = p.tiles_m * p.tiles_n;
   for (int b0 = 0; b0 < p.batch; b0 += 65535) {
     p.batch0 = b0;
-    const dim3 grid(ntiles, 1, std::min(p.batch - b0, 65535));
+    const dim3 grid(ntiles, p.splits, std::min(p.batch - b0, 65535));
     hipLaunchKernelGGL((gemm_kernel<D, MA, MB>), grid, dim3(kThreads), 0, s, p);
     MX_HIP(hipGetLastError());
   }
@@ -195,35 +249,65 @@ using TileSmall = Cfg<64, 64, 16, 2, 4>;   // 4 waves of 32 x 32
 
 struct TileChoice {
   int bm, bn, per_cu;
-  double rate;  // throughput of a CU full of such tiles, relative to 256 x 128
+  double rate;  // throughput of a CU full of such tiles, relative to 85% of its FP32 MFMA peak
 };
-constexpr TileChoice kTiles[] = {{256, 128, 2, 1.0}, {128, 256, 2, 0.98}, {128, 128, 2, 0.94}, {64, 64, 4, 0.77}};
+constexpr TileChoice kTiles[] = {{256, 128, 2, 1.81}, {128, 256, 2, 1.75}, {128, 128, 2, 1.70}, {64, 64, 4, 1.36}};
 
-// Cheapest tile by a wave-quantised cost model: rounds of resident tiles
-// times the time of one round (per_cu tiles per CU at the relative rate).
-// MX_GEMM_TILE=<index into kTiles> forces a tile (tuning and diagnosis; the
-// 256-wide tiles only for 16-byte operand modes).  `kernel` (mx_gemm_kernel)
-// forces the 64x64 tile or keeps the choice among the large ones.
-int pick_gemm_tile(int64_t m, int64_t n, int64_t batch, bool vec, int kernel) {
+constexpr int64_t kMaxSplitBytes = int64_t(64) << 20;  // partial products of one call
+constexpr int kSplitBK = 32;                           // K granularity of a split
+constexpr int kMinSplitSpan = 64;                      // shortest K range worth a split
+
+// Estimated time: a CU holding n tiles runs at rate * occ(n), occ rising from
+// 0.71 with one resident tile to 1 with per_cu; a tile's first loads and its
+// stores cost as much as 41 more k; the sum of the partials moves
+// (splits + 1) outputs at 3.6 TB/s after a launch.  The figures are the
+// convolution planner's, whose tiles run the same product.
+double tile_cost(const TileChoice& t, int64_t m, int64_t n, int64_t batch, int64_t splits, int64_t kps) {
+  const double cu = cu_count();
+  const int64_t tiles = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch * splits;
+  const double per_cu = double((tiles + int64_t(cu) - 1) / int64_t(cu));
+  const double occ = std::min(1.0, 0.71 + 0.29 * (per_cu - 1) / double(t.per_cu - 1));
+  double s = per_cu * 2.0 * t.bm * t.bn * (double(kps) + 41.0) / (0.85 * 157.3e12 / 256.0 * t.rate * occ) + 2e-6;
+  if (splits > 1) s += double(splits + 1) * double(m * n * batch) * 4.0 / 3.6e12 + 3e-6;
+  return s;
+}
+
+// Cheapest (tile, K split).  Few tiles over a long K leave most of the chip
+// idle (8 x 2048 x 1000: 16 workgroups walking 128 slabs each, 38 us), so K is
+// split where the model finds it faster, the partials summed by a second
+// launch.  `split_ok`: the call may allocate.  MX_GEMM_TILE=<index into
+// kTiles> forces a tile in one pass over K (tests and diagnosis; the 256-wide
+// tiles only for 16-byte operand modes).  `kernel` (mx_gemm_kernel) forces the 64x64 tile or
+// keeps the choice among the large ones.
+void pick_gemm_tile(int64_t m, int64_t n, int64_t k, int64_t batch, bool vec, int kernel, bool split_ok, int* tile,
+                    int* splits, int* kps) {
+  int first = vec ? 0 : 2, last = 3;
+  if (kernel == MX_GEMM_KERNEL_TILED) first = 3;
+  if (kernel == MX_GEMM_KERNEL_REGISTER) last = 2;
   if (const char* e = std::getenv("MX_GEMM_TILE")) {
     const int t = std::atoi(e);
-    if (t >= (vec ? 0 : 2) && t < 4) return t;
-  }
-  if (kernel == MX_GEMM_KERNEL_TILED) return 3;
-  const int last = kernel == MX_GEMM_KERNEL_REGISTER ? 3 : 4;
-  int best = 2;
-  double best_cost = 0;
-  for (int i = vec ? 0 : 2; i < last; ++i) {
-    const TileChoice& t = kTiles[i];
-    const int64_t tiles = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch;
-    const int64_t slots = int64_t(cu_count()) * t.per_cu;
-    const double cost = double((tiles + slots - 1) / slots) * t.per_cu * t.bm * t.bn / t.rate;
-    if (i == (vec ? 0 : 2) || cost < best_cost) {
-      best = i;
-      best_cost = cost;
+    if (t >= (vec ? 0 : 2) && t < 4) {
+      first = last = t;
+      split_ok = false;
     }
   }
-  return best;
+  static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
+  double best = -1;
+  for (int i = first; i <= last; ++i) {
+    for (const int want : kSplits) {
+      int64_t span = ((k + want - 1) / want + kSplitBK - 1) / kSplitBK * kSplitBK;
+      const int64_t s = (k + span - 1) / span;
+      if (s > 1 && (!split_ok || span < kMinSplitSpan || s * m * n * batch * 4 > kMaxSplitBytes)) break;
+      if (s == 1) span = k;
+      const double cost = tile_cost(kTiles[i], m, n, batch, s, span);
+      if (best < 0 || cost < best) {
+        best = cost;
+        *tile = i;
+        *splits = int(s);
+        *kps = int(span);
+      }
+    }
+  }
 }
 
 }  // namespace
@@ -253,7 +337,8 @@ struct GemmPlan {
   bool empty = false;
 };
 
-int plan_gemm(const mx_gemm_desc* d, const float* a, const float* b, const float* bias, float* c, GemmPlan* g) {
+int plan_gemm(const mx_gemm_desc* d, const float* a, const float* b, const float* bias, float* c, bool split_ok,
+              GemmPlan* g) {
   MX_REQUIRE(d, MX_ERR_INVALID, "mx_gemm_f32: null descriptor");
   MX_REQUIRE(d->batch >= 0 && d->m >= 0 && d->n >= 0 && d->k >= 0, MX_ERR_INVALID,
              "mx_gemm_f32: negative dimension");
@@ -292,7 +377,30 @@ int plan_gemm(const mx_gemm_desc* d, const float* a, const float* b, const float
   MX_REQUIRE(((d->m + 63) / 64) * ((d->n + 63) / 64) <= INT32_MAX, MX_ERR_INVALID, "mx_gemm_f32: too many tiles");
   g->ma = pick_mode(p.a, p.a_sm, p.a_sk, p.a_sb, p.batch, p.M, p.K);
   g->mb = pick_mode(p.b, p.b_sn, p.b_sk, p.b_sb, p.batch, p.N, p.K);
-  g->tile = pick_gemm_tile(d->m, d->n, d->batch, is_vec(g->ma) && is_vec(g->mb), d->kernel);
+  pick_gemm_tile(d->m, d->n, d->k, d->batch, is_vec(g->ma) && is_vec(g->mb), d->kernel,
+                 split_ok && d->n <= kVecStrideMax && d->m * d->n <= INT32_MAX, &g->tile, &p.splits, &p.kps);
+  return MX_OK;
+}
+
+// A call whose stream is being captured into a graph must not take scratch
+// from the allocator: the block would return to the cache while replays of the
+// graph still use it.
+bool may_allocate(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st == hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return false;
+}
+
+int launch_sum(const GemmArgs& p, hipStream_t s) {
+  const bool vec = p.N % 4 == 0 && p.ldc % 4 == 0 && p.c_sb % 4 == 0 && aligned16(p.c) && aligned16(p.ws);
+  const int64_t items = int64_t(p.batch) * p.M * p.N / (vec ? 4 : 1);
+  const int blocks = int(std::min<int64_t>((items + 255) / 256, 65535));
+  if (vec)
+    hipLaunchKernelGGL(gemm_sum_kernel<true>, dim3(blocks), dim3(256), 0, s, p);
+  else
+    hipLaunchKernelGGL(gemm_sum_kernel<false>, dim3(blocks), dim3(256), 0, s, p);
+  MX_HIP(hipGetLastError());
   return MX_OK;
 }
 
@@ -304,12 +412,12 @@ constexpr const char* kTileNames[] = {"256x128x16", "128x256x16", "128x128x16", 
 extern "C" int mx_gemm_f32(const mx_gemm_desc* d, const float* a, const float* b, const float* bias,
                            float* c, void* stream) {
   MX_ABI_BEGIN
+  hipStream_t s = resolve_stream(stream);
   GemmPlan g;
-  MX_TRY(plan_gemm(d, a, b, bias, c, &g));
+  MX_TRY(plan_gemm(d, a, b, bias, c, may_allocate(s), &g));
   if (g.empty) return MX_OK;
   MX_REQUIRE(c, MX_ERR_INVALID, "mx_gemm_f32: null output");
   MX_REQUIRE(d->bias_kind == MX_BIAS_NONE || bias, MX_ERR_INVALID, "mx_gemm_f32: null bias");
-  hipStream_t s = resolve_stream(stream);
   GemmArgs& p = g.p;
   if (d->k == 0) {
     const int64_t total = d->batch * d->m * d->n;
@@ -319,12 +427,22 @@ extern "C" int mx_gemm_f32(const mx_gemm_desc* d, const float* a, const float* b
     return MX_OK;
   }
   MX_REQUIRE(a && b, MX_ERR_INVALID, "mx_gemm_f32: null operand");
-  switch (g.tile) {
-    case 0: return launch1_vec<TileTall>(p, g.ma, g.mb, s);
-    case 1: return launch1_vec<TileWide>(p, g.ma, g.mb, s);
-    case 2: return launch1<TileSq>(p, g.ma, g.mb, s);
-    default: return launch1<TileSmall>(p, g.ma, g.mb, s);
+  Scratch ws;
+  if (p.splits > 1) {
+    if (ws.alloc(size_t(p.splits) * p.batch * p.M * p.N * 4, s) == MX_OK) {
+      p.ws = ws.as<float>();
+    } else {  // no room for partials: one pass over K
+      clear_error();
+      MX_TRY(plan_gemm(d, a, b, bias, c, false, &g));
+    }
   }
+  switch (g.tile) {
+    case 0: MX_TRY(launch1_vec<TileTall>(p, g.ma, g.mb, s)); break;
+    case 1: MX_TRY(launch1_vec<TileWide>(p, g.ma, g.mb, s)); break;
+    case 2: MX_TRY(launch1<TileSq>(p, g.ma, g.mb, s)); break;
+    default: MX_TRY(launch1<TileSmall>(p, g.ma, g.mb, s));
+  }
+  return p.splits > 1 ? launch_sum(p, s) : MX_OK;
   MX_ABI_END
 }
 
@@ -332,7 +450,7 @@ extern "C" int mx_gemm_variant(const mx_gemm_desc* d, const float* a, const floa
   MX_ABI_BEGIN
   MX_REQUIRE(buf || !len, MX_ERR_INVALID, "mx_gemm_variant: null buffer");
   GemmPlan g;
-  MX_TRY(plan_gemm(d, a, b, nullptr, nullptr, &g));
+  MX_TRY(plan_gemm(d, a, b, nullptr, nullptr, true, &g));
   std::string name;
   if (g.empty) {
     name = "none";
@@ -340,7 +458,7 @@ extern "C" int mx_gemm_variant(const mx_gemm_desc* d, const float* a, const floa
     name = "gemm_k0_kernel";
   } else {
     const int kind = (d->bias_kind == MX_BIAS_NONE || d->beta == 0.f) ? MX_BIAS_NONE : d->bias_kind;
-    name = cat("gemm_kernel<", kTileNames[g.tile], ",", mode_name(g.ma), ",", mode_name(g.mb), ">",
+    name = cat("gemm_kernel<", kTileNames[g.tile], ",", mode_name(g.ma), ",", mode_name(g.mb), ">", g.p.splits > 1 ? "+split" : "",
                kind == MX_BIAS_COL ? "+bias_col" : kind == MX_BIAS_MATRIX ? "+bias_matrix" : "",
                d->batch > 65535 ? "+batch_chunks" : "");
   }

@@ -137,3 +137,49 @@ def test_conv_phases(mx, case, geometry):
     check(dx, grads(0), w, dy)
     check(dw, grads(1), x, dy_w.cpu())
     check(db, lambda a: a.sum((0, 2, 3)), dy_w.cpu())
+
+
+@pytest.mark.parametrize("bias_kind", ["none", "col", "matrix"])
+@pytest.mark.parametrize("m,n,k,batch", [(8, 1000, 2048, None), (1, 37, 1111, None), (65, 130, 4096, None),
+                                         (33, 64, 1500, 3)])
+def test_gemm_k_split(mx, m, n, k, batch, bias_kind):
+    """Few tiles over a long K: partial products of K ranges, summed with alpha,
+    beta and the bias in a second launch."""
+    g = torch.Generator().manual_seed(m + n + k)
+    lead = (batch,) if batch else ()
+    a, b = torch.randn(*lead, m, k, generator=g), torch.randn(*lead, k, n, generator=g)
+    bias = {"none": None, "col": torch.randn(n, generator=g), "matrix": torch.randn(m, n, generator=g)}[bias_kind]
+    ac, bc, c = a.cuda(), b.cuda(), torch.full((*lead, m, n), float("nan"), device="cuda")
+    bd = None if bias is None else bias.cuda()
+    beta = 0.0 if bias is None else -0.5
+    assert "+split" in mx.gemm_variant(mx.gemm_desc(ac, bc, c, bias=bd, alpha=1.5, beta=beta))
+    mx.gemm(ac, bc, c, bias=bd, alpha=1.5, beta=beta, stream=torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    ref, mag = 1.5 * (a.double() @ b.double()), 1.5 * (a.double().abs() @ b.double().abs())
+    if bias is not None:
+        ref, mag = ref + beta * bias.double(), mag + bias.double().abs()
+    assert ((c.cpu().double() - ref).abs() <= (k / 16 + 72) * 2.0 ** -23 * mag).all()
+
+
+def test_gemm_under_capture_takes_no_scratch(mx):
+    """A captured call runs in one pass: replays read and write only the
+    operands, whatever the allocator does between them."""
+    a, b = torch.randn(8, 2048, device="cuda"), torch.randn(2048, 1000, device="cuda")
+    c, eager = torch.empty(8, 1000, device="cuda"), torch.empty(8, 1000, device="cuda")
+    s = torch.cuda.Stream()
+    mx.gemm(a, b, c, stream=s.cuda_stream)  # loads the kernels
+    torch.cuda.synchronize()
+    before = mx.memory_stats().device_mallocs if hasattr(mx, "memory_stats") else None
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        mx.gemm(a, b, c, stream=s.cuda_stream)
+    for i in range(3):
+        a.normal_()
+        c.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        mx.gemm(a, b, eager, stream=s.cuda_stream)
+        torch.cuda.synchronize()
+        assert ((c - eager).norm() / eager.norm()).item() < 2e-6
+    assert before is None or mx.memory_stats().device_mallocs == before
