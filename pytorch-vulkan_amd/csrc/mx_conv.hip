@@ -27,6 +27,8 @@ namespace mx {
 namespace {
 
 using conv::ConvArgs;
+using conv::FastDiv;
+using conv::fdiv;
 using mfma::Mode;
 
 // ----------------------------------------------------------- direct kernels
@@ -113,28 +115,198 @@ __global__ void conv_dw_direct_kernel(ConvArgs p) {
   }
 }
 
-// Depthwise forward (groups == Cin, Cout = m * Cin; conv2d_depthwise.comp:15-41).
-// One workgroup per (image, input channel, 16 x 64 output tile): the input
-// patch the tile reads (halo and zero padding included) is staged once in LDS
-// and all m output channels that read this input channel are computed from
-// it, so x is read from HBM once per tile and y written once.  Wave w owns
-// output rows 4w .. 4w+3 of the tile, lane l output column l.  Each output
-// starts from its bias and adds the taps in (kh, kw) order, as the shader
-// does; a padded tap adds 0 * w.  A patch larger than the LDS budget (very
-// large dilation) reads x directly (kStaged = false).
-constexpr int kDwTileW = 64, kDwTileH = 16, kDwRowsPerWave = 4;
+// Depthwise layers (groups == Cin, Cout = m * Cin; conv2d_depthwise.comp:15-41)
+// are bound by memory and by the index work around a handful of multiply-adds
+// per value.  A workgroup stages the patches of several (image, channel)
+// planes in LDS, zeros where the patch leaves the plane, and its threads take
+// items of four rows of one column, all columns of all its planes numbered
+// through, so planes smaller than a wave's 64 columns leave no lane idle and a
+// value is read from HBM once.  32 x 192 x 28 x 28, 3x3: forward 71.6 -> 12,
+// input gradient (one thread per value before) 65 -> 15 us.
+constexpr int kDwRows = 4;           // rows of an item
 constexpr int kDwLdsFloats = 12288;  // 48 KiB
+// Tile of the kernel that reads x directly where a patch is larger than that
+// (very large dilation).
+constexpr int kDwTileW = 64, kDwTileH = 16, kDwRowsPerWave = 4;
 
 struct DepthwiseArgs {
   ConvArgs p;
-  int tiles_w, tiles_h;
+  int tile_h, tile_w, tiles_h, tiles_w, strips;  // one plane's tile, tile_h = strips * kDwRows
+  int planes;                                    // planes of one workgroup
+  int total_planes;
+  int patch_h, patch_w, patch;  // staged rows, columns and floats of one plane's tile
   int64_t tiles;
-  int patch_h, patch_w;  // staged input rows / columns of one tile
+  FastDiv f_tw, f_strips, f_pw, f_patch, f_cin, f_sh, f_sw;
 };
 
-template <bool kStaged>
+// Items of a tile: f(plane in the workgroup, first row, column).
+template <class F>
+__device__ __forceinline__ void depthwise_items(const DepthwiseArgs& a, int np, F&& f) {
+  for (uint32_t it = threadIdx.x; it < uint32_t(np * a.strips * a.tile_w); it += 256) {
+    const uint32_t q = fdiv(it, a.f_tw), pl = fdiv(q, a.f_strips);
+    f(int(pl), int(q - pl * a.strips) * kDwRows, int(it - q * a.tile_w));
+  }
+}
+
+// Forward: each output starts from its bias and adds the taps in (kh, kw)
+// order, as the shader does; a padded tap adds 0 * w.  K > 0: a K x K filter.
+template <int K>
+__global__ __launch_bounds__(256) void conv_depthwise_staged_kernel(DepthwiseArgs a) {
+  extern __shared__ float patch[];
+  const ConvArgs& p = a.p;
+  const int KH = K ? K : p.KH, KW = K ? K : p.KW, m = p.Cout_g;
+  for (int64_t t = blockIdx.x; t < a.tiles; t += gridDim.x) {
+    const int tw = int(t % a.tiles_w), th = int((t / a.tiles_w) % a.tiles_h);
+    const int plane0 = int(t / (int64_t(a.tiles_w) * a.tiles_h)) * a.planes;
+    const int np = min(a.planes, a.total_planes - plane0);
+    const int oh0 = th * a.tile_h, ow0 = tw * a.tile_w;
+    const int ih0 = oh0 * p.sh - p.ph, iw0 = ow0 * p.sw - p.pw;
+    const float* const xp = p.x + int64_t(plane0) * p.HW;
+    for (uint32_t e = threadIdx.x; e < uint32_t(np * a.patch); e += 256) {
+      const uint32_t pl = fdiv(e, a.f_patch), q = e - pl * a.patch, r = fdiv(q, a.f_pw);
+      const int ih = ih0 + int(r), iw = iw0 + int(q - r * a.patch_w);
+      patch[e] = unsigned(ih) < unsigned(p.H) && unsigned(iw) < unsigned(p.W) ? xp[pl * p.HW + ih * p.W + iw] : 0.f;
+    }
+    __syncthreads();
+    for (int j = 0; j < m; ++j)
+      depthwise_items(a, np, [&](int pl, int row, int col) {
+        const uint32_t plane = plane0 + pl, img = fdiv(plane, a.f_cin);
+        const int oc = int(plane - img * p.Cin) * m + j;
+        const float* const wk = p.w + int64_t(oc) * (KH * KW);
+        const float* const src = patch + pl * a.patch + row * p.sh * a.patch_w + col * p.sw;
+        float acc[kDwRows];
+        const float b = p.bias ? p.bias[oc] : 0.f;
+#pragma unroll
+        for (int r = 0; r < kDwRows; ++r) acc[r] = b;
+#pragma unroll(K ? K : 1)
+        for (int kh = 0; kh < KH; ++kh)
+#pragma unroll(K ? K : 1)
+          for (int kw = 0; kw < KW; ++kw) {
+            const float wv = wk[kh * KW + kw];
+#pragma unroll
+            for (int r = 0; r < kDwRows; ++r)
+              acc[r] += src[(r * p.sh + kh * p.dh) * a.patch_w + kw * p.dw] * wv;
+          }
+        float* const yp = p.out + (int64_t(img) * p.Cout + oc) * p.OHOW + (oh0 + row) * p.OW + ow0 + col;
+#pragma unroll
+        for (int r = 0; r < kDwRows; ++r)
+          if (oh0 + row + r < p.OH && ow0 + col < p.OW) yp[r * p.OW] = acc[r];
+      });
+    __syncthreads();  // the next tile restages the patches
+  }
+}
+
+// Input gradient: dx[ih][iw] = sum over output channel j of the channel and
+// taps of w * dy[(ih + ph - kh dh) / sh][...] where the division is exact, in
+// (j, kh, kw) order.  The patches hold dy of the m output channels.  UNIT:
+// stride 1.
+template <int K, bool UNIT>
+__global__ __launch_bounds__(256) void conv_depthwise_dx_kernel(DepthwiseArgs a) {
+  extern __shared__ float patch[];
+  const ConvArgs& p = a.p;
+  const int KH = K ? K : p.KH, KW = K ? K : p.KW, m = p.Cout_g;
+  for (int64_t t = blockIdx.x; t < a.tiles; t += gridDim.x) {
+    const int tw = int(t % a.tiles_w), th = int((t / a.tiles_w) % a.tiles_h);
+    const int plane0 = int(t / (int64_t(a.tiles_w) * a.tiles_h)) * a.planes;
+    const int np = min(a.planes, a.total_planes - plane0);
+    const int ih0 = th * a.tile_h, iw0 = tw * a.tile_w;
+    // First dy row / column any tap of the tile reads (rounded down).
+    const int top = ih0 + p.ph - (KH - 1) * p.dh, left = iw0 + p.pw - (KW - 1) * p.dw;
+    const int oh0 = UNIT ? top : top >= 0 ? top / p.sh : -((p.sh - 1 - top) / p.sh);
+    const int ow0 = UNIT ? left : left >= 0 ? left / p.sw : -((p.sw - 1 - left) / p.sw);
+    const float* const dyp = p.dy + int64_t(plane0) * m * p.OHOW;  // planes of dy follow (image, channel, j)
+    for (uint32_t e = threadIdx.x; e < uint32_t(np * m * a.patch); e += 256) {
+      const uint32_t pl = fdiv(e, a.f_patch), q = e - pl * a.patch, r = fdiv(q, a.f_pw);
+      const int oh = oh0 + int(r), ow = ow0 + int(q - r * a.patch_w);
+      patch[e] = unsigned(oh) < unsigned(p.OH) && unsigned(ow) < unsigned(p.OW) ? dyp[pl * p.OHOW + oh * p.OW + ow]
+                                                                                : 0.f;
+    }
+    __syncthreads();
+    depthwise_items(a, np, [&](int pl, int row, int col) {
+      const uint32_t plane = plane0 + pl, img = fdiv(plane, a.f_cin);
+      const int ic = int(plane - img * p.Cin);
+      const int y0 = ih0 + row + p.ph - oh0 * p.sh, x0 = iw0 + col + p.pw - ow0 * p.sw;
+      float acc[kDwRows] = {};
+      for (int j = 0; j < m; ++j) {
+        const float* const wk = p.w + (int64_t(ic) * m + j) * (KH * KW);
+        const float* const src = patch + (pl * m + j) * a.patch;
+#pragma unroll(K ? K : 1)
+        for (int kh = 0; kh < KH; ++kh)
+#pragma unroll(K ? K : 1)
+          for (int kw = 0; kw < KW; ++kw) {
+            const float wv = wk[kh * KW + kw];
+            const int tx = x0 - kw * p.dw;
+            const int qx = UNIT ? tx : int(fdiv(uint32_t(tx), a.f_sw));
+            const bool xok = UNIT || qx * p.sw == tx;
+#pragma unroll
+            for (int r = 0; r < kDwRows; ++r) {
+              const int ty = y0 + r - kh * p.dh;
+              const int qy = UNIT ? ty : int(fdiv(uint32_t(ty), a.f_sh));
+              if (UNIT || (xok && qy * p.sh == ty)) acc[r] += src[qy * a.patch_w + qx] * wv;
+            }
+          }
+      }
+      float* const dst = p.out + int64_t(plane) * p.HW + (ih0 + row) * p.W + iw0 + col;
+#pragma unroll
+      for (int r = 0; r < kDwRows; ++r)
+        if (ih0 + row + r < p.H && iw0 + col < p.W) dst[r * p.W] = acc[r];
+    });
+    __syncthreads();
+  }
+}
+
+// Depthwise weight gradient, no scratch: one workgroup of 16 waves per (output
+// channel, filter row); a thread takes every 1024th output position with all
+// KW taps of the row (x from the caches), the sums meet in a fixed tree.  Row
+// 0's workgroup also sums dBias from the dy it reads.  One workgroup per
+// weight, with 64-bit divisions per position, took 121 us plus 38 us for dBias
+// at 32 x 192 x 28 x 28, 3x3.
+template <int KW>
+__global__ __launch_bounds__(1024) void conv_depthwise_dw_kernel(ConvArgs p) {
+  __shared__ float part[16][KW + 1];
+  const int oc = blockIdx.x, kh = blockIdx.y, ic = oc / p.Cout_g;
+  float acc[KW + 1] = {};
+  const uint32_t positions = uint32_t(p.N) * uint32_t(p.OHOW);
+#pragma unroll 2
+  for (uint32_t r = threadIdx.x; r < positions; r += 1024) {
+    const uint32_t img = fdiv(r, p.f_ohow), q = r - img * uint32_t(p.OHOW), oh = fdiv(q, p.f_ow);
+    const int ih = int(oh) * p.sh - p.ph + kh * p.dh, iw0 = int(q - oh * uint32_t(p.OW)) * p.sw - p.pw;
+    const float g = p.dy[(img * uint32_t(p.Cout) + oc) * uint32_t(p.OHOW) + q];
+    const float* const xr = p.x + (img * uint32_t(p.Cin) + ic) * uint32_t(p.HW);
+    float xv[KW];
+    bool ok[KW];
+#pragma unroll
+    for (int k = 0; k < KW; ++k) {
+      const int iw = iw0 + k * p.dw;
+      ok[k] = unsigned(ih) < unsigned(p.H) && unsigned(iw) < unsigned(p.W);
+      xv[k] = xr[ok[k] ? ih * p.W + iw : 0];
+    }
+#pragma unroll
+    for (int k = 0; k < KW; ++k) acc[k] += ok[k] ? xv[k] * g : 0.f;
+    acc[KW] += g;
+  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int k = 0; k <= KW; ++k) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) acc[k] += __shfl_xor(acc[k], d);
+    if (lane == 0) part[wave][k] = acc[k];
+  }
+  __syncthreads();
+  if (threadIdx.x <= KW) {
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s += part[i][threadIdx.x];
+    if (threadIdx.x < KW)
+      p.out[(int64_t(oc) * p.KH + kh) * KW + threadIdx.x] = s;
+    else if (kh == 0 && p.db)
+      p.db[oc] = s;
+  }
+}
+
+// Forward where no patch fits in LDS: wave w owns output rows 4w .. 4w + 3 of
+// a 16 x 64 tile, lane l output column l, x read directly.
 __global__ __launch_bounds__(256) void conv_depthwise_kernel(DepthwiseArgs a) {
-  __shared__ float patch[kStaged ? kDwLdsFloats : 1];
   const ConvArgs& p = a.p;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = p.Cout_g;
@@ -147,15 +319,6 @@ __global__ __launch_bounds__(256) void conv_depthwise_kernel(DepthwiseArgs a) {
     const float* xp = p.x + plane * p.HW;
     const int oh0 = th * kDwTileH, ow0 = tw * kDwTileW;
     const int ih0 = oh0 * p.sh - p.ph, iw0 = ow0 * p.sw - p.pw;
-    if constexpr (kStaged) {
-      const int n = a.patch_h * a.patch_w;
-      for (int e = threadIdx.x; e < n; e += 256) {
-        const int r = e / a.patch_w, c = e - r * a.patch_w;
-        const int ih = ih0 + r, iw = iw0 + c;
-        patch[e] = (ih >= 0 && ih < p.H && iw >= 0 && iw < p.W) ? xp[ih * p.W + iw] : 0.f;
-      }
-      __syncthreads();
-    }
     const int ow = ow0 + lane;
     const int orow = wave * kDwRowsPerWave;
     for (int j = 0; j < m; ++j) {
@@ -172,14 +335,8 @@ __global__ __launch_bounds__(256) void conv_depthwise_kernel(DepthwiseArgs a) {
 #pragma unroll
           for (int r = 0; r < kDwRowsPerWave; ++r) {
             const int rr = (orow + r) * p.sh + kh * p.dh;
-            float xv;
-            if constexpr (kStaged) {
-              // rr <= 15 sh + (KH-1) dh < patch_h and c <= 63 sw + (KW-1) dw < patch_w.
-              xv = patch[rr * a.patch_w + c];
-            } else {
-              const int ih = ih0 + rr, iw = iw0 + c;
-              xv = (ih >= 0 && ih < p.H && iw >= 0 && iw < p.W) ? xp[ih * p.W + iw] : 0.f;
-            }
+            const int ih = ih0 + rr, iw = iw0 + c;
+            const float xv = (ih >= 0 && ih < p.H && iw >= 0 && iw < p.W) ? xp[ih * p.W + iw] : 0.f;
             acc[r] += xv * wv;
           }
         }
@@ -190,7 +347,6 @@ __global__ __launch_bounds__(256) void conv_depthwise_kernel(DepthwiseArgs a) {
         if (oh < p.OH && ow < p.OW) yp[oh * p.OW + ow] = acc[r];
       }
     }
-    if constexpr (kStaged) __syncthreads();  // the next tile restages the patch
   }
 }
 
@@ -227,24 +383,38 @@ __global__ __launch_bounds__(256) void conv_dw_reduce_kernel(ConvArgs p) {
   }
 }
 
-// dBias: one workgroup per output channel, strided partial sums + LDS tree.
-__global__ __launch_bounds__(256) void conv_db_reduce_kernel(ConvArgs p) {
-  __shared__ float part[256];
-  const int64_t positions = int64_t(p.N) * p.OHOW;
+// dBias: one workgroup of 16 waves per output channel, a wave per image plane
+// in turn (16 bytes a lane where VEC), summed in a fixed tree.
+template <bool VEC>
+__global__ __launch_bounds__(1024) void conv_db_reduce_kernel(ConvArgs p) {
+  __shared__ float part[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int oc = blockIdx.x; oc < p.Cout; oc += gridDim.x) {
     float sum = 0.f;
-    for (int64_t r = threadIdx.x; r < positions; r += 256) {
-      const int img = int(r / p.OHOW);
-      const int q = int(r - int64_t(img) * p.OHOW);
-      sum += p.dy[(int64_t(img) * p.Cout + oc) * p.OHOW + q];
+    for (int img = wave; img < p.N; img += 16) {
+      const float* const src = p.dy + (int64_t(img) * p.Cout + oc) * p.OHOW;
+      if constexpr (VEC) {
+        const float4* const v4 = reinterpret_cast<const float4*>(src);
+#pragma unroll 4
+        for (int i = lane; i < p.OHOW / 4; i += 64) {
+          const float4 v = v4[i];
+          sum += (v.x + v.y) + (v.z + v.w);
+        }
+      } else {
+#pragma unroll 4
+        for (int i = lane; i < p.OHOW; i += 64) sum += src[i];
+      }
     }
-    part[threadIdx.x] = sum;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d);
+    if (lane == 0) part[wave] = sum;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-      if (int(threadIdx.x) < s) part[threadIdx.x] += part[threadIdx.x + s];
-      __syncthreads();
+    if (threadIdx.x == 0) {
+      float s = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s += part[i];
+      p.db[oc] = s;
     }
-    if (threadIdx.x == 0) p.db[oc] = part[0];
     __syncthreads();
   }
 }
@@ -325,6 +495,46 @@ bool depthwise_staged(const mx_conv2d_desc& d) {
   return ph * pw <= kDwLdsFloats;
 }
 
+// Tile of the staged depthwise kernels over planes of h x w values, of which
+// `per_plane` patches each are staged: columns up to 64, rows up to about 1024
+// values (a multiple of an item's rows), then as many planes as make up about
+// 3072 values, all within the LDS budget.  patch_dim(tile extent, axis) gives
+// the patch's rows / columns.  False when not even four rows fit.
+template <class F>
+bool depthwise_tile(DepthwiseArgs* a, int h, int w, int per_plane, F&& patch_dim) {
+  a->tile_w = std::min(w, kDwTileW);
+  a->patch_w = int(std::min<int64_t>(patch_dim(a->tile_w, 1), INT32_MAX));
+  int rows = std::min((h + kDwRows - 1) / kDwRows, std::max(1, 1024 / a->tile_w / kDwRows)) * kDwRows;
+  for (;; rows -= kDwRows) {
+    if (rows <= 0) return false;
+    const int64_t floats = int64_t(patch_dim(rows, 0)) * a->patch_w;
+    if (floats * per_plane <= kDwLdsFloats) {
+      a->patch_h = int(patch_dim(rows, 0));
+      a->patch = int(floats);
+      break;
+    }
+  }
+  a->tile_h = rows;
+  a->strips = rows / kDwRows;
+  a->tiles_h = (h + rows - 1) / rows;
+  a->tiles_w = (w + a->tile_w - 1) / a->tile_w;
+  a->total_planes = a->p.N * a->p.Cin;
+  a->planes = std::max(1, std::min({3072 / (rows * a->tile_w), kDwLdsFloats / (a->patch * per_plane), a->total_planes}));
+  a->tiles = int64_t((a->total_planes + a->planes - 1) / a->planes) * a->tiles_w * a->tiles_h;
+  a->f_tw = conv::fast_div(uint32_t(a->tile_w));
+  a->f_strips = conv::fast_div(uint32_t(a->strips));
+  a->f_pw = conv::fast_div(uint32_t(a->patch_w));
+  a->f_patch = conv::fast_div(uint32_t(a->patch));
+  a->f_cin = conv::fast_div(uint32_t(a->p.Cin));
+  a->f_sh = conv::fast_div(uint32_t(a->p.sh));
+  a->f_sw = conv::fast_div(uint32_t(a->p.sw));
+  return true;
+}
+
+size_t depthwise_lds(const DepthwiseArgs& a, int per_plane) {
+  return size_t(a.planes) * per_plane * a.patch * sizeof(float);
+}
+
 int conv_depthwise_forward(const mx_conv2d_desc& d, const float* x, const float* w, const float* bias, float* y,
                            hipStream_t s) {
   DepthwiseArgs a{};
@@ -333,20 +543,80 @@ int conv_depthwise_forward(const mx_conv2d_desc& d, const float* x, const float*
   a.p.w = w;
   a.p.bias = bias;
   a.p.out = y;
-  a.tiles_w = int((d.ow + kDwTileW - 1) / kDwTileW);
-  a.tiles_h = int((d.oh + kDwTileH - 1) / kDwTileH);
-  a.tiles = d.n * d.cin * a.tiles_w * a.tiles_h;
-  if (a.tiles == 0) return MX_OK;
-  const dim3 grid(unsigned(std::min<int64_t>(a.tiles, 1 << 20)));
-  if (depthwise_staged(d)) {
-    a.patch_h = int((kDwTileH - 1) * d.sh + (d.kh - 1) * d.dh + 1);
-    a.patch_w = int((kDwTileW - 1) * d.sw + (d.kw - 1) * d.dw + 1);
-    hipLaunchKernelGGL(conv_depthwise_kernel<true>, grid, dim3(256), 0, s, a);
+  const auto patch_dim = [&](int64_t n, int axis) {
+    return (n - 1) * (axis ? d.sw : d.sh) + (axis ? (d.kw - 1) * d.dw : (d.kh - 1) * d.dh) + 1;
+  };
+  if (depthwise_staged(d) && depthwise_tile(&a, int(d.oh), int(d.ow), 1, patch_dim)) {
+    const dim3 grid(unsigned(std::min<int64_t>(a.tiles, 1 << 20)));
+    const size_t lds = depthwise_lds(a, 1);
+    if (d.kh == 3 && d.kw == 3)
+      hipLaunchKernelGGL(conv_depthwise_staged_kernel<3>, grid, dim3(256), lds, s, a);
+    else if (d.kh == 5 && d.kw == 5)
+      hipLaunchKernelGGL(conv_depthwise_staged_kernel<5>, grid, dim3(256), lds, s, a);
+    else
+      hipLaunchKernelGGL(conv_depthwise_staged_kernel<0>, grid, dim3(256), lds, s, a);
   } else {
-    hipLaunchKernelGGL(conv_depthwise_kernel<false>, grid, dim3(256), 0, s, a);
+    a.tiles_w = int((d.ow + kDwTileW - 1) / kDwTileW);
+    a.tiles_h = int((d.oh + kDwTileH - 1) / kDwTileH);
+    a.tiles = d.n * d.cin * a.tiles_w * a.tiles_h;
+    hipLaunchKernelGGL(conv_depthwise_kernel, dim3(unsigned(std::min<int64_t>(a.tiles, 1 << 20))), dim3(256), 0, s, a);
   }
   MX_HIP(hipGetLastError());
   return MX_OK;
+}
+
+bool is_depthwise(const mx_conv2d_desc& d) { return d.groups == d.cin && d.groups > 1; }
+
+// Input gradient of a depthwise layer in place of the one-thread-per-value
+// kernel; false where no patch fits (then nothing was launched).
+bool conv_depthwise_dx(const mx_conv2d_desc& d, const ConvArgs& p, hipStream_t s) {
+  DepthwiseArgs a{};
+  a.p = p;
+  const int64_t m = d.cout / d.groups;
+  const auto patch_dim = [&](int64_t n, int axis) {
+    return (n - 1 + (axis ? (d.kw - 1) * d.dw : (d.kh - 1) * d.dh)) / (axis ? d.sw : d.sh) + 2;
+  };
+  if (m > kDwLdsFloats || !depthwise_tile(&a, int(d.h), int(d.w), int(m), patch_dim)) return false;
+  const dim3 grid(unsigned(std::min<int64_t>(a.tiles, 1 << 20)));
+  const size_t lds = depthwise_lds(a, int(m));
+  const int k = d.kh == d.kw && (d.kh == 3 || d.kh == 5) ? int(d.kh) : 0;
+  const bool unit = d.sh == 1 && d.sw == 1;
+#define MX_DW_DX(K)                                                                                     \
+  if (unit)                                                                                             \
+    hipLaunchKernelGGL((conv_depthwise_dx_kernel<K, true>), grid, dim3(256), lds, s, a);                \
+  else                                                                                                  \
+    hipLaunchKernelGGL((conv_depthwise_dx_kernel<K, false>), grid, dim3(256), lds, s, a);
+  if (k == 3) {
+    MX_DW_DX(3)
+  } else if (k == 5) {
+    MX_DW_DX(5)
+  } else {
+    MX_DW_DX(0)
+  }
+#undef MX_DW_DX
+  return true;
+}
+
+// Weight gradient (and dBias) of a depthwise layer with 1, 3, 5 or 7 filter
+// columns in place of the one-workgroup-per-weight reduction; false otherwise.
+bool conv_depthwise_dw(const mx_conv2d_desc& d, const ConvArgs& p, hipStream_t s) {
+  if (d.cout > INT32_MAX / 16 || d.kh > 65535) return false;
+  const dim3 grid(unsigned(d.cout), unsigned(d.kh));
+  switch (d.kw) {
+    case 1: hipLaunchKernelGGL(conv_depthwise_dw_kernel<1>, grid, dim3(1024), 0, s, p); return true;
+    case 3: hipLaunchKernelGGL(conv_depthwise_dw_kernel<3>, grid, dim3(1024), 0, s, p); return true;
+    case 5: hipLaunchKernelGGL(conv_depthwise_dw_kernel<5>, grid, dim3(1024), 0, s, p); return true;
+    case 7: hipLaunchKernelGGL(conv_depthwise_dw_kernel<7>, grid, dim3(1024), 0, s, p); return true;
+    default: return false;
+  }
+}
+
+void launch_db_reduce(const ConvArgs& p, hipStream_t s) {
+  const dim3 grid(unsigned(std::min<int64_t>(p.Cout, 65535)));
+  if (p.OHOW % 4 == 0 && (reinterpret_cast<uintptr_t>(p.dy) & 15) == 0)
+    hipLaunchKernelGGL(conv_db_reduce_kernel<true>, grid, dim3(1024), 0, s, p);
+  else
+    hipLaunchKernelGGL(conv_db_reduce_kernel<false>, grid, dim3(1024), 0, s, p);
 }
 
 int linear_blocks(int64_t total) { return int(std::min<int64_t>((total + 255) / 256, 1 << 20)); }
@@ -1156,7 +1426,8 @@ int mx_conv2d_backward_input(const mx_conv2d_desc* desc, const float* dy, const 
     p.dy = dy;
     p.w = w;
     p.out = dx;
-    hipLaunchKernelGGL(conv_dx_direct_kernel, dim3(linear_blocks(d.n * d.cin * d.h * d.w)), dim3(256), 0, s, p);
+    if (!is_depthwise(d) || !conv_depthwise_dx(d, p, s))
+      hipLaunchKernelGGL(conv_dx_direct_kernel, dim3(linear_blocks(d.n * d.cin * d.h * d.w)), dim3(256), 0, s, p);
     MX_HIP(hipGetLastError());
     return MX_OK;
   }
@@ -1227,7 +1498,7 @@ int mx_conv2d_backward_bias(const mx_conv2d_desc* desc, const float* dy, float* 
   if (chosen == MX_CONV_ALGO_DIRECT)
     hipLaunchKernelGGL(conv_db_direct_kernel, dim3(linear_blocks(d.cout)), dim3(256), 0, s, p);
   else
-    hipLaunchKernelGGL(conv_db_reduce_kernel, dim3(unsigned(std::min<int64_t>(d.cout, 65535))), dim3(256), 0, s, p);
+    launch_db_reduce(p, s);
   MX_HIP(hipGetLastError());
   return MX_OK;
   MX_ABI_END
@@ -1271,6 +1542,11 @@ int dweight_impl(const mx_conv2d_desc* desc, const float* x, const float* dy, fl
     p.x = x;
     p.dy = dy;
     p.out = dw;
+    p.db = db;
+    if (chosen == MX_CONV_ALGO_REDUCE && is_depthwise(d) && conv_depthwise_dw(d, p, s)) {
+      MX_HIP(hipGetLastError());
+      return MX_OK;
+    }
     if (chosen == MX_CONV_ALGO_DIRECT)
       hipLaunchKernelGGL(conv_dw_direct_kernel, dim3(linear_blocks(d.cout * (d.cin / d.groups) * d.kh * d.kw)),
                          dim3(256), 0, s, p);

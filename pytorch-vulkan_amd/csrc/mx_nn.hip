@@ -170,33 +170,56 @@ __device__ __forceinline__ void wave_max_n(float (&v)[R]) {
 }
 
 // ------------------------------------------------------------ row statistics
+// Where a row's statistics go: rows in order, or for BatchNorm (tn = N
+// samples) all samples of a channel together, [C][N], so that the merge reads
+// them contiguously.
+__device__ __forceinline__ int64_t stat_index(int64_t r, int C, int tn) {
+  return tn ? (r % C) * tn + r / C : r;
+}
+
 // mean_r and M2_r = sum (x - mean_r)^2 of each row of `hw` contiguous floats.
+// Rows of up to 1024 floats (VEC) stay in registers between the two sums.
 template <bool VEC>
 __global__ __launch_bounds__(kThreads) void row_moments_kernel(const float* __restrict__ x, int64_t rows, int hw,
-                                                               float* __restrict__ rmean, float* __restrict__ rm2) {
+                                                               int C, int tn, float* __restrict__ rmean,
+                                                               float* __restrict__ rm2) {
   const int lane = threadIdx.x & 63;
   const int64_t r = int64_t(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6);
   if (r >= rows) return;
   const float* p = x + r * hw;
+  const float4* p4 = reinterpret_cast<const float4*>(p);
+  constexpr int NREG = 4;
+  const bool regs = VEC && hw <= 64 * 4 * NREG;
+  float4 v[NREG];
   float s = 0.f;
-  if (VEC) {
-    const float4* p4 = reinterpret_cast<const float4*>(p);
+  if (regs) {
+#pragma unroll
+    for (int k = 0; k < NREG; ++k) {
+      const int i = lane + 64 * k;
+      v[k] = i < hw / 4 ? p4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int k = 0; k < NREG; ++k) s += (v[k].x + v[k].y) + (v[k].z + v[k].w);
+  } else if (VEC) {
     for (int i = lane; i < hw / 4; i += 64) {
-      const float4 v = p4[i];
-      s += (v.x + v.y) + (v.z + v.w);
+      const float4 t = p4[i];
+      s += (t.x + t.y) + (t.z + t.w);
     }
   } else {
     for (int i = lane; i < hw; i += 64) s += p[i];
   }
   const float m = wave_sum(s) / float(hw);
   float q = 0.f;
-  if (VEC) {
-    const float4* p4 = reinterpret_cast<const float4*>(p);
-    for (int i = lane; i < hw / 4; i += 64) {
-      const float4 v = p4[i];
-      const float a = v.x - m, b = v.y - m, c = v.z - m, d = v.w - m;
-      q += (a * a + b * b) + (c * c + d * d);
-    }
+  const auto spread = [&](const float4& t) {
+    const float a = t.x - m, b = t.y - m, c = t.z - m, d = t.w - m;
+    q += (a * a + b * b) + (c * c + d * d);
+  };
+  if (regs) {
+#pragma unroll
+    for (int k = 0; k < NREG; ++k)
+      if (lane + 64 * k < hw / 4) spread(v[k]);
+  } else if (VEC) {
+    for (int i = lane; i < hw / 4; i += 64) spread(p4[i]);
   } else {
     for (int i = lane; i < hw; i += 64) {
       const float a = p[i] - m;
@@ -205,8 +228,9 @@ __global__ __launch_bounds__(kThreads) void row_moments_kernel(const float* __re
   }
   q = wave_sum(q);
   if (lane == 0) {
-    rmean[r] = m;
-    rm2[r] = q;
+    const int64_t o = stat_index(r, C, tn);
+    rmean[o] = m;
+    rm2[o] = q;
   }
 }
 
@@ -216,8 +240,8 @@ __global__ __launch_bounds__(kThreads) void row_moments_kernel(const float* __re
 template <bool VEC>
 __global__ __launch_bounds__(kThreads) void row_grad_kernel(const float* __restrict__ dy, const float* __restrict__ x,
                                                             const float* __restrict__ mean, int64_t rows, int hw,
-                                                            int C, int stat_n, int cpg, float* __restrict__ sdy,
-                                                            float* __restrict__ sdyx) {
+                                                            int C, int stat_n, int cpg, int tn,
+                                                            float* __restrict__ sdy, float* __restrict__ sdyx) {
   const int lane = threadIdx.x & 63;
   const int64_t r = int64_t(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6);
   if (r >= rows) return;
@@ -243,8 +267,9 @@ __global__ __launch_bounds__(kThreads) void row_grad_kernel(const float* __restr
   a = wave_sum(a);
   b = wave_sum(b);
   if (lane == 0) {
-    sdy[r] = a;
-    sdyx[r] = b;
+    const int64_t o = stat_index(r, C, tn);
+    sdy[o] = a;
+    sdyx[o] = b;
   }
 }
 
@@ -899,71 +924,129 @@ __global__ __launch_bounds__(64 * W) void gn_bwd_regs_kernel(const float* __rest
 }
 
 // ---------------------------------------------------------------- BatchNorm
-// One thread per channel: merge the N rows of channel c.  Training: batch
-// mean / inverse std (0 when var == eps == 0, as torch's InvStd) and the
-// running-statistics update with the unbiased variance; evaluation: running
-// statistics.  Writes the forward coefficients of every row of the channel.
-__global__ void bn_merge_kernel(const float* __restrict__ rmean, const float* __restrict__ rm2,
-                                const float* __restrict__ gamma, const float* __restrict__ beta,
-                                float* __restrict__ run_mean, int64_t rm_stride, float* __restrict__ run_var,
-                                int64_t rv_stride, int N, int C, int hw, int training, float momentum, float eps,
-                                float* __restrict__ save_mean, float* __restrict__ save_inv,
-                                float4* __restrict__ coef) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= C) return;
-  float m, inv;
-  if (training) {
-    float s = 0.f;
-    for (int n = 0; n < N; ++n) s += rmean[int64_t(n) * C + c];
-    m = s / float(N);
-    float m2 = 0.f, spread = 0.f;
-    for (int n = 0; n < N; ++n) {
-      const float d = rmean[int64_t(n) * C + c] - m;
-      m2 += rm2[int64_t(n) * C + c];
-      spread += d * d;
-    }
-    m2 += spread * float(hw);
-    const float cnt = float(N) * float(hw);
-    const float var = m2 / cnt;
-    inv = (var == 0.f && eps == 0.f) ? 0.f : 1.f / sqrtf(var + eps);
-    save_mean[c] = m;
-    save_inv[c] = inv;
-    if (run_mean) run_mean[c * rm_stride] = momentum * m + (1.f - momentum) * run_mean[c * rm_stride];
-    if (run_var) run_var[c * rv_stride] = momentum * (m2 / (cnt - 1.f)) + (1.f - momentum) * run_var[c * rv_stride];
-  } else {
-    m = run_mean[c * rm_stride];
-    inv = 1.f / sqrtf(run_var[c * rv_stride] + eps);
-  }
-  const float a = gamma ? inv * gamma[c] : inv, b = beta ? beta[c] : 0.f;
-  for (int n = 0; n < N; ++n) coef[int64_t(n) * C + c] = make_float4(m, a, b, 0.f);
+// The merge of a channel's N row statistics runs inside the pass that applies
+// them: every wave sums the channel's [C][N] statistics itself (N / 64 loads a
+// lane, from L2) and then takes its rows, blockIdx.x = channel * chunks +
+// chunk, rows_per_wave rows to a wave.  A merge launch of one thread per
+// channel walked the N samples serially on C / 256 workgroups, 34 us forward
+// and 19 us backward at 64 x 128 x 28 x 28, more than the data takes.
+struct BnArgs {
+  const float *a, *b;  // [C][N] statistics: row means and M2, or sums of dy and of dy * (x - mean)
+  const float *gamma, *beta;
+  float *run_mean, *run_var;
+  int64_t rm_stride, rv_stride;
+  const float *mean, *inv_or_var;  // backward
+  float *out0, *out1;              // forward: saved mean and inverse std; backward: dgamma and dbeta
+  int N, C, hw, chunks, rows_per_wave, training;
+  float momentum, eps;
+};
+
+// f(row offset in floats) for every row of this wave.
+template <class F>
+__device__ __forceinline__ void bn_rows(const BnArgs& p, int c, int chunk, F&& f) {
+  const int64_t first = (int64_t(chunk) * kWavesPerBlock + (threadIdx.x >> 6)) * p.rows_per_wave;
+  for (int64_t n = first; n < p.N && n < first + p.rows_per_wave; ++n) f((n * p.C + c) * p.hw);
 }
 
-// One thread per channel: dx coefficients and the affine gradients.
+// Training: batch mean / inverse std (0 when var == eps == 0, as torch's
+// InvStd) and the running-statistics update with the unbiased variance;
+// evaluation: running statistics.
+template <bool VEC>
+__global__ __launch_bounds__(kThreads) void bn_apply_kernel(BnArgs p, const float* __restrict__ x,
+                                                            float* __restrict__ y) {
+  const int c = blockIdx.x / p.chunks, chunk = blockIdx.x - c * p.chunks, lane = threadIdx.x & 63;
+  float m, inv;
+  if (p.training) {
+    const float *rmean = p.a + int64_t(c) * p.N, *rm2 = p.b + int64_t(c) * p.N;
+    float s = 0.f;
+    for (int n = lane; n < p.N; n += 64) s += rmean[n];
+    m = wave_sum(s) / float(p.N);
+    float m2 = 0.f, spread = 0.f;
+    for (int n = lane; n < p.N; n += 64) {
+      const float d = rmean[n] - m;
+      m2 += rm2[n];
+      spread += d * d;
+    }
+    m2 = wave_sum(m2) + wave_sum(spread) * float(p.hw);
+    const float cnt = float(p.N) * float(p.hw);
+    const float var = m2 / cnt;
+    inv = (var == 0.f && p.eps == 0.f) ? 0.f : 1.f / sqrtf(var + p.eps);
+    if (chunk == 0 && threadIdx.x == 0) {
+      p.out0[c] = m;
+      p.out1[c] = inv;
+      if (p.run_mean) {
+        float& r = p.run_mean[c * p.rm_stride];
+        r = p.momentum * m + (1.f - p.momentum) * r;
+      }
+      if (p.run_var) {
+        float& r = p.run_var[c * p.rv_stride];
+        r = p.momentum * (m2 / (cnt - 1.f)) + (1.f - p.momentum) * r;
+      }
+    }
+  } else {
+    m = p.run_mean[c * p.rm_stride];
+    inv = 1.f / sqrtf(p.run_var[c * p.rv_stride] + p.eps);
+  }
+  const float a = p.gamma ? inv * p.gamma[c] : inv, b = p.beta ? p.beta[c] : 0.f;
+  bn_rows(p, c, chunk, [&](int64_t at) {
+    if (VEC) {
+      const float4* x4 = reinterpret_cast<const float4*>(x + at);
+      float4* y4 = reinterpret_cast<float4*>(y + at);
+#pragma unroll 4
+      for (int i = lane; i < p.hw / 4; i += 64) {
+        const float4 v = x4[i];
+        y4[i] = make_float4((v.x - m) * a + b, (v.y - m) * a + b, (v.z - m) * a + b, (v.w - m) * a + b);
+      }
+    } else {
+#pragma unroll 4
+      for (int i = lane; i < p.hw; i += 64) y[at + i] = (x[at + i] - m) * a + b;
+    }
+  });
+}
+
+// Affine gradients and, where dx is wanted,
 //   training: dx = gamma*inv*(dy - S1/M - (x-mean)*inv^2*S2/M)
 //   eval:     dx = gamma*inv*dy   (inv from the running variance)
-__global__ void bn_grad_merge_kernel(const float* __restrict__ sdy, const float* __restrict__ sdyx,
-                                     const float* __restrict__ mean, const float* __restrict__ inv_or_var,
-                                     const float* __restrict__ gamma, int N, int C, int hw, int training, float eps,
-                                     float* __restrict__ dgamma, float* __restrict__ dbeta,
-                                     float4* __restrict__ coef) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= C) return;
+template <bool VEC>
+__global__ __launch_bounds__(kThreads) void bn_grad_apply_kernel(BnArgs p, const float* __restrict__ dy,
+                                                                 const float* __restrict__ x,
+                                                                 float* __restrict__ dx) {
+  const int c = blockIdx.x / p.chunks, chunk = blockIdx.x - c * p.chunks, lane = threadIdx.x & 63;
+  const float *sdy = p.a + int64_t(c) * p.N, *sdyx = p.b + int64_t(c) * p.N;
   float s1 = 0.f, s2 = 0.f;
-  for (int n = 0; n < N; ++n) {
-    s1 += sdy[int64_t(n) * C + c];
-    s2 += sdyx[int64_t(n) * C + c];
+  for (int n = lane; n < p.N; n += 64) {
+    s1 += sdy[n];
+    s2 += sdyx[n];
   }
-  const float inv = training ? inv_or_var[c] : 1.f / sqrtf(inv_or_var[c] + eps);
-  const float w = gamma ? gamma[c] : 1.f;
-  const float cnt = float(N) * float(hw);
-  if (dgamma) dgamma[c] = s2 * inv;
-  if (dbeta) dbeta[c] = s1;
-  if (!coef) return;
-  const float p = w * inv;
-  const float k = training ? -p * inv * inv * (s2 / cnt) : 0.f;
-  const float q = training ? -p * (s1 / cnt) : 0.f;
-  const float mu = mean[c];
-  for (int n = 0; n < N; ++n) coef[int64_t(n) * C + c] = make_float4(p, k, q, mu);
+  s1 = wave_sum(s1);
+  s2 = wave_sum(s2);
+  const float inv = p.training ? p.inv_or_var[c] : 1.f / sqrtf(p.inv_or_var[c] + p.eps);
+  if (chunk == 0 && threadIdx.x == 0) {
+    if (p.out0) p.out0[c] = s2 * inv;
+    if (p.out1) p.out1[c] = s1;
+  }
+  if (!dx) return;
+  const float cnt = float(p.N) * float(p.hw);
+  const float w = (p.gamma ? p.gamma[c] : 1.f) * inv;
+  const float k = p.training ? -w * inv * inv * (s2 / cnt) : 0.f;
+  const float q = p.training ? -w * (s1 / cnt) : 0.f;
+  const float mu = p.mean[c];
+  bn_rows(p, c, chunk, [&](int64_t at) {
+    if (VEC) {
+      const float4* g4 = reinterpret_cast<const float4*>(dy + at);
+      const float4* x4 = reinterpret_cast<const float4*>(x + at);
+      float4* d4 = reinterpret_cast<float4*>(dx + at);
+#pragma unroll 4
+      for (int i = lane; i < p.hw / 4; i += 64) {
+        const float4 g = g4[i], v = x4[i];
+        d4[i] = make_float4(w * g.x + k * (v.x - mu) + q, w * g.y + k * (v.y - mu) + q, w * g.z + k * (v.z - mu) + q,
+                            w * g.w + k * (v.w - mu) + q);
+      }
+    } else {
+#pragma unroll 4
+      for (int i = lane; i < p.hw; i += 64) dx[at + i] = w * dy[at + i] + k * (x[at + i] - mu) + q;
+    }
+  });
 }
 
 // ------------------------------------------------------------- apply passes
@@ -1439,6 +1522,22 @@ void launch_copy_rows(void* dst, int64_t dst_pitch, const void* src, int64_t src
 
 int launch_rows(int64_t rows) { return int((rows + kWavesPerBlock - 1) / kWavesPerBlock); }
 
+// Rows of a channel per wave of the BatchNorm apply passes: one while that
+// takes at most 16 workgroups per CU, more beyond, so that a workgroup's sum
+// over the channel's statistics is shared by more data.
+BnArgs bn_args(int64_t n, int64_t c, int64_t hw, int training, float eps) {
+  BnArgs p{};
+  p.N = int(n);
+  p.C = int(c);
+  p.hw = int(hw);
+  p.training = training;
+  p.eps = eps;
+  const int64_t groups = launch_rows(n) * c;
+  p.rows_per_wave = int(std::max<int64_t>(1, (groups + 16 * cu_count() - 1) / (16 * cu_count())));
+  p.chunks = launch_rows((n + p.rows_per_wave - 1) / p.rows_per_wave);
+  return p;
+}
+
 // Smallest register-array size of {1, 2, 4, ..., cap} holding `need` float4
 // per thread (0: more than cap).
 int regs_for(int64_t need, int cap = 16) {
@@ -1533,10 +1632,10 @@ int mx_group_norm_forward(const float* x, const float* gamma, const float* beta,
   const bool vec = hw % 4 == 0 && aligned16(x) && aligned16(y);
   if (vec)
     hipLaunchKernelGGL(row_moments_kernel<true>, dim3(launch_rows(rows)), dim3(kThreads), 0, s, x, rows, int(hw),
-                       rmean, rm2);
+                       int(c), 0, rmean, rm2);
   else
     hipLaunchKernelGGL(row_moments_kernel<false>, dim3(launch_rows(rows)), dim3(kThreads), 0, s, x, rows, int(hw),
-                       rmean, rm2);
+                       int(c), 0, rmean, rm2);
   MX_HIP(hipGetLastError());
   const int64_t ng = n * groups;
   hipLaunchKernelGGL(gn_merge_kernel, dim3(int((ng + 255) / 256)), dim3(256), 0, s, rmean, rm2, gamma, beta, int(n),
@@ -1627,10 +1726,10 @@ int mx_group_norm_backward(const float* dy, const float* x, const float* mean, c
   }
   if (vec)
     hipLaunchKernelGGL(row_grad_kernel<true>, dim3(launch_rows(rows)), dim3(kThreads), 0, s, dy, x, mean, rows,
-                       int(hw), int(c), int(groups), cpg, sdy, sdyx);
+                       int(hw), int(c), int(groups), cpg, 0, sdy, sdyx);
   else
     hipLaunchKernelGGL(row_grad_kernel<false>, dim3(launch_rows(rows)), dim3(kThreads), 0, s, dy, x, mean, rows,
-                       int(hw), int(c), int(groups), cpg, sdy, sdyx);
+                       int(hw), int(c), int(groups), cpg, 0, sdy, sdyx);
   MX_HIP(hipGetLastError());
   if (dgamma || dbeta) {
     hipLaunchKernelGGL(gn_affine_kernel, dim3(int((c + 255) / 256)), dim3(256), 0, s, sdy, sdyx, rstd, int(n),
@@ -1670,33 +1769,35 @@ int mx_batch_norm_forward(const float* x, const float* gamma, const float* beta,
              "mx_batch_norm_forward: training requires the saved-statistics outputs");
   hipStream_t s = resolve_stream(stream);
   const int64_t rows = n * c;
-  Scratch stats, coef;
-  MX_TRY(coef.alloc(size_t(rows) * sizeof(float4), s));
+  Scratch stats;
   const bool vec = hw % 4 == 0 && aligned16(x) && aligned16(y);
-  float *rmean = nullptr, *rm2 = nullptr;
+  BnArgs p = bn_args(n, c, hw, training, eps);
   if (training) {
     MX_TRY(stats.alloc(size_t(rows) * 2 * sizeof(float), s));
-    rmean = stats.as<float>();
-    rm2 = rmean + rows;
+    float* const rmean = stats.as<float>();
+    p.a = rmean;
+    p.b = rmean + rows;
     if (vec)
       hipLaunchKernelGGL(row_moments_kernel<true>, dim3(launch_rows(rows)), dim3(kThreads), 0, s, x, rows, int(hw),
-                         rmean, rm2);
+                         int(c), int(n), rmean, rmean + rows);
     else
-      hipLaunchKernelGGL(row_moments_kernel<false>, dim3(launch_rows(rows)), dim3(kThreads), 0, s, x, rows,
-                         int(hw), rmean, rm2);
+      hipLaunchKernelGGL(row_moments_kernel<false>, dim3(launch_rows(rows)), dim3(kThreads), 0, s, x, rows, int(hw),
+                         int(c), int(n), rmean, rmean + rows);
     MX_HIP(hipGetLastError());
   }
-  hipLaunchKernelGGL(bn_merge_kernel, dim3(int((c + 255) / 256)), dim3(256), 0, s, rmean, rm2, gamma, beta,
-                     running_mean, rm_stride, running_var, rv_stride, int(n), int(c), int(hw), training, momentum, eps,
-                     save_mean, save_invstd, coef.as<float4>());
-  MX_HIP(hipGetLastError());
-  const int64_t total = rows * hw;
+  p.gamma = gamma;
+  p.beta = beta;
+  p.run_mean = running_mean;
+  p.rm_stride = rm_stride;
+  p.run_var = running_var;
+  p.rv_stride = rv_stride;
+  p.out0 = save_mean;
+  p.out1 = save_invstd;
+  p.momentum = momentum;
   if (vec)
-    hipLaunchKernelGGL(norm_apply_kernel<true>, dim3(grid_for(total / 4)), dim3(kThreads), 0, s, x,
-                       coef.as<const float4>(), total, int(hw), y);
+    hipLaunchKernelGGL(bn_apply_kernel<true>, dim3(unsigned(c) * p.chunks), dim3(kThreads), 0, s, p, x, y);
   else
-    hipLaunchKernelGGL(norm_apply_kernel<false>, dim3(grid_for(total)), dim3(kThreads), 0, s, x,
-                       coef.as<const float4>(), total, int(hw), y);
+    hipLaunchKernelGGL(bn_apply_kernel<false>, dim3(unsigned(c) * p.chunks), dim3(kThreads), 0, s, p, x, y);
   MX_HIP(hipGetLastError());
   return MX_OK;
   MX_ABI_END
@@ -1712,33 +1813,32 @@ int mx_batch_norm_backward(const float* dy, const float* x, const float* gamma, 
   MX_REQUIRE(dy && x && mean && invstd_or_var, MX_ERR_INVALID, "mx_batch_norm_backward: null tensor");
   hipStream_t s = resolve_stream(stream);
   const int64_t rows = n * c;
-  Scratch sums, coef;
+  Scratch sums;
   MX_TRY(sums.alloc(size_t(rows) * 2 * sizeof(float), s));
   float* sdy = sums.as<float>();
   float* sdyx = sdy + rows;
   const bool vec = hw % 4 == 0 && aligned16(x) && aligned16(dy) && (!dx || aligned16(dx));
   if (vec)
     hipLaunchKernelGGL(row_grad_kernel<true>, dim3(launch_rows(rows)), dim3(kThreads), 0, s, dy, x, mean, rows,
-                       int(hw), int(c), 0, 1, sdy, sdyx);
+                       int(hw), int(c), 0, 1, int(n), sdy, sdyx);
   else
     hipLaunchKernelGGL(row_grad_kernel<false>, dim3(launch_rows(rows)), dim3(kThreads), 0, s, dy, x, mean, rows,
-                       int(hw), int(c), 0, 1, sdy, sdyx);
+                       int(hw), int(c), 0, 1, int(n), sdy, sdyx);
   MX_HIP(hipGetLastError());
-  if (dx) MX_TRY(coef.alloc(size_t(rows) * sizeof(float4), s));
-  hipLaunchKernelGGL(bn_grad_merge_kernel, dim3(int((c + 255) / 256)), dim3(256), 0, s, sdy, sdyx, mean,
-                     invstd_or_var, gamma, int(n), int(c), int(hw), training, eps, dgamma, dbeta,
-                     dx ? coef.as<float4>() : nullptr);
+  BnArgs p = bn_args(n, c, hw, training, eps);
+  if (!dx) p.chunks = 1;  // the affine gradients alone
+  p.a = sdy;
+  p.b = sdyx;
+  p.gamma = gamma;
+  p.mean = mean;
+  p.inv_or_var = invstd_or_var;
+  p.out0 = dgamma;
+  p.out1 = dbeta;
+  if (vec)
+    hipLaunchKernelGGL(bn_grad_apply_kernel<true>, dim3(unsigned(c) * p.chunks), dim3(kThreads), 0, s, p, dy, x, dx);
+  else
+    hipLaunchKernelGGL(bn_grad_apply_kernel<false>, dim3(unsigned(c) * p.chunks), dim3(kThreads), 0, s, p, dy, x, dx);
   MX_HIP(hipGetLastError());
-  if (dx) {
-    const int64_t total = rows * hw;
-    if (vec)
-      hipLaunchKernelGGL(norm_grad_apply_kernel<true>, dim3(grid_for(total / 4)), dim3(kThreads), 0, s, dy, x,
-                         coef.as<const float4>(), total, int(hw), dx);
-    else
-      hipLaunchKernelGGL(norm_grad_apply_kernel<false>, dim3(grid_for(total)), dim3(kThreads), 0, s, dy, x,
-                         coef.as<const float4>(), total, int(hw), dx);
-    MX_HIP(hipGetLastError());
-  }
   return MX_OK;
   MX_ABI_END
 }
