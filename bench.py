@@ -1267,11 +1267,12 @@ def sq_summary(directory, xcds=8, cus=256):
     return "\n".join(out)
 
 
-WINOGRAD_KERNELS = ("filter_kernel", "wino_ws_kernel", "wino_ws16_kernel",   # fused path
+WINOGRAD_KERNELS = ("filter_kernel", "split_filter_kernel", "wino_ws_kernel", "wino_ws16_kernel",   # fused path
+                    "wino_ws_filter_kernel",
                     "wino_filter_kernel", "wino_input_kernel", "wino_output_kernel", "gemm_kernel")
 # First dispatch of a Winograd call: its filter transform, or the fused
 # kernel itself when that transforms the filter (no filter launch before it).
-WINOGRAD_CALL_START = ("filter_kernel", "wino_filter_kernel")
+WINOGRAD_CALL_START = ("filter_kernel", "split_filter_kernel", "wino_filter_kernel")
 BEFORE_HELPERS = ("conv_fwd_pack_kernel", "conv_dx_pack_kernel")       # run before their tile kernel
 AFTER_HELPERS = ("conv_dw_finalize_kernel", "conv_sum_splits_kernel")   # run after it
 
@@ -1354,7 +1355,8 @@ def trace_summary(trace_csv, bench_log):
             owner[i] = last_tile = "winograd_dweight"
         elif label in WINOGRAD_KERNELS:
             wino_calls += label in WINOGRAD_CALL_START or (
-                label in ("wino_ws_kernel", "wino_ws16_kernel") and (i == 0 or seq[i - 1][0] != "filter_kernel"))
+                label in ("wino_ws_kernel", "wino_ws16_kernel", "wino_ws_filter_kernel") and
+                (i == 0 or seq[i - 1][0] not in ("filter_kernel", "split_filter_kernel")))
             owner[i] = "winograd_dinput" if (wino_dx and wino_calls % 2 == 0) else "winograd_forward"
         elif label in AFTER_HELPERS or label == "conv_dx_zero_kernel":
             owner[i] = last_tile

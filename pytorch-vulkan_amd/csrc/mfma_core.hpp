@@ -99,6 +99,9 @@ extern "C" __device__ f32x2 mx_raw_buffer_load_v2f32(i32x4 rsrc, int voffset, in
 extern "C" __device__ void mx_raw_buffer_store_f32(float v, i32x4 rsrc, int voffset, int soffset, int aux) __asm(
     "llvm.amdgcn.raw.buffer.store.f32");
 
+extern "C" __device__ void mx_raw_buffer_store_v2f32(f32x2 v, i32x4 rsrc, int voffset, int soffset, int aux) __asm(
+    "llvm.amdgcn.raw.buffer.store.v2f32");
+
 constexpr uint32_t kOffNone = 0x80000000u;
 constexpr int64_t kBufMaxBytes = 0x7FFF0000;
 
@@ -123,6 +126,10 @@ __device__ __forceinline__ f32x2 bload2(const i32x4& r, uint32_t voff, uint32_t 
 }
 __device__ __forceinline__ void bstore(float v, const i32x4& r, uint32_t voff, uint32_t soff) {
   mx_raw_buffer_store_f32(v, r, int(voff), int(soff), 0);
+}
+
+__device__ __forceinline__ void bstore2(f32x2 v, const i32x4& r, uint32_t voff, uint32_t soff) {
+  mx_raw_buffer_store_v2f32(v, r, int(voff), int(soff), 0);
 }
 
 // n / d for n < 2^31 by multiply-high (m, l from fast_div(d) on the host):
@@ -296,6 +303,17 @@ __device__ __forceinline__ Frag3 load_frag3(const float* stage, int row0, int k0
     }
   }
   return {f[0], f[1], f[2]};
+}
+
+// The pieces of eight values already in registers.
+__device__ __forceinline__ Frag3 split8(const f32x4& a, const f32x4& b) {
+  u32x4 w[3];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const Pieces2 s = q < 2 ? split2(a[2 * q], a[2 * q + 1]) : split2(b[2 * q - 4], b[2 * q - 3]);
+    w[0][q] = s.hi, w[1][q] = s.mid, w[2][q] = s.lo;
+  }
+  return {__builtin_bit_cast(bf16x8, w[0]), __builtin_bit_cast(bf16x8, w[1]), __builtin_bit_cast(bf16x8, w[2])};
 }
 
 template <class C>

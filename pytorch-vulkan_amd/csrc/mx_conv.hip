@@ -155,6 +155,7 @@ __global__ __launch_bounds__(256) void conv_depthwise_staged_kernel(DepthwiseArg
   extern __shared__ float patch[];
   const ConvArgs& p = a.p;
   const int KH = K ? K : p.KH, KW = K ? K : p.KW, m = p.Cout_g;
+  constexpr int U = K ? K : 1;
   for (int64_t t = blockIdx.x; t < a.tiles; t += gridDim.x) {
     const int tw = int(t % a.tiles_w), th = int((t / a.tiles_w) % a.tiles_h);
     const int plane0 = int(t / (int64_t(a.tiles_w) * a.tiles_h)) * a.planes;
@@ -178,9 +179,9 @@ __global__ __launch_bounds__(256) void conv_depthwise_staged_kernel(DepthwiseArg
         const float b = p.bias ? p.bias[oc] : 0.f;
 #pragma unroll
         for (int r = 0; r < kDwRows; ++r) acc[r] = b;
-#pragma unroll(K ? K : 1)
+#pragma unroll U
         for (int kh = 0; kh < KH; ++kh)
-#pragma unroll(K ? K : 1)
+#pragma unroll U
           for (int kw = 0; kw < KW; ++kw) {
             const float wv = wk[kh * KW + kw];
 #pragma unroll
@@ -205,6 +206,7 @@ __global__ __launch_bounds__(256) void conv_depthwise_dx_kernel(DepthwiseArgs a)
   extern __shared__ float patch[];
   const ConvArgs& p = a.p;
   const int KH = K ? K : p.KH, KW = K ? K : p.KW, m = p.Cout_g;
+  constexpr int U = K ? K : 1;
   for (int64_t t = blockIdx.x; t < a.tiles; t += gridDim.x) {
     const int tw = int(t % a.tiles_w), th = int((t / a.tiles_w) % a.tiles_h);
     const int plane0 = int(t / (int64_t(a.tiles_w) * a.tiles_h)) * a.planes;
@@ -230,9 +232,9 @@ __global__ __launch_bounds__(256) void conv_depthwise_dx_kernel(DepthwiseArgs a)
       for (int j = 0; j < m; ++j) {
         const float* const wk = p.w + (int64_t(ic) * m + j) * (KH * KW);
         const float* const src = patch + (pl * m + j) * a.patch;
-#pragma unroll(K ? K : 1)
+#pragma unroll U
         for (int kh = 0; kh < KH; ++kh)
-#pragma unroll(K ? K : 1)
+#pragma unroll U
           for (int kw = 0; kw < KW; ++kw) {
             const float wv = wk[kh * KW + kw];
             const int tx = x0 - kw * p.dw;

@@ -17,16 +17,15 @@
 // on 4x4 input tiles at stride 2, M_t = U_t V_t for each of the 16 transform
 // coordinates t.
 //
-// Fused kernel (the default): one workgroup computes 64 output channels x 32
-// tiles for all 16 coordinates.  Per slab of 8 input channels it stages the
-// transformed filter U (precomputed once per call by the filter launch,
-// [G][16][Cpad][Opad], output channels contiguous, zero padded, or for
-// short channel walks transformed from w in the kernel) and transforms the
-// 4x4 input patches it loads straight into LDS, so V never goes to HBM; the
-// 16 products run as
-// v_mfma_f32_16x16x4f32 with each wave holding all 16 coordinates of a 32
-// channel x 16 tile block, so the output transform A^T M A and the bias are
-// applied in registers and M never goes to HBM either.
+// Fused kernels (the default): one workgroup computes 64 output channels x a
+// block of tiles for all 16 coordinates.  Per slab of input channels it takes
+// the transformed filter U (precomputed once per call by the filter launch,
+// zero padded, or for short channel walks transformed from w in the kernel)
+// and transforms the 4x4 input patches it loads straight into LDS, so V never
+// goes to HBM; the output transform A^T M A and the bias are applied before
+// the stores, so M never goes to HBM either.  Grids that fill the CUs run
+// 64-tile blocks with the products as six bf16 MFMAs over three-piece
+// operands; smaller ones run 16- or 32-tile blocks on v_mfma_f32_16x16x4f32.
 //
 // Unfused kernels (launches with few tiles, or MX_WINOGRAD_FUSED=0): the
 // filter, input and output
@@ -190,6 +189,7 @@ struct Args {
   float* y;          // [N][Cout][OH][OW]
   int64_t x_bytes, u_bytes, y_bytes, w_bytes;
   int Cin, H, W, Cout, OH, OW, ph, pw, C, O, Cpad, Opad, TH, TW, T, n_ob, nslab;
+  int flip, y_even;  // split kernel: w read flipped and channel-swapped; y is 8-byte aligned
   mfma::FastDiv f_thw, f_tw;
 };
 
@@ -623,8 +623,9 @@ __device__ __forceinline__ void ws_body(const fused::Args& p, int b, int g, floa
     }
 }
 
+// The 32-tile kernel on its own launch, for walks of at most 4 slabs.
 template <bool RAGGED, int FILT>
-__global__ __launch_bounds__(512) void wino_ws_kernel(fused::Args p) {
+__global__ __launch_bounds__(512) void wino_ws_filter_kernel(fused::Args p) {
   __shared__ __attribute__((aligned(16))) float As0[A_FLOATS];
   __shared__ __attribute__((aligned(16))) float Bs0[B_FLOATS];
   __shared__ __attribute__((aligned(16))) float As1[A_FLOATS];
@@ -894,6 +895,324 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     mfma::bstore(r0[1] - r0[2] - r0[3] + bb, ry, (ok && right) ? off + 4u : kOffNone, 0);
     mfma::bstore(r1[0] + r1[1] + r1[2] + bb, ry, (ok && below) ? off + row_step : kOffNone, 0);
     mfma::bstore(r1[1] - r1[2] - r1[3] + bb, ry, (ok && below && right) ? off + row_step + 4u : kOffNone, 0);
+  }
+}
+
+// ------------------------------------------------------------ split fused kernel
+// 64 output channels x 64 tiles per workgroup of eight waves, each wave two of
+// the 16 coordinates (128 accumulators a lane), the products as six bf16 MFMAs
+// over three-piece operands (mfma_core.hpp).  Per slab of 16 channels:
+//   - U' comes split from the filter launch and goes from L2 straight into the
+//     fragments of the one wave that needs it (98 KB a slab, no LDS);
+//   - V = B^T d B goes through LDS in FP32 (64 KB, two stages) and is split
+//     after the read: one wave reads each value, so that costs no more than
+//     splitting before, and LDS carries a third less;
+//   - every wave both produces (two patches a thread, their loads half a slab
+//     ahead) and multiplies, the patch work between its two coordinates.
+// The output transform needs all coordinates of an output, which eight waves
+// hold: they meet in LDS, 32 channels at a time.  Against the 16-tile kernel
+// on FP32 MFMA, this shape reads U' from L2 a quarter as often per tile and
+// spends 6 x 32 matrix cycles where that one spends 16 x 32.  16 x 512 x 32^2
+// -> 256: 114 us (6 x 17 GF on bf16 MFMA at 0.9 PF/s; 166 us on FP32 MFMA);
+// without its loads the loop takes two thirds of the time and without its
+// products nearly as much, so what bounds it is how far the two overlap at
+// two waves a SIMD.
+constexpr int SO = 64, STILES = 64, SK = 16;
+constexpr int V_FLOATS = 16 * SK * STILES;  // [coordinate][k][tile], one stage
+
+// The bf16 matrix instruction rounds its sums down (the FP32 one to nearest),
+// which over a chain of slabs pulls every accumulator the same way.  Slabs
+// from this one on are summed negated (U' carries the sign, the accumulators
+// change theirs once here and once at the end), so the two parts' biases
+// cancel: the bias of a step goes as the sum's last place, with the square
+// root of the slabs so far, and sum_{s < m} sqrt(s) is half of the whole at
+// m = 0.63 ns.  512 -> 256 channels: mean error -1.4e-8 -> -4e-10 of the
+// outputs' norm, error 5.9e-7 (FP32 MFMA 7.0e-7); it costs 1% of the time.
+__host__ __device__ inline int negated_from(int ns) { return (5 * ns + 2) / 8; }
+
+template <bool RAGGED>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void wino_ws_kernel(fused::Args p) {
+  __shared__ __attribute__((aligned(16))) float smem[2 * V_FLOATS];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = blockIdx.y;
+  const int b = mfma::xcd_remap(blockIdx.x, gridDim.x);
+  const int ob = b % p.n_ob, tb = b / p.n_ob;
+  const int o0 = ob * SO, t0 = tb * STILES;
+  const int ns = p.nslab / 2;  // slabs of 16 channels
+
+  // ---- patches: lane = tile, wave = channel kc and kc + 8 of the slab, so a
+  // row load covers one channel's consecutive tiles (lanes along the channels
+  // would touch a line each: 76 -> 66 us at 16 x 256 x 32 x 32).
+  const int kc = wave;
+  const i32x4 rx = mfma::buffer_rsrc(p.x, p.x_bytes);
+  PatchRows px;
+  {
+    const int t = t0 + lane;
+    const bool tok = t < p.T;
+    const uint32_t tt = tok ? uint32_t(t) : 0u;
+    const uint32_t img = mfma::fdiv(tt, p.f_thw);
+    const uint32_t pos = tt - img * uint32_t(p.TH * p.TW);
+    const uint32_t ty = mfma::fdiv(pos, p.f_tw), tx = pos - ty * uint32_t(p.TW);
+    px.init((int64_t(img) * p.Cin + int64_t(g) * p.C + kc) * p.H, int(2 * ty) - p.ph, int(2 * tx) - p.pw, tok, p.H,
+            p.W);
+  }
+  const uint32_t x_half = uint32_t(8) * p.H * p.W * 4;  // 8 channels
+  // Half h of slab s (channels s * 16 + h * 8 + kc); past the last slab, the
+  // last one again.
+  auto load_patch = [&](int s, int h) {
+    const int c8 = 2 * min(s, ns - 1) + h;
+    px.load(rx, uint32_t(c8) * x_half, uint32_t(p.x_bytes), !RAGGED || c8 * 8 + kc < p.C);
+  };
+  auto store_patch = [&](float* V, int h) {
+    px.fix(rx);
+    float d[16], z[16];
+    px.patch(d);
+#pragma unroll
+    for (int cc = 0; cc < 4; ++cc) {
+      z[0 * 4 + cc] = d[0 * 4 + cc] - d[2 * 4 + cc];
+      z[1 * 4 + cc] = d[1 * 4 + cc] + d[2 * 4 + cc];
+      z[2 * 4 + cc] = d[2 * 4 + cc] - d[1 * 4 + cc];
+      z[3 * 4 + cc] = d[1 * 4 + cc] - d[3 * 4 + cc];
+    }
+    float* const dst = V + (8 * h + kc) * STILES + lane;
+    constexpr int T = SK * STILES;  // one coordinate
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      dst[(i * 4 + 0) * T] = z[i * 4 + 0] - z[i * 4 + 2];
+      dst[(i * 4 + 1) * T] = z[i * 4 + 1] + z[i * 4 + 2];
+      dst[(i * 4 + 2) * T] = z[i * 4 + 2] - z[i * 4 + 1];
+      dst[(i * 4 + 3) * T] = z[i * 4 + 1] - z[i * 4 + 3];
+    }
+  };
+
+  // ---- products: coordinates 2 wave and 2 wave + 1.
+  const int r = lane & 31, h = lane >> 5;
+  const i32x4 ru = mfma::buffer_rsrc(p.U, p.u_bytes);
+  const uint32_t u_lane = uint32_t((h * p.Opad + o0 + r) * 16);
+  const uint32_t u_plane = uint32_t(32) * p.Opad, u_slab = 3 * u_plane;
+  const uint32_t u_coord = uint32_t(ns) * u_slab;
+  const uint32_t u_first = uint32_t(g * 16 + 2 * wave) * u_coord;
+  mfma::Frag3 a[2][2];  // [coordinate][32-channel block]
+  auto load_u = [&](int e, int s) {
+    const uint32_t at = u_first + uint32_t(e) * u_coord + uint32_t(min(s, ns - 1)) * u_slab;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      a[e][i].hi = __builtin_bit_cast(mfma::bf16x8, mfma::bload4(ru, u_lane + i * 512, at));
+      a[e][i].mid = __builtin_bit_cast(mfma::bf16x8, mfma::bload4(ru, u_lane + i * 512, at + u_plane));
+      a[e][i].lo = __builtin_bit_cast(mfma::bf16x8, mfma::bload4(ru, u_lane + i * 512, at + 2 * u_plane));
+    }
+  };
+  typedef float f32x16 __attribute__((ext_vector_type(16)));
+  f32x16 acc[2][2][2];  // [coordinate][channel block][tile block]
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[e][i][j][v] = 0.f;
+  auto multiply = [&](const float* V, int e) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const float* const src = V + ((2 * wave + e) * SK + 8 * h) * STILES + j * 32 + r;
+      f32x4 k0, k4;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) k0[k] = src[k * STILES], k4[k] = src[(4 + k) * STILES];
+      const mfma::Frag3 f = mfma::split8(k0, k4);
+#define MX_WINO_PRODUCT(P, Q)                                                                                      \
+  _Pragma("unroll") for (int i = 0; i < 2; ++i) acc[e][i][j] =                                                     \
+      __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[e][i].P, f.Q, acc[e][i][j], 0, 0, 0);
+      MX_WINO_PRODUCT(lo, hi)
+      MX_WINO_PRODUCT(hi, lo)
+      MX_WINO_PRODUCT(mid, mid)
+      MX_WINO_PRODUCT(mid, hi)
+      MX_WINO_PRODUCT(hi, mid)
+      MX_WINO_PRODUCT(hi, hi)
+#undef MX_WINO_PRODUCT
+    }
+  };
+
+  auto negate = [&]() {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[e][i][j][v] = -acc[e][i][j][v];
+  };
+  const int turn = negated_from(ns);
+
+  load_patch(0, 0);
+  load_u(0, 0);
+  load_u(1, 0);
+  store_patch(smem, 0);
+  load_patch(0, 1);
+  store_patch(smem, 1);
+  load_patch(1, 0);
+  __syncthreads();
+  // Slab s is read from stage s & 1 while slab s + 1 goes into the other (past
+  // the last slab the last one again, which nobody reads).
+  for (int s = 0; s < ns; ++s) {
+    const float* const cur = smem + (s & 1) * V_FLOATS;
+    float* const next = smem + ((s & 1) ^ 1) * V_FLOATS;
+    if (s == turn) negate();
+    multiply(cur, 0);
+    load_u(0, s + 1);
+    store_patch(next, 0);
+    load_patch(s + 1, 1);
+    multiply(cur, 1);
+    load_u(1, s + 1);
+    store_patch(next, 1);
+    load_patch(s + 2, 0);
+    __syncthreads();
+  }
+
+  negate();
+
+  // Products that the pieces cannot carry (not finite, or nonzero below
+  // 2^-80: see acc_out_of_range) send the whole workgroup to the direct sum.
+  {
+    uint32_t top = 0, low = ~0u;
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) {
+            const uint32_t mag = __float_as_uint(acc[e][i][j][v]) << 1;
+            top = max(top, mag);
+            low = min(low, mag - 1);
+          }
+    const bool bad = top >= 0xFF000000u || low < (uint32_t(127 - 80) << 24) - 1;
+    int* const flags = reinterpret_cast<int*>(smem);
+    const bool any = __any(bad);
+    if (lane == 0) flags[wave] = any;
+    __syncthreads();
+    int all = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) all |= flags[i];
+    __syncthreads();
+    if (all) {
+      const int t = t0 + (tid & 63);
+      if (t >= p.T) return;
+      const uint32_t img = mfma::fdiv(uint32_t(t), p.f_thw);
+      const uint32_t pos = uint32_t(t) - img * uint32_t(p.TH * p.TW);
+      const uint32_t ty = mfma::fdiv(pos, p.f_tw), tx = pos - ty * uint32_t(p.TW);
+      for (int o = o0 + (tid >> 6); o < min(o0 + SO, p.O); o += 8)
+        for (int q = 0; q < 4; ++q) {
+          const int oy = int(2 * ty) + (q >> 1), ox = int(2 * tx) + (q & 1);
+          if (oy >= p.OH || ox >= p.OW) continue;
+          float sum = 0.f;
+          for (int c = 0; c < p.C; ++c) {
+            const float* const xp = p.x + (int64_t(img) * p.Cin + int64_t(g) * p.C + c) * p.H * p.W;
+            const float* const wk = p.flip ? p.w + ((int64_t(g) * p.C + c) * p.O + o) * 9
+                                           : p.w + ((int64_t(g) * p.O + o) * p.C + c) * 9;
+            for (int k = 0; k < 9; ++k) {
+              const int iy = oy - p.ph + k / 3, ix = ox - p.pw + k % 3;
+              if (unsigned(iy) < unsigned(p.H) && unsigned(ix) < unsigned(p.W))
+                sum += xp[iy * p.W + ix] * wk[p.flip ? 8 - k : k];
+            }
+          }
+          p.y[((int64_t(img) * p.Cout + int64_t(g) * p.O + o) * p.OH + oy) * p.OW + ox] =
+              sum + (p.bias ? p.bias[g * p.O + o] : 0.f);
+        }
+      return;
+    }
+  }
+
+  // Output transform, 32 channels at a time: [coordinate][channel][tile] in
+  // LDS, then each thread takes one tile of four channels.
+  const int t = t0 + lane;
+  const bool tok = t < p.T;
+  const uint32_t tt = tok ? uint32_t(t) : 0u;
+  const uint32_t img = mfma::fdiv(tt, p.f_thw);
+  const uint32_t pos = tt - img * uint32_t(p.TH * p.TW);
+  const uint32_t ty = mfma::fdiv(pos, p.f_tw), tx = pos - ty * uint32_t(p.TW);
+  const int oy = int(2 * ty), ox = int(2 * tx);
+  const bool right = ox + 1 < p.OW, below = oy + 1 < p.OH;
+  const i32x4 ry = mfma::buffer_rsrc(p.y, p.y_bytes);
+  const uint32_t plane4 = uint32_t(p.OH) * uint32_t(p.OW) * 4u, row4 = uint32_t(p.OW) * 4u;
+  const uint32_t y_tile = ((img * uint32_t(p.Cout) + uint32_t(g * p.O)) * uint32_t(p.OH) + uint32_t(oy)) * row4 +
+                          uint32_t(ox) * 4u;
+  const bool pairs = p.OW % 2 == 0 && p.y_even;  // both outputs of a row exist and share an 8-byte slot
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          smem[((2 * wave + e) * 32 + 8 * (v >> 2) + 4 * h + (v & 3)) * STILES + j * 32 + r] = acc[e][i][j][v];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int ol = wave + 8 * q, o = o0 + i * 32 + ol;
+      float m[16];
+#pragma unroll
+      for (int c = 0; c < 16; ++c) m[c] = smem[(c * 32 + ol) * STILES + lane];
+      float r0[4], r1[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        r0[c] = m[c] + m[4 + c] + m[8 + c];
+        r1[c] = m[4 + c] - m[8 + c] - m[12 + c];
+      }
+      const bool ok = o < p.O && tok;
+      const float bb = (p.bias && o < p.O) ? p.bias[g * p.O + o] : 0.f;
+      const uint32_t off = y_tile + uint32_t(o) * plane4;
+      const float y00 = r0[0] + r0[1] + r0[2] + bb, y01 = r0[1] - r0[2] - r0[3] + bb;
+      const float y10 = r1[0] + r1[1] + r1[2] + bb, y11 = r1[1] - r1[2] - r1[3] + bb;
+      if (pairs) {
+        mfma::bstore2(f32x2{y00, y01}, ry, ok ? off : kOffNone, 0);
+        mfma::bstore2(f32x2{y10, y11}, ry, (ok && below) ? off + row4 : kOffNone, 0);
+      } else {
+        mfma::bstore(y00, ry, ok ? off : kOffNone, 0);
+        mfma::bstore(y01, ry, (ok && right) ? off + 4u : kOffNone, 0);
+        mfma::bstore(y10, ry, (ok && below) ? off + row4 : kOffNone, 0);
+        mfma::bstore(y11, ry, (ok && below && right) ? off + row4 + 4u : kOffNone, 0);
+      }
+    }
+    if (i == 0) __syncthreads();
+  }
+}
+
+// U' of the split kernel: the pieces of channels c .. c + 7 of coordinate t,
+// output channel o, at [g][t][c / 16][piece][(c / 8) % 2][o][8] (16 bytes).
+// A workgroup transforms 32 output channels x 8 input channels, a filter per
+// thread, and assembles the 16-byte groups in LDS.
+__global__ __launch_bounds__(256) void split_filter_kernel(const float* __restrict__ w, uint16_t* __restrict__ U, int C,
+                                                           int O, int Cpad, int Opad, bool flip) {
+  __shared__ __attribute__((aligned(16))) uint16_t buf[16 * 3 * 32 * 8];
+  const int tid = threadIdx.x, g = blockIdx.z;
+  const int ob = blockIdx.x * 32, cg = blockIdx.y;
+  // Lanes along the layer filter's inner axis.
+  const int ol = flip ? tid & 31 : tid >> 3, cl = flip ? tid >> 5 : tid & 7;
+  float u[16];
+  fused::filter_transform(w, C, O, g, ob + ol, cg * 8 + cl, flip, u);
+  const int ns = Cpad / SK, slab = cg >> 1, half = cg & 1;
+  const float sign = slab >= negated_from(ns) ? -1.f : 1.f;
+#pragma unroll
+  for (int t = 0; t < 16; t += 2) {
+    const mfma::Pieces2 s = mfma::split2(sign * u[t], sign * u[t + 1]);
+    const uint32_t piece[3] = {s.hi, s.mid, s.lo};
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      buf[((t * 3 + q) * 32 + ol) * 8 + cl] = uint16_t(piece[q]);
+      buf[(((t + 1) * 3 + q) * 32 + ol) * 8 + cl] = uint16_t(piece[q] >> 16);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    const int e = tid + 256 * k, o = e & 31, q = (e >> 5) % 3, t = e / 96;
+    const int64_t at = ((((int64_t(g) * 16 + t) * ns + slab) * 3 + q) * 2 + half) * Opad + ob + o;
+    reinterpret_cast<mfma::u32x4*>(U)[at] = reinterpret_cast<const mfma::u32x4*>(buf)[e];
   }
 }
 }  // namespace ws
@@ -1548,7 +1867,32 @@ struct RunPlan {
   int64_t unfused_bytes = 0;  // U, V and M of one pass
 };
 
-int plan_run(const mx_conv2d_desc& d, int64_t ws_limit, RunPlan* r) {
+// Workgroups per group and transformed-filter bytes of the split kernel.
+int64_t split_blocks(const RunPlan& r) { return (int64_t(r.p.T) + ws::STILES - 1) / ws::STILES * r.p.n_ob; }
+int64_t split_filter_bytes(const RunPlan& r) { return int64_t(r.G) * 16 * r.p.Cpad * r.p.Opad * 6; }
+
+// The cheaper of the 16-tile and the split kernel, in us on MI355X: rounds of
+// workgroups over the CUs times a fixed part and a part per slab.  The split
+// kernel holds one workgroup per CU (10 + 2.9 per slab of 16); the 16-tile
+// kernel two (3 + 1.25 per slab of 8), a last round of at most one per CU
+// taking three quarters.  Measured, split / 16-tile: 128 channels 64 x 28^2
+// 67 / 79, 16 x 64^2 70 / 91; 256 channels 64 x 14^2 61 / 87, 16 x 32^2
+// 65 / 90; 512 -> 256 16 x 32^2 114 / 166; 64 channels 64 x 56^2 85 / 88,
+// 8 x 56^2 23 / 18; 96 -> 160 8 x 40^2 30 / 33 and its input gradient 40 / 32;
+// 256 channels 2 x 48^2 59 / 49; 512 channels 64 x 7^2 105 / 93.
+bool prefer_t16(const RunPlan& r, bool dinput) {
+  if (r.filt) return int64_t(r.p.Cpad) * r.p.Opad <= 256 * 256;
+  // The one-launch backward computes the 16-tile kernel's bits.
+  if (dinput && r.p.nslab <= 8 && r.blocks * r.G <= cu_count()) return true;
+  const int64_t cus = cu_count();
+  const int64_t split_rounds = (split_blocks(r) * r.G + cus - 1) / cus;
+  const int64_t b16 = (int64_t(r.p.T) + ws::BT16 - 1) / ws::BT16 * r.p.n_ob * r.G;
+  const int64_t tail = b16 % (2 * cus);
+  const double t16_rounds = double(b16 / (2 * cus)) + (tail == 0 ? 0.0 : tail <= cus ? 0.75 : 1.0);
+  return t16_rounds * (3.0 + 1.25 * r.p.nslab) <= double(split_rounds) * (10.0 + 2.9 * (r.p.nslab / 2));
+}
+
+int plan_run(const mx_conv2d_desc& d, int64_t ws_limit, bool dinput, RunPlan* r) {
   fused::Args& p = r->p;
   p.Cin = int(d.cin);
   p.H = int(d.h);
@@ -1609,15 +1953,12 @@ int plan_run(const mx_conv2d_desc& d, int64_t ws_limit, RunPlan* r) {
   if (const char* e = std::getenv("MX_WINOGRAD_FILTER"))
     if (e[0] == '0' || e[0] == '1') r->filt = e[0] == '1';
   r->filt = r->filt && r->fused;
-  // The 16-tile kernel (two workgroups per CU, one's prologue and epilogue
-  // under the other's products) wins while the transformed filter is small
-  // enough to stay in L2 for the twice as many workgroups that read it: 64 x
-  // 64 channels at 56^2, batch 64, 96.3 -> 84.4 us, 128 x 128 at 28^2 93.9 ->
-  // 79.5, 256 x 256 at 16^2, batch 16, 49.0 -> 34.7; at 512 x 512 (a 16.8 MB
-  // U') it loses (91.2 -> 94.9).  MX_WINOGRAD_T16=0 / 1 forces it off / on.
-  r->t16 = int64_t(p.Cpad) * p.Opad <= 256 * 256;
+  r->t16 = prefer_t16(*r, dinput);
   if (const char* e = std::getenv("MX_WINOGRAD_T16"))
     if (e[0] == '0' || e[0] == '1') r->t16 = e[0] == '1';
+  // The split filter takes half as much again; past the buffer bound the
+  // 16-tile kernel runs.
+  if (!r->filt && split_filter_bytes(*r) >= mfma::kBufMaxBytes) r->t16 = true;
   r->t16 = r->t16 && r->fused;
   if (r->filt) {
     p.w_bytes = int64_t(d.cout) * p.C * 9 * 4;
@@ -1631,7 +1972,7 @@ int plan_run(const mx_conv2d_desc& d, int64_t ws_limit, RunPlan* r) {
 int winograd_run(const mx_conv2d_desc& d, const float* x, const float* w, const float* bias, float* y, bool flip,
                  int64_t ws_limit, hipStream_t s) {
   RunPlan r;
-  MX_TRY(plan_run(d, ws_limit, &r));
+  MX_TRY(plan_run(d, ws_limit, flip, &r));
   fused::Args& p = r.p;
   if (p.T == 0) return MX_OK;
   if (!r.fused) return winograd_unfused(d, x, w, bias, y, flip, r.chunk, s);
@@ -1651,13 +1992,31 @@ int winograd_run(const mx_conv2d_desc& d, const float* x, const float* w, const 
   }
   if (r.filt) {
     p.w = w;
-    void (*kern)(fused::Args) = flip ? (ragged ? ws::wino_ws_kernel<true, 2> : ws::wino_ws_kernel<false, 2>)
-                                     : (ragged ? ws::wino_ws_kernel<true, 1> : ws::wino_ws_kernel<false, 1>);
+    void (*kern)(fused::Args) =
+        flip ? (ragged ? ws::wino_ws_filter_kernel<true, 2> : ws::wino_ws_filter_kernel<false, 2>)
+             : (ragged ? ws::wino_ws_filter_kernel<true, 1> : ws::wino_ws_filter_kernel<false, 1>);
     hipLaunchKernelGGL(kern, grid, dim3(512), 0, s, p);
     MX_HIP(hipGetLastError());
     return MX_OK;
   }
   Scratch U;
+  if (!r.t16) {
+    p.u_bytes = split_filter_bytes(r);
+    MX_TRY(U.alloc(size_t(p.u_bytes), s));
+    p.U = U.as<float>();
+    p.w = w;
+    p.flip = flip ? 1 : 0;
+    p.y_even = (reinterpret_cast<uintptr_t>(y) & 7) == 0;
+    const dim3 fgrid(unsigned(p.Opad / 32), unsigned(p.Cpad / 8), unsigned(r.G));
+    hipLaunchKernelGGL(ws::split_filter_kernel, fgrid, dim3(256), 0, s, w, U.as<uint16_t>(), p.C, p.O, p.Cpad, p.Opad,
+                       flip);
+    MX_HIP(hipGetLastError());
+    const dim3 sgrid(unsigned(split_blocks(r)), unsigned(r.G));
+    void (*kern)(fused::Args) = ragged ? ws::wino_ws_kernel<true> : ws::wino_ws_kernel<false>;
+    hipLaunchKernelGGL(kern, sgrid, dim3(512), 0, s, p);
+    MX_HIP(hipGetLastError());
+    return MX_OK;
+  }
   MX_TRY(U.alloc(size_t(p.u_bytes), s));
   p.U = U.as<float>();
   // 64-thread blocks: a small filter (64 x 64 is 2,048 threads) then spreads
@@ -1666,15 +2025,9 @@ int winograd_run(const mx_conv2d_desc& d, const float* x, const float* w, const 
   hipLaunchKernelGGL(fused::filter_kernel, dim3(unsigned(std::min<int64_t>((filter_threads + 63) / 64, 1 << 20))),
                      dim3(64), 0, s, w, U.as<float>(), p.C, p.O, p.Cpad, p.Opad, r.G, flip);
   MX_HIP(hipGetLastError());
-  if (r.t16) {
-    const dim3 grid16{unsigned((int64_t(p.T) + ws::BT16 - 1) / ws::BT16 * p.n_ob), unsigned(r.G), 1u};
-    void (*k16)(fused::Args) = ragged ? ws::wino_ws16_kernel<true, 0> : ws::wino_ws16_kernel<false, 0>;
-    hipLaunchKernelGGL(k16, grid16, dim3(512), 0, s, p);
-    MX_HIP(hipGetLastError());
-    return MX_OK;
-  }
-  void (*kern)(fused::Args) = ragged ? ws::wino_ws_kernel<true, 0> : ws::wino_ws_kernel<false, 0>;
-  hipLaunchKernelGGL(kern, grid, dim3(512), 0, s, p);
+  const dim3 grid16{unsigned((int64_t(p.T) + ws::BT16 - 1) / ws::BT16 * p.n_ob), unsigned(r.G), 1u};
+  void (*k16)(fused::Args) = ragged ? ws::wino_ws16_kernel<true, 0> : ws::wino_ws16_kernel<false, 0>;
+  hipLaunchKernelGGL(k16, grid16, dim3(512), 0, s, p);
   MX_HIP(hipGetLastError());
   return MX_OK;
 }
@@ -1823,7 +2176,7 @@ int winograd_describe(const mx_conv2d_desc& d, int phase, bool with_bias, int64_
     return MX_OK;
   }
   RunPlan r;
-  MX_TRY(plan_run(phase == MX_CONV_DINPUT ? dinput_as_forward(d) : d, ws_limit, &r));
+  MX_TRY(plan_run(phase == MX_CONV_DINPUT ? dinput_as_forward(d) : d, ws_limit, phase == MX_CONV_DINPUT, &r));
   if (r.fused) {
     *variant = cat(r.t16 ? "wino_ws16_kernel<" : "wino_ws_kernel<", r.p.C % (2 * fused::BK) ? "ragged" : "even",
                    r.filt ? ",filter>" : ">");
@@ -1863,7 +2216,7 @@ static int winograd_backward_plan(const mx_conv2d_desc& d, int64_t ws_limit, boo
                                   DwRunPlan* rw, bool* one) {
   *one = false;
   if (d.ph > 2 || d.pw > 2) return MX_OK;
-  MX_TRY(plan_run(dinput_as_forward(d), ws_limit, rf));
+  MX_TRY(plan_run(dinput_as_forward(d), ws_limit, true, rf));
   MX_TRY(plan_dw_run(d, ws_limit, with_db, rw));
   if (!rf->fused || !rw->ws || rf->p.T == 0 || rw->p.T == 0) return MX_OK;
   const int64_t cus = cu_count(), n_dx32 = rf->blocks * rf->G, n_dw_all = rw->blocks * rw->ranges;

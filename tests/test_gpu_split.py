@@ -183,3 +183,93 @@ def test_gemm_under_capture_takes_no_scratch(mx):
         torch.cuda.synchronize()
         assert ((c - eager).norm() / eager.norm()).item() < 2e-6
     assert before is None or mx.memory_stats().device_mallocs == before
+
+
+def winograd_magnitude(x, w, pad, oh, ow):
+    """|A^T| (|G| |g| |G^T| * |B^T| |d| |B|) |A|: what the roundings of an
+    F(2x2, 3x3) output are relative to."""
+    bt = torch.tensor([[1, 0, -1, 0], [0, 1, 1, 0], [0, -1, 1, 0], [0, 1, 0, -1]], dtype=torch.float64).abs()
+    gm = torch.tensor([[1, 0, 0], [.5, .5, .5], [.5, -.5, .5], [0, 0, 1]], dtype=torch.float64).abs()
+    at = torch.tensor([[1, 1, 1, 0], [0, 1, -1, -1]], dtype=torch.float64).abs()
+    th, tw = (oh + 1) // 2, (ow + 1) // 2
+    xp = F.pad(x.double().abs(), (pad[1], 2 * tw + 2 - x.shape[3] - pad[1], pad[0], 2 * th + 2 - x.shape[2] - pad[0]))
+    d = xp.unfold(2, 4, 2).unfold(3, 4, 2)[:, :, :th, :tw]
+    v, u = bt @ d @ bt.t(), gm @ w.double().abs() @ gm.t()
+    m = torch.einsum("ncyxab,ocab->noyxab", v, u)
+    return (at @ m @ at.t()).permute(0, 1, 2, 4, 3, 5).reshape(x.shape[0], w.shape[0], 2 * th, 2 * tw)[:, :, :oh, :ow]
+
+
+@pytest.mark.parametrize("n,c,h,wd,o,pad,groups", [
+    (1, 16, 16, 16, 64, (1, 1), 1),    # exactly one block: 64 tiles x 64 channels, one slab
+    (1, 17, 16, 18, 65, (1, 1), 1),    # one past each of them
+    (3, 31, 9, 7, 40, (0, 2), 1),      # odd outputs, padding apart, tiles across images
+    (2, 32, 5, 66, 64, (2, 0), 1),
+    (1, 80, 34, 31, 129, (1, 1), 1),   # odd row width: single stores
+    (2, 24, 12, 12, 70, (1, 1), 3),    # groups
+    (1, 1, 2, 2, 1, (2, 2), 1),
+])
+@pytest.mark.parametrize("flip", [False, True])
+def test_winograd_split_kernel(mx, monkeypatch, n, c, h, wd, o, pad, groups, flip):
+    """The 64 x 64 Winograd kernel at the edges of its blocks, slabs and
+    stores: seven additions' and a slab chain's roundings of the transforms'
+    magnitudes, (C / 16 + 16) 2^-23."""
+    for k, val in (("FUSED", "1"), ("T16", "0"), ("FILTER", "0")):
+        monkeypatch.setenv(f"MX_WINOGRAD_{k}", val)
+    g = torch.Generator().manual_seed(n + c + h + o)
+    d = mx.conv_desc((n, c * groups, h, wd), (o * groups, c, 3, 3), (1, 1), pad, (1, 1), groups)
+    x, w = torch.randn(n, c * groups, h, wd, generator=g), torch.randn(o * groups, c, 3, 3, generator=g)
+    bias = torch.randn(o * groups, generator=g)
+    st = torch.cuda.current_stream().cuda_stream
+    if flip:
+        x = torch.randn(n, o * groups, d.oh, d.ow, generator=g)  # dy
+        out = torch.full((n, c * groups, h, wd), float("nan"), device="cuda")
+        wt = w.reshape(groups, o, c, 3, 3).flip(3, 4).transpose(1, 2).reshape(groups * c, o, 3, 3)
+        pad_t, bias = (2 - pad[0], 2 - pad[1]), None
+        xd, wdv = x.cuda(), w.cuda()
+        torch.cuda.synchronize()
+        mx.conv2d_backward_input(d, xd, wdv, out, 3, st)
+    else:
+        out = torch.full((n, o * groups, d.oh, d.ow), float("nan"), device="cuda")
+        wt, pad_t = w, pad
+        xd, wdv, bd = x.cuda(), w.cuda(), bias.cuda()
+        torch.cuda.synchronize()
+        mx.conv2d_forward(d, xd, wdv, bd, out, 3, st)
+    torch.cuda.synchronize()
+    got = out.cpu().double()
+    ref = F.conv2d(x.double(), wt.double(), None if bias is None else bias.double(), padding=pad_t, groups=groups)
+    mag = torch.cat([winograd_magnitude(xs, ws, pad_t, *ref.shape[2:])
+                     for xs, ws in zip(x.chunk(groups, 1), wt.chunk(groups, 0))], 1)
+    if bias is not None:
+        mag = mag + bias.double().abs().view(1, -1, 1, 1)
+    assert got.shape == ref.shape
+    assert ((got - ref).abs() <= (wt.shape[1] / 16 + 16) * 2.0 ** -23 * mag).all()
+
+
+def test_winograd_split_kernel_infinite_and_tiny(mx, monkeypatch):
+    """Products without pieces take the direct sum: infinities and NaN where
+    the definition has them and nowhere else in the block, and inputs whose
+    products are denormal keep their digits (9 C roundings of the sum)."""
+    for k, val in (("FUSED", "1"), ("T16", "0"), ("FILTER", "0")):
+        monkeypatch.setenv(f"MX_WINOGRAD_{k}", val)
+    g = torch.Generator().manual_seed(5)
+    d = mx.conv_desc((2, 20, 16, 16), (70, 20, 3, 3), (1, 1), (1, 1))
+    w = torch.randn(70, 20, 3, 3, generator=g)
+    st = torch.cuda.current_stream().cuda_stream
+
+    def run(x):
+        xd, wd = x.cuda(), w.cuda()
+        y = torch.empty(2, 70, 16, 16, device="cuda")
+        torch.cuda.synchronize()
+        mx.conv2d_forward(d, xd, wd, None, y, 3, st)
+        torch.cuda.synchronize()
+        return y.cpu()
+
+    x = torch.randn(2, 20, 16, 16, generator=g)
+    x[0, 3, 5, 6], x[1, 7, 0, 0] = float("inf"), float("nan")
+    got, ref = run(x), F.conv2d(x, w, padding=1)
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isposinf(), ref.isposinf())
+    assert torch.equal(got.isneginf(), ref.isneginf())
+    tiny = torch.randn(2, 20, 16, 16, generator=g) * 2.0 ** -128
+    ref, mag = (F.conv2d(t, u, padding=1) for t, u in ((tiny.double(), w.double()), (tiny.double().abs(),
+                                                                                     w.double().abs())))
+    assert ((run(tiny).double() - ref).abs() <= 180 * (2.0 ** -24 * mag + 2.0 ** -149)).all()
