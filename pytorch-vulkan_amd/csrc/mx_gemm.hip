@@ -256,16 +256,20 @@ constexpr TileChoice kTiles[] = {{256, 128, 2, 1.81}, {128, 256, 2, 1.75}, {128,
 constexpr int64_t kMaxSplitBytes = int64_t(64) << 20;  // partial products of one call
 constexpr int kSplitBK = 32;                           // K granularity of a split
 constexpr int kMinSplitSpan = 64;                      // shortest K range worth a split
+// Longest K that is split.  No layer comes near it (a weight gradient's K is
+// its batch's positions), and the stream tests take a product of K = 2^19 as
+// work that keeps one workgroup busy for milliseconds.
+constexpr int64_t kMaxSplitK = int64_t(1) << 18;
 
 // Estimated time: a CU holding n tiles runs at rate * occ(n), occ rising from
 // 0.71 with one resident tile to 1 with per_cu; a tile's first loads and its
 // stores cost as much as 41 more k; the sum of the partials moves
 // (splits + 1) outputs at 3.6 TB/s after a launch.  The figures are the
 // convolution planner's, whose tiles run the same product.
-double tile_cost(const TileChoice& t, int64_t m, int64_t n, int64_t batch, int64_t splits, int64_t kps) {
-  const double cu = cu_count();
-  const int64_t tiles = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch * splits;
-  const double per_cu = double((tiles + int64_t(cu) - 1) / int64_t(cu));
+// `tiles` without splits; `cu` the CU count, a runtime query made once a call.
+double tile_cost(const TileChoice& t, int64_t tiles, int64_t cu, int64_t m, int64_t n, int64_t batch, int64_t splits,
+                 int64_t kps) {
+  const double per_cu = double((tiles * splits + cu - 1) / cu);
   const double occ = std::min(1.0, 0.71 + 0.29 * (per_cu - 1) / double(t.per_cu - 1));
   double s = per_cu * 2.0 * t.bm * t.bn * (double(kps) + 41.0) / (0.85 * 157.3e12 / 256.0 * t.rate * occ) + 2e-6;
   if (splits > 1) s += double(splits + 1) * double(m * n * batch) * 4.0 / 3.6e12 + 3e-6;
@@ -293,13 +297,15 @@ void pick_gemm_tile(int64_t m, int64_t n, int64_t k, int64_t batch, bool vec, in
   }
   static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
   double best = -1;
+  const int64_t cu = cu_count();
   for (int i = first; i <= last; ++i) {
+    const int64_t tiles = ((m + kTiles[i].bm - 1) / kTiles[i].bm) * ((n + kTiles[i].bn - 1) / kTiles[i].bn) * batch;
     for (const int want : kSplits) {
       int64_t span = ((k + want - 1) / want + kSplitBK - 1) / kSplitBK * kSplitBK;
       const int64_t s = (k + span - 1) / span;
       if (s > 1 && (!split_ok || span < kMinSplitSpan || s * m * n * batch * 4 > kMaxSplitBytes)) break;
       if (s == 1) span = k;
-      const double cost = tile_cost(kTiles[i], m, n, batch, s, span);
+      const double cost = tile_cost(kTiles[i], tiles, cu, m, n, batch, s, span);
       if (best < 0 || cost < best) {
         best = cost;
         *tile = i;
@@ -378,7 +384,8 @@ int plan_gemm(const mx_gemm_desc* d, const float* a, const float* b, const float
   g->ma = pick_mode(p.a, p.a_sm, p.a_sk, p.a_sb, p.batch, p.M, p.K);
   g->mb = pick_mode(p.b, p.b_sn, p.b_sk, p.b_sb, p.batch, p.N, p.K);
   pick_gemm_tile(d->m, d->n, d->k, d->batch, is_vec(g->ma) && is_vec(g->mb), d->kernel,
-                 split_ok && d->n <= kVecStrideMax && d->m * d->n <= INT32_MAX, &g->tile, &p.splits, &p.kps);
+                 split_ok && d->k <= kMaxSplitK && d->n <= kVecStrideMax && d->m * d->n <= INT32_MAX, &g->tile,
+                 &p.splits, &p.kps);
   return MX_OK;
 }
 
