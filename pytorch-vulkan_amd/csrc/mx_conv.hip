@@ -856,7 +856,7 @@ int select_algo_heuristic(const mx_conv2d_desc& d, int phase, int requested, int
 // (forward / dInput, dWeight) the workgroups resident per CU and the CU's
 // throughput with a full set of such tiles, relative to 85% of its FP32 MFMA
 // peak (the split bf16 product passes 1).  Fitted with the constants of
-// plan_cost to measured times of every (tile, split) plan on MI355X.
+// TileCost to measured times of every (tile, split) plan on MI355X.
 struct TileRate {
   int per_cu;
   double rate;
@@ -889,18 +889,27 @@ const char* tile_name(int tile, int phase) {
 // forced and timed: the planner's picks sum to 0.7% above the best plan per
 // phase on phases over 40 us and 0.9% on the shorter ones, where the figures
 // that fitted the FP32 products were 10.2% and 1.5% above.
-double plan_cost(const TileInfo& ti, bool dweight, int64_t M, int64_t Ncols, int64_t G, int64_t splits, int64_t kps,
-                 int64_t out_elems) {
-  const TileRate& tr = dweight ? ti.dw : ti.fwd;
-  const double cu = cu_count();
-  const double cu_flops = 0.85 * 157.3e12 / 256.0;
-  const int64_t tiles = ((M + ti.bm - 1) / ti.bm) * ((Ncols + ti.bn - 1) / ti.bn) * G;
-  const int64_t per_cu = (tiles * splits + int64_t(cu) - 1) / int64_t(cu);
-  const double occ = std::min(1.0, 0.71 + 0.29 * double(per_cu - 1) / double(tr.per_cu - 1));
-  double t = double(per_cu) * 2.0 * ti.bm * ti.bn * (double(kps) + 41.0) / (cu_flops * tr.rate * occ) + 2e-6;
-  if (splits > 1) t += double(splits + 1) * double(out_elems) * 4.0 / 3.6e12 + 3e-6;
-  return t;
-}
+//
+// A call runs the planner each time, over up to 108 plans: the tile's share is
+// worked out once per tile and the CU count (a runtime query) once per call.
+struct TileCost {
+  double tile_s_per_k;  // seconds per k of one resident tile at rate 1
+  int64_t tiles, cu;
+  int per_cu;
+  TileCost(const TileInfo& ti, bool dweight, int64_t M, int64_t Ncols, int64_t G, int64_t cus) : cu(cus) {
+    const TileRate& tr = dweight ? ti.dw : ti.fwd;
+    tile_s_per_k = 2.0 * ti.bm * ti.bn / (0.85 * 157.3e12 / 256.0 * tr.rate);
+    tiles = ((M + ti.bm - 1) / ti.bm) * ((Ncols + ti.bn - 1) / ti.bn) * G;
+    per_cu = tr.per_cu;
+  }
+  double operator()(int64_t splits, int64_t kps, int64_t out_elems) const {
+    const int64_t n = (tiles * splits + cu - 1) / cu;
+    const double occ = std::min(1.0, 0.71 + 0.29 * double(n - 1) / double(per_cu - 1));
+    double t = double(n) * tile_s_per_k * (double(kps) + 41.0) / occ + 2e-6;
+    if (splits > 1) t += double(splits + 1) * double(out_elems) * 4.0 / 3.6e12 + 3e-6;
+    return t;
+  }
+};
 
 constexpr int kSplitBK = 32;         // K granularity of a split (a multiple of every loader run)
 constexpr int kMinSplitSpan = 128;   // shortest K range worth a split
@@ -931,9 +940,11 @@ int plan_gemm(bool dweight, int64_t M, int64_t Ncols, int64_t K, int64_t G, unsi
   GemmPlan best;
   double best_t = -1;
   bool budget_stop = false;
+  const int64_t cus = cu_count();
   static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256, 384, 512};
   for (int t = 0; t < conv::NTILES; ++t) {
     if (!(tiles & (1u << t)) || (force_tile >= 0 && t != force_tile)) continue;
+    const TileCost tile_cost(kTileInfo[t], dweight, M, Ncols, G, cus);
     for (int want : kSplits) {
       if (want > max_splits || (force_tile >= 0 && want > force_splits)) break;
       int64_t kps = (K + want - 1) / want;
@@ -944,7 +955,7 @@ int plan_gemm(bool dweight, int64_t M, int64_t Ncols, int64_t K, int64_t G, unsi
         budget_stop = true;
         break;
       }
-      const double cost = plan_cost(kTileInfo[t], dweight, M, Ncols, G, splits, kps, out_elems);
+      const double cost = tile_cost(splits, kps, out_elems);
       if (force_tile >= 0 || best_t < 0 || cost < best_t) {  // forced: the largest split that fits
         best_t = cost;
         best.tile = t;
@@ -996,7 +1007,14 @@ int plan_forward(const mx_conv2d_desc& d, const float* x, const float* w, const 
   p.M = p.Cout_g;
   p.Ncols = p.N * p.OHOW;
   p.K = p.Cin_g * p.KK;
-  f->packed = p.KK > 1 && conv::blocked_channels(p.Cin_g);
+  // The blocked K order makes the gather cheaper (one tap per slab) and costs
+  // a pass over the weights, so it pays from a number of positions on, which
+  // every weight value meets.  Measured, copy and all, blocked / plain order:
+  // 512 channels 4^2 20.9 / 12.0 us, 8^2 22.6 / 14.7, 16^2 31.7 / 29.6, 4 x
+  // 16^2 49.1 / 45.7; 256 channels 32^2 27.3 / 27.0; 32 x 512 at 8^2 73.6 /
+  // 77.3, 16 x 256 at 16^2 47.4 / 49.5, at 32^2 124 / 136.
+  f->packed = p.KK > 1 && conv::blocked_channels(p.Cin_g) && (int64_t(p.N) * p.OHOW > 1024 || !aligned16(w));
+  p.cols_blocked = f->packed || (p.KK == 1 && conv::blocked_channels(p.Cin_g));
   // Weight rows are read 16 bytes per lane: a K that is not a multiple of
   // four, or unaligned weights, get a copy with rows padded to a multiple of
   // four floats.
@@ -1015,7 +1033,7 @@ int plan_forward(const mx_conv2d_desc& d, const float* x, const float* w, const 
 
 std::string fwd_variant(const FwdPlan& f) {
   const char* b = f.bmode == conv::B_VEC ? "PosQuad"
-                  : conv::blocked_channels(f.p.Cin_g) ? "Im2col<blocked>" : "Im2col";
+                  : f.p.cols_blocked ? "Im2col<blocked>" : "Im2col";
   return cat("conv_fwd_kernel<", tile_name(f.gp.tile, MX_CONV_FORWARD), ",KVEC,", b, ">",
              f.gp.splits > 1 ? "+split" : "");
 }

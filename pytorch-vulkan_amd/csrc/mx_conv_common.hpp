@@ -69,8 +69,9 @@ struct ConvArgs {
   // (forward: KK * 16 and KW; dInput phase: nth * ntw * 16 and ntw).
   FastDiv f_kblk, f_tapw;
   FastDiv f_kk;  // non-blocked gathers: taps per channel (forward KK, dInput phase nth * ntw)
-  // dWeight: the B gather runs its columns in the channel-blocked order
-  // (channel block, kh, kw, channel in block); the epilogue maps them back.
+  // Forward: the B gather walks k in the channel-blocked order (channel block,
+  // kh, kw, channel in block), the weights packed to match.  dWeight: the B
+  // gather runs its columns in that order; the epilogue maps them back.
   int cols_blocked;
 };
 

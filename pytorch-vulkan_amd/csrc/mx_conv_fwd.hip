@@ -99,7 +99,7 @@ int launch_b(ConvArgs p, int bmode, hipStream_t s) {
   if (bmode == B_VEC) {
     hipLaunchKernelGGL((conv_fwd_kernel<C, MA, PosQuadLoader<C::BN, C::BK, false>>), grid, dim3(kThreads), 0, s, p);
   } else if constexpr (MA == Mode::KVEC) {
-    if (blocked_channels(p.Cin_g))
+    if (p.cols_blocked)
       hipLaunchKernelGGL((conv_fwd_kernel<C, MA, Im2colLoader<C::BN, C::BK, true>>), grid, dim3(kThreads), 0, s, p);
     else
       hipLaunchKernelGGL((conv_fwd_kernel<C, MA, Im2colLoader<C::BN, C::BK, false>>), grid, dim3(kThreads), 0, s, p);

@@ -273,3 +273,31 @@ def test_winograd_split_kernel_infinite_and_tiny(mx, monkeypatch):
     ref, mag = (F.conv2d(t, u, padding=1) for t, u in ((tiny.double(), w.double()), (tiny.double().abs(),
                                                                                      w.double().abs())))
     assert ((run(tiny).double() - ref).abs() <= 180 * (2.0 ** -24 * mag + 2.0 ** -149)).all()
+
+
+@pytest.mark.parametrize("n,c,h,wd,o,k,stride,dil,groups,shift", [
+    (1, 16, 32, 32, 64, 3, 1, 1, 1, 0),    # 1024 positions: the plain order's last
+    (1, 16, 25, 41, 64, 3, 1, 1, 1, 0),    # 1025: the blocked order's first
+    (1, 48, 8, 8, 70, 3, 1, 1, 1, 0),
+    (2, 32, 9, 11, 33, 5, 2, 1, 1, 0),
+    (1, 64, 7, 7, 130, 3, 1, 2, 2, 0),
+    (1, 512, 4, 4, 64, 3, 1, 1, 1, 0),     # long K: split
+    (1, 32, 8, 8, 40, 3, 1, 1, 1, 1),      # weights off a 16-byte boundary: packed at any size
+])
+def test_forward_weight_order(mx, n, c, h, wd, o, k, stride, dil, groups, shift):
+    """Forward layers of few positions read the weights where they are, in
+    their own K order; the others a copy in the blocked order."""
+    g = torch.Generator().manual_seed(c + o + h)
+    pad = dil * (k // 2)
+    d = mx.conv_desc((n, c * groups, h, wd), (o * groups, c, k, k), (stride, stride), (pad, pad), (dil, dil), groups)
+    x, w = torch.randn(n, c * groups, h, wd, generator=g), torch.randn(o * groups, c, k, k, generator=g)
+    xd, store = x.cuda(), torch.zeros(w.numel() + 4, device="cuda")
+    wdv = store[shift:shift + w.numel()].view_as(w)
+    wdv.copy_(w)
+    y = torch.full((n, o * groups, d.oh, d.ow), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    mx.conv2d_forward(d, xd, wdv, None, y, mx.ALGO_IMPLICIT_GEMM, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    ref, mag = (F.conv2d(a.double(), b.double(), None, stride, pad, dil, groups)
+                for a, b in ((x, w), (x.abs(), w.abs())))
+    assert ((y.cpu().double() - ref).abs() <= (c * k * k / 16 + 8) * 2.0 ** -23 * mag).all()
