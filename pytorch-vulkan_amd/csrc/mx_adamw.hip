@@ -281,22 +281,28 @@ struct Interval {
 // (one of them writes bytes the other reads or writes), or -1.  Gradients are
 // written when `grads_written` (a grad_scale unscales them in place).
 std::vector<int64_t> latest_conflict(const mx_adamw_tensor* t, int64_t n, bool ams, bool grads_written) {
+  std::vector<int64_t> conf(size_t(n), -1);
+  // Each list on its own usually comes in address order (parameters allocated
+  // in turn, or views of one flat buffer), so the intervals are appended list
+  // by list and merged, sorting only what is out of order.
   std::vector<Interval> iv;
   iv.reserve(size_t(n) * 5);
-  for (int64_t i = 0; i < n; ++i) {
-    if (t[i].numel <= 0) continue;
-    const uintptr_t bytes = uintptr_t(t[i].numel) * 4;
-    auto add = [&](const void* ptr, bool w) {
-      if (ptr) iv.push_back({reinterpret_cast<uintptr_t>(ptr), reinterpret_cast<uintptr_t>(ptr) + bytes, i, w});
-    };
-    add(t[i].param, true);
-    add(t[i].grad, grads_written);
-    add(t[i].exp_avg, true);
-    add(t[i].exp_avg_sq, true);
-    if (ams) add(t[i].max_exp_avg_sq, true);
-  }
-  std::sort(iv.begin(), iv.end(), [](const Interval& a, const Interval& b) { return a.lo < b.lo; });
-  std::vector<int64_t> conf(size_t(n), -1);
+  const auto below = [](const Interval& a, const Interval& b) { return a.lo < b.lo; };
+  auto add_list = [&](float* mx_adamw_tensor::*member, bool written) {
+    const auto from = iv.end() - iv.begin();
+    for (int64_t i = 0; i < n; ++i) {
+      const uintptr_t lo = reinterpret_cast<uintptr_t>(t[i].*member);
+      if (t[i].numel > 0 && lo) iv.push_back({lo, lo + uintptr_t(t[i].numel) * 4, i, written});
+    }
+    const auto mid = iv.begin() + from;
+    if (!std::is_sorted(mid, iv.end(), below)) std::sort(mid, iv.end(), below);
+    if (from && mid != iv.end() && below(*mid, mid[-1])) std::inplace_merge(iv.begin(), mid, iv.end(), below);
+  };
+  add_list(&mx_adamw_tensor::param, true);
+  add_list(&mx_adamw_tensor::grad, grads_written);
+  add_list(&mx_adamw_tensor::exp_avg, true);
+  add_list(&mx_adamw_tensor::exp_avg_sq, true);
+  if (ams) add_list(&mx_adamw_tensor::max_exp_avg_sq, true);
   // Sweep: compare each interval with the following ones that start before it ends.
   for (size_t a = 0; a < iv.size(); ++a)
     for (size_t b = a + 1; b < iv.size() && iv[b].lo < iv[a].hi; ++b) {
@@ -346,6 +352,9 @@ extern "C" int mx_adamw_step(const mx_adamw_tensor* tensors, int64_t count, cons
   hp.found_inf = h.found_inf;
   hp.maximize = h.maximize;
   std::vector<AdamEntry> tab;
+  tab.reserve(size_t(count));
+  int64_t corrected = 0;  // the step that the two factors below belong to (steps are 1 and up)
+  float neg_step_size = 0.f, bc2_sqrt = 0.f;
   int64_t first = 0;
   while (first < count) {
     // Extend the launch while no entry conflicts with one already in it.
@@ -366,10 +375,15 @@ extern "C" int mx_adamw_step(const mx_adamw_tensor* tensors, int64_t count, cons
       e.numel = t.numel;
       e.chunk_begin = chunks;
       if (!t.step_dev) {
-        const double bc1 = 1.0 - std::pow(h.beta1, double(t.step));
-        const double bc2 = 1.0 - std::pow(h.beta2, double(t.step));
-        e.neg_step_size = h.lr_dev ? float(-1.0 / bc1) : float(-(h.lr / bc1));
-        e.bc2_sqrt = float(std::sqrt(bc2));
+        if (t.step != corrected) {  // parameters of a group share their step: no pow() each
+          corrected = t.step;
+          const double bc1 = 1.0 - std::pow(h.beta1, double(t.step));
+          const double bc2 = 1.0 - std::pow(h.beta2, double(t.step));
+          neg_step_size = h.lr_dev ? float(-1.0 / bc1) : float(-(h.lr / bc1));
+          bc2_sqrt = float(std::sqrt(bc2));
+        }
+        e.neg_step_size = neg_step_size;
+        e.bc2_sqrt = bc2_sqrt;
       }
       e.vec = aligned16(e.p) && aligned16(e.g) && aligned16(e.m) && aligned16(e.v) && (!ams || aligned16(e.vmax));
       chunks += (t.numel + kChunk - 1) / kChunk;
