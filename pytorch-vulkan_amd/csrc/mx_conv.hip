@@ -29,6 +29,11 @@ namespace {
 using conv::ConvArgs;
 using conv::FastDiv;
 using conv::fdiv;
+using mfma::bload;
+using mfma::buffer_rsrc;
+using mfma::i32x4;
+using mfma::kBufMaxBytes;
+using mfma::kOffNone;
 using mfma::Mode;
 
 // ----------------------------------------------------------- direct kernels
@@ -121,10 +126,11 @@ __global__ void conv_dw_direct_kernel(ConvArgs p) {
 // planes in LDS, zeros where the patch leaves the plane, and its threads take
 // items of four rows of one column, all columns of all its planes numbered
 // through, so planes smaller than a wave's 64 columns leave no lane idle and a
-// value is read from HBM once.  32 x 192 x 28 x 28, 3x3: forward 71.6 -> 12,
-// input gradient (one thread per value before) 65 -> 15 us.
+// value is read from HBM once.  32 x 192 x 28 x 28, 3x3: forward 71.6 -> 18,
+// input gradient (one thread per value before) 65 -> 20 us.
 constexpr int kDwRows = 4;           // rows of an item
 constexpr int kDwLdsFloats = 12288;  // 48 KiB
+constexpr int kDwLoads = 6;          // values a thread has in flight while it stages
 // Tile of the kernel that reads x directly where a patch is larger than that
 // (very large dilation).
 constexpr int kDwTileW = 64, kDwTileH = 16, kDwRowsPerWave = 4;
@@ -138,6 +144,30 @@ struct DepthwiseArgs {
   int64_t tiles;
   FastDiv f_tw, f_strips, f_pw, f_patch, f_cin, f_sh, f_sw;
 };
+
+// The patches of consecutive h x w planes from `src` into LDS: rows y0 .. and
+// columns x0 .., zeros outside a plane.  A thread's next kDwLoads values are
+// loaded together, without branches (positions outside read the first value
+// and drop it): one load and LDS store at a time, each iteration waited for
+// its own load (forward 20.7 -> 17.9 us at the size above).
+__device__ __forceinline__ void depthwise_stage(const DepthwiseArgs& a, float* patch, const float* src, uint32_t total,
+                                                int y0, int x0, int h, int w) {
+  const uint32_t plane = uint32_t(h) * uint32_t(w);
+  for (uint32_t e0 = threadIdx.x; e0 < total; e0 += 256 * kDwLoads) {
+    float v[kDwLoads];
+    bool ok[kDwLoads];
+#pragma unroll
+    for (int u = 0; u < kDwLoads; ++u) {
+      const uint32_t e = e0 + 256 * u, pl = fdiv(e, a.f_patch), q = e - pl * a.patch, r = fdiv(q, a.f_pw);
+      const int y = y0 + int(r), x = x0 + int(q - r * a.patch_w);
+      ok[u] = e < total && unsigned(y) < unsigned(h) && unsigned(x) < unsigned(w);
+      v[u] = src[ok[u] ? pl * plane + uint32_t(y) * uint32_t(w) + uint32_t(x) : 0u];
+    }
+#pragma unroll
+    for (int u = 0; u < kDwLoads; ++u)
+      if (e0 + 256 * u < total) patch[e0 + 256 * u] = ok[u] ? v[u] : 0.f;
+  }
+}
 
 // Items of a tile: f(plane in the workgroup, first row, column).
 template <class F>
@@ -163,11 +193,7 @@ __global__ __launch_bounds__(256) void conv_depthwise_staged_kernel(DepthwiseArg
     const int oh0 = th * a.tile_h, ow0 = tw * a.tile_w;
     const int ih0 = oh0 * p.sh - p.ph, iw0 = ow0 * p.sw - p.pw;
     const float* const xp = p.x + int64_t(plane0) * p.HW;
-    for (uint32_t e = threadIdx.x; e < uint32_t(np * a.patch); e += 256) {
-      const uint32_t pl = fdiv(e, a.f_patch), q = e - pl * a.patch, r = fdiv(q, a.f_pw);
-      const int ih = ih0 + int(r), iw = iw0 + int(q - r * a.patch_w);
-      patch[e] = unsigned(ih) < unsigned(p.H) && unsigned(iw) < unsigned(p.W) ? xp[pl * p.HW + ih * p.W + iw] : 0.f;
-    }
+    depthwise_stage(a, patch, xp, uint32_t(np * a.patch), ih0, iw0, p.H, p.W);
     __syncthreads();
     for (int j = 0; j < m; ++j)
       depthwise_items(a, np, [&](int pl, int row, int col) {
@@ -217,12 +243,7 @@ __global__ __launch_bounds__(256) void conv_depthwise_dx_kernel(DepthwiseArgs a)
     const int oh0 = UNIT ? top : top >= 0 ? top / p.sh : -((p.sh - 1 - top) / p.sh);
     const int ow0 = UNIT ? left : left >= 0 ? left / p.sw : -((p.sw - 1 - left) / p.sw);
     const float* const dyp = p.dy + int64_t(plane0) * m * p.OHOW;  // planes of dy follow (image, channel, j)
-    for (uint32_t e = threadIdx.x; e < uint32_t(np * m * a.patch); e += 256) {
-      const uint32_t pl = fdiv(e, a.f_patch), q = e - pl * a.patch, r = fdiv(q, a.f_pw);
-      const int oh = oh0 + int(r), ow = ow0 + int(q - r * a.patch_w);
-      patch[e] = unsigned(oh) < unsigned(p.OH) && unsigned(ow) < unsigned(p.OW) ? dyp[pl * p.OHOW + oh * p.OW + ow]
-                                                                                : 0.f;
-    }
+    depthwise_stage(a, patch, dyp, uint32_t(np * m * a.patch), oh0, ow0, p.OH, p.OW);
     __syncthreads();
     depthwise_items(a, np, [&](int pl, int row, int col) {
       const uint32_t plane = plane0 + pl, img = fdiv(plane, a.f_cin);
@@ -258,34 +279,61 @@ __global__ __launch_bounds__(256) void conv_depthwise_dx_kernel(DepthwiseArgs a)
 }
 
 // Depthwise weight gradient, no scratch: one workgroup of 16 waves per (output
-// channel, filter row); a thread takes every 1024th output position with all
-// KW taps of the row (x from the caches), the sums meet in a fixed tree.  Row
-// 0's workgroup also sums dBias from the dy it reads.  One workgroup per
-// weight, with 64-bit divisions per position, took 121 us plus 38 us for dBias
-// at 32 x 192 x 28 x 28, 3x3.
+// channel, filter row).  A thread keeps one output position of `step` images
+// at a time and walks the images, so its offsets and bounds are worked out
+// once (decoded per position they were two thirds of the instructions) and
+// the loads of kDwImages steps are in flight together; the sums meet in a
+// fixed tree.  Row 0's workgroup also sums dBias from the dy it reads.
+// 32 x 192 x 28 x 28, 3x3: 33 -> 20 us (39 MB from HBM: 7.5 us; x and dy come
+// from the caches once per filter row).
+constexpr int kDwImages = 4;
+
 template <int KW>
-__global__ __launch_bounds__(1024) void conv_depthwise_dw_kernel(ConvArgs p) {
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) void conv_depthwise_dw_kernel(ConvArgs p,
+                                                                                                          int step) {
   __shared__ float part[16][KW + 1];
   const int oc = blockIdx.x, kh = blockIdx.y, ic = oc / p.Cout_g;
+  const uint32_t ohow = uint32_t(p.OHOW), hw = uint32_t(p.HW);
+  const uint32_t g_step = uint32_t(step) * p.Cout * ohow * 4u, x_step = uint32_t(step) * p.Cin * hw * 4u;
+  const i32x4 rdy = buffer_rsrc(p.dy, int64_t(p.N) * p.Cout * ohow * 4);
+  const i32x4 rx = buffer_rsrc(p.x, int64_t(p.N) * p.Cin * hw * 4);
   float acc[KW + 1] = {};
-  const uint32_t positions = uint32_t(p.N) * uint32_t(p.OHOW);
-#pragma unroll 2
-  for (uint32_t r = threadIdx.x; r < positions; r += 1024) {
-    const uint32_t img = fdiv(r, p.f_ohow), q = r - img * uint32_t(p.OHOW), oh = fdiv(q, p.f_ow);
+  for (uint32_t q0 = 0; q0 < ohow; q0 += blockDim.x) {
+    // Planes of up to 1024 positions: `step` images side by side.
+    const uint32_t il = ohow <= 1024 ? fdiv(threadIdx.x, p.f_ohow) : 0u;
+    const uint32_t q = q0 + threadIdx.x - il * ohow, oh = fdiv(q, p.f_ow);
+    const bool live = il < uint32_t(step) && q < ohow;
     const int ih = int(oh) * p.sh - p.ph + kh * p.dh, iw0 = int(q - oh * uint32_t(p.OW)) * p.sw - p.pw;
-    const float g = p.dy[(img * uint32_t(p.Cout) + oc) * uint32_t(p.OHOW) + q];
-    const float* const xr = p.x + (img * uint32_t(p.Cin) + ic) * uint32_t(p.HW);
-    float xv[KW];
+    // Offsets of the thread's values in the whole tensors; kOffNone plus what
+    // the walk adds stays out of range, and so do images past the last.
+    uint32_t g_off = live ? ((il * uint32_t(p.Cout) + oc) * ohow + q) * 4u : kOffNone;
+    uint32_t x_off[KW];
     bool ok[KW];
 #pragma unroll
     for (int k = 0; k < KW; ++k) {
       const int iw = iw0 + k * p.dw;
-      ok[k] = unsigned(ih) < unsigned(p.H) && unsigned(iw) < unsigned(p.W);
-      xv[k] = xr[ok[k] ? ih * p.W + iw : 0];
+      ok[k] = live && unsigned(ih) < unsigned(p.H) && unsigned(iw) < unsigned(p.W);
+      x_off[k] = ok[k] ? ((il * uint32_t(p.Cin) + ic) * hw + uint32_t(ih) * uint32_t(p.W) + uint32_t(iw)) * 4u : kOffNone;
     }
+    for (int img = 0; img < p.N; img += kDwImages * step) {
+      float g[kDwImages], xv[kDwImages][KW];
 #pragma unroll
-    for (int k = 0; k < KW; ++k) acc[k] += ok[k] ? xv[k] * g : 0.f;
-    acc[KW] += g;
+      for (int u = 0; u < kDwImages; ++u) {
+        g[u] = bload(rdy, g_off, 0);
+        g_off += g_step;
+#pragma unroll
+        for (int k = 0; k < KW; ++k) {
+          xv[u][k] = bload(rx, x_off[k], 0);
+          x_off[k] += x_step;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kDwImages; ++u) {
+#pragma unroll
+        for (int k = 0; k < KW; ++k) acc[k] = __builtin_fmaf(xv[u][k], ok[k] ? g[u] : 0.f, acc[k]);
+        acc[KW] += g[u];
+      }
+    }
   }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
@@ -298,7 +346,8 @@ __global__ __launch_bounds__(1024) void conv_depthwise_dw_kernel(ConvArgs p) {
   if (threadIdx.x <= KW) {
     float s = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) s += part[i][threadIdx.x];
+    for (int i = 0; i < 16; ++i)
+      if (i < int(blockDim.x) / 64) s += part[i][threadIdx.x];
     if (threadIdx.x < KW)
       p.out[(int64_t(oc) * p.KH + kh) * KW + threadIdx.x] = s;
     else if (kh == 0 && p.db)
@@ -600,15 +649,22 @@ bool conv_depthwise_dx(const mx_conv2d_desc& d, const ConvArgs& p, hipStream_t s
 }
 
 // Weight gradient (and dBias) of a depthwise layer with 1, 3, 5 or 7 filter
-// columns in place of the one-workgroup-per-weight reduction; false otherwise.
+// columns in place of the one-workgroup-per-weight reduction; false otherwise
+// (also where the walk over a tensor's images would pass a buffer's range).
 bool conv_depthwise_dw(const mx_conv2d_desc& d, const ConvArgs& p, hipStream_t s) {
-  if (d.cout > INT32_MAX / 16 || d.kh > 65535) return false;
-  const dim3 grid(unsigned(d.cout), unsigned(d.kh));
+  const int64_t step = std::max<int64_t>(1, 1024 / (d.oh * d.ow));
+  if (d.cout > INT32_MAX / 16 || d.kh > 65535 ||
+      (d.n + kDwImages * step) * std::max(d.cin * d.h * d.w, d.cout * d.oh * d.ow) * 4 >= kBufMaxBytes)
+    return false;
+  // As many waves as the positions taken at once fill: 28 x 28 runs on 13,
+  // so 576 workgroups (192 channels) are on the chip together.
+  const int64_t positions = step * d.oh * d.ow, chunks = (positions + 1023) / 1024;
+  const dim3 grid(unsigned(d.cout), unsigned(d.kh)), block(unsigned((positions + 64 * chunks - 1) / (64 * chunks) * 64));
   switch (d.kw) {
-    case 1: hipLaunchKernelGGL(conv_depthwise_dw_kernel<1>, grid, dim3(1024), 0, s, p); return true;
-    case 3: hipLaunchKernelGGL(conv_depthwise_dw_kernel<3>, grid, dim3(1024), 0, s, p); return true;
-    case 5: hipLaunchKernelGGL(conv_depthwise_dw_kernel<5>, grid, dim3(1024), 0, s, p); return true;
-    case 7: hipLaunchKernelGGL(conv_depthwise_dw_kernel<7>, grid, dim3(1024), 0, s, p); return true;
+    case 1: hipLaunchKernelGGL(conv_depthwise_dw_kernel<1>, grid, block, 0, s, p, int(step)); return true;
+    case 3: hipLaunchKernelGGL(conv_depthwise_dw_kernel<3>, grid, block, 0, s, p, int(step)); return true;
+    case 5: hipLaunchKernelGGL(conv_depthwise_dw_kernel<5>, grid, block, 0, s, p, int(step)); return true;
+    case 7: hipLaunchKernelGGL(conv_depthwise_dw_kernel<7>, grid, block, 0, s, p, int(step)); return true;
     default: return false;
   }
 }

@@ -39,6 +39,8 @@ DEPTHWISE = [  # x shape, multiplier, kernel, stride, padding, dilation
     ((2, 8, 16, 200), 1, (1, 4), (1, 2), (0, 3), (1, 7)),
     ((1, 8, 90, 90), 1, (3, 3), (1, 1), (40, 40), (40, 40)),  # patches beyond LDS
     ((130, 8, 4, 4), 1, (3, 3), (1, 1), (1, 1), (1, 1)),      # many planes to a workgroup
+    ((13, 8, 28, 28), 1, (3, 3), (1, 1), (1, 1), (1, 1)),     # images past a whole number of walks
+    ((333, 8, 7, 7), 2, (3, 3), (1, 1), (1, 1), (1, 1)),      # 20 images side by side
 ]
 
 
