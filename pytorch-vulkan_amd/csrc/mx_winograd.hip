@@ -27,7 +27,8 @@
 // 64-tile blocks with the products as six bf16 MFMAs over three-piece
 // operands; smaller ones run 16- or 32-tile blocks on v_mfma_f32_16x16x4f32.
 //
-// Unfused kernels (launches with few tiles, or MX_WINOGRAD_FUSED=0): the
+// Unfused kernels (few tiles and a channel walk that splitting the 16-tile
+// kernel's does not shorten enough, or MX_WINOGRAD_FUSED=0): the
 // filter, input and output
 // transforms run as separate passes around one batched MFMA GEMM of batch
 // 16*groups over U [16*G][Cout_g][Cin_g], V [16*G][Cin_g][T],
@@ -45,6 +46,8 @@ namespace mx {
 namespace conv {
 int sum_partials(const float* ws, const float* ws_db, int splits, int64_t n, int n_db, float* out, float* out_db,
                  hipStream_t s);
+int conv_sum_splits(const float* ws, int splits, int64_t n, float* out, const float* bias, int hw, int cout,
+                    hipStream_t s);
 }
 namespace {
 
@@ -190,6 +193,10 @@ struct Args {
   int64_t x_bytes, u_bytes, y_bytes, w_bytes;
   int Cin, H, W, Cout, OH, OW, ph, pw, C, O, Cpad, Opad, TH, TW, T, n_ob, nslab;
   int flip, y_even;  // split kernel: w read flipped and channel-swapped; y is 8-byte aligned
+  // 16-tile kernel with its channel walk split over gridDim.z: slabs of one
+  // part (even), and the floats between the parts' outputs (0 in one pass).
+  int part_slabs;
+  int64_t part_stride;
   mfma::FastDiv f_thw, f_tw;
 };
 
@@ -658,7 +665,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   const int b = mfma::xcd_remap(blockIdx.x, gridDim.x);
   const int ob = b % p.n_ob, tb = b / p.n_ob;
   const int o0 = ob * BO, t0 = tb * BT16;
-  const int nslab = p.nslab;  // even: the host pads the channels to 16
+  // This part's slabs (even: the host pads the channels to 16).
+  const int first = FILT ? 0 : int(blockIdx.z) * p.part_slabs;
+  const int nslab = FILT ? p.nslab : min(p.part_slabs, p.nslab - first);
 
   if (wave >= 6) {
     // ---- filter producers: rows a_row .. of the slab's U' block, 16 floats
@@ -680,7 +689,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     float wk[FILT ? 36 : 1];
     auto load = [&](int slab) {
       if constexpr (FILT == 0) {
-        const uint32_t sa = uint32_t(slab) * a_sstep;
+        const uint32_t sa = uint32_t(first + slab) * a_sstep;
 #pragma unroll
         for (int q = 0; q < 16; ++q) av[q] = mfma::bload4(ru, a_off, sa + uint32_t(q) * a_cstep);
       } else {
@@ -772,7 +781,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     }
     const uint32_t x_sstep = uint32_t(BK) * p.H * p.W * 4;
     auto load = [&](int slab) {
-      px.load(rx, uint32_t(slab) * x_sstep, uint32_t(p.x_bytes), !RAGGED || slab * BK + b_c < p.C);
+      px.load(rx, uint32_t(first + slab) * x_sstep, uint32_t(p.x_bytes), !RAGGED || (first + slab) * BK + b_c < p.C);
     };
     auto store = [&](float* Bs) {
       px.fix(rx);
@@ -871,7 +880,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const int o = o0 + wave * 16 + 4 * kq + v;
     bias_v[v] = (p.bias && o < p.O) ? p.bias[g * p.O + o] : 0.f;
   }
-  const i32x4 ry = mfma::buffer_rsrc(p.y, p.y_bytes);
+  const i32x4 ry = mfma::buffer_rsrc(p.y + (FILT ? 0 : blockIdx.z * p.part_stride), p.y_bytes);
   const uint32_t row_step = uint32_t(p.OW) * 4u;
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
@@ -1863,6 +1872,7 @@ struct RunPlan {
   bool fused = true;
   bool filt = false;          // the fused kernel transforms the filter itself (no filter launch)
   bool t16 = false;           // the 16-tile fused kernel (two workgroups per CU)
+  int parts = 1;              // parts of its channel walk, each with an output of its own to be summed
   int64_t chunk = 0;          // images per unfused pass
   int64_t unfused_bytes = 0;  // U, V and M of one pass
 };
@@ -1871,11 +1881,41 @@ struct RunPlan {
 int64_t split_blocks(const RunPlan& r) { return (int64_t(r.p.T) + ws::STILES - 1) / ws::STILES * r.p.n_ob; }
 int64_t split_filter_bytes(const RunPlan& r) { return int64_t(r.G) * 16 * r.p.Cpad * r.p.Opad * 6; }
 
+// The 16-tile kernel in us on MI355X: rounds of two workgroups per CU, 3 us and
+// 1.25 per slab of 8 each, a last round of at most one per CU taking three
+// quarters.
+double t16_cost(const RunPlan& r, int parts, int slabs) {
+  const int64_t cus = cu_count();
+  const int64_t wgs = (int64_t(r.p.T) + ws::BT16 - 1) / ws::BT16 * r.p.n_ob * r.G * parts;
+  const int64_t tail = wgs % (2 * cus);
+  const double rounds = double(wgs / (2 * cus)) + (tail == 0 ? 0.0 : tail <= cus ? 0.75 : 1.0);
+  return rounds * (3.0 + 1.25 * slabs);
+}
+
+// Splits the 16-tile kernel's channel walk where a few workgroups walk long
+// (kMinPart slabs a part and up), the parts' outputs summed by a second launch
+// (6 us with what it costs the host, and their bytes at 3.6 TB/s).
+constexpr int kMinPart = 8;
+void split_walk(RunPlan* r, int64_t out_elems, int64_t ws_limit) {
+  fused::Args& p = r->p;
+  double best = t16_cost(*r, 1, p.nslab);
+  for (int want = 2; want <= 8; ++want) {
+    const int slabs = (p.nslab + 2 * want - 1) / (2 * want) * 2, parts = (p.nslab + slabs - 1) / slabs;
+    if (slabs < kMinPart || parts < 2 || parts * out_elems * 4 > ws_limit) break;
+    const double cost = t16_cost(*r, parts, slabs) + 6.0 + double(parts + 1) * double(out_elems) * 4.0 / 3.6e6;
+    if (cost < best) {
+      best = cost;
+      r->parts = parts;
+      p.part_slabs = slabs;
+      p.part_stride = out_elems;
+    }
+  }
+}
+
 // The cheaper of the 16-tile and the split kernel, in us on MI355X: rounds of
 // workgroups over the CUs times a fixed part and a part per slab.  The split
-// kernel holds one workgroup per CU (10 + 2.9 per slab of 16); the 16-tile
-// kernel two (3 + 1.25 per slab of 8), a last round of at most one per CU
-// taking three quarters.  Measured, split / 16-tile: 128 channels 64 x 28^2
+// kernel holds one workgroup per CU (10 + 2.9 per slab of 16).
+// Measured, split / 16-tile: 128 channels 64 x 28^2
 // 67 / 79, 16 x 64^2 70 / 91; 256 channels 64 x 14^2 61 / 87, 16 x 32^2
 // 65 / 90; 512 -> 256 16 x 32^2 114 / 166; 64 channels 64 x 56^2 85 / 88,
 // 8 x 56^2 23 / 18; 96 -> 160 8 x 40^2 30 / 33 and its input gradient 40 / 32;
@@ -1886,10 +1926,7 @@ bool prefer_t16(const RunPlan& r, bool dinput) {
   if (dinput && r.p.nslab <= 8 && r.blocks * r.G <= cu_count()) return true;
   const int64_t cus = cu_count();
   const int64_t split_rounds = (split_blocks(r) * r.G + cus - 1) / cus;
-  const int64_t b16 = (int64_t(r.p.T) + ws::BT16 - 1) / ws::BT16 * r.p.n_ob * r.G;
-  const int64_t tail = b16 % (2 * cus);
-  const double t16_rounds = double(b16 / (2 * cus)) + (tail == 0 ? 0.0 : tail <= cus ? 0.75 : 1.0);
-  return t16_rounds * (3.0 + 1.25 * r.p.nslab) <= double(split_rounds) * (10.0 + 2.9 * (r.p.nslab / 2));
+  return t16_cost(r, 1, r.p.nslab) <= double(split_rounds) * (10.0 + 2.9 * (r.p.nslab / 2));
 }
 
 int plan_run(const mx_conv2d_desc& d, int64_t ws_limit, bool dinput, RunPlan* r) {
@@ -1931,8 +1968,19 @@ int plan_run(const mx_conv2d_desc& d, int64_t ws_limit, bool dinput, RunPlan* r)
   const int64_t wgs = r->blocks * r->G;
   // MX_WINOGRAD_FUSED=1 / 0 forces the fused / unfused kernels (tests, tuning).
   r->fused = fused::prefer_fused(wgs, p.nslab);
+  p.part_slabs = p.nslab;
+  bool forced = false;
   if (const char* e = std::getenv("MX_WINOGRAD_FUSED"))
-    if (e[0] == '0' || e[0] == '1') r->fused = e[0] == '1';
+    if (e[0] == '0' || e[0] == '1') r->fused = e[0] == '1', forced = true;
+  if (!r->fused && !forced) {
+    // In place of the unfused passes, whose four launches move V and M through
+    // memory.  Measured, unfused / split walk: 256 channels 32^2 28.9 / 20.5 us,
+    // 8 x 16^2 31.6 / 25.5; 512 -> 256 32^2 34.7 / 27.8; 384 -> 128 64^2 39.8 /
+    // 30.3; 512 channels 16 x 8^2 41.5 / 39.4, 8 x 14^2 61.3 / 57.1; 320
+    // channels 2 x 16^2 30.7 / 21.8; 1024 -> 512 24^2 56.3 / 60.3.
+    split_walk(r, d.n * int64_t(p.Cout) * p.OH * p.OW, ws_limit);
+    if (r->parts > 1) r->fused = true;
+  }
   const int64_t u_plain = 16 * int64_t(p.Cout) * p.C * 4;
   const int64_t per_image = 16 * (int64_t(p.Cin) + p.Cout) * p.TH * p.TW * 4;
   const int64_t fit = ws_limit > u_plain ? (ws_limit - u_plain) / per_image : 0;
@@ -1953,13 +2001,14 @@ int plan_run(const mx_conv2d_desc& d, int64_t ws_limit, bool dinput, RunPlan* r)
   if (const char* e = std::getenv("MX_WINOGRAD_FILTER"))
     if (e[0] == '0' || e[0] == '1') r->filt = e[0] == '1';
   r->filt = r->filt && r->fused;
-  r->t16 = prefer_t16(*r, dinput);
+  r->t16 = r->parts > 1 || prefer_t16(*r, dinput);
   if (const char* e = std::getenv("MX_WINOGRAD_T16"))
-    if (e[0] == '0' || e[0] == '1') r->t16 = e[0] == '1';
+    if (e[0] == '0' || e[0] == '1') r->t16 = e[0] == '1', forced = true;
   // The split filter takes half as much again; past the buffer bound the
   // 16-tile kernel runs.
   if (!r->filt && split_filter_bytes(*r) >= mfma::kBufMaxBytes) r->t16 = true;
   r->t16 = r->t16 && r->fused;
+  if (!r->t16 || r->filt) r->parts = 1, p.part_slabs = p.nslab, p.part_stride = 0;
   if (r->filt) {
     p.w_bytes = int64_t(d.cout) * p.C * 9 * 4;
     MX_REQUIRE(p.w_bytes < mfma::kBufMaxBytes, MX_ERR_UNSUPPORTED, "winograd: the filter exceeds 2 GiB");
@@ -2025,11 +2074,18 @@ int winograd_run(const mx_conv2d_desc& d, const float* x, const float* w, const 
   hipLaunchKernelGGL(fused::filter_kernel, dim3(unsigned(std::min<int64_t>((filter_threads + 63) / 64, 1 << 20))),
                      dim3(64), 0, s, w, U.as<float>(), p.C, p.O, p.Cpad, p.Opad, r.G, flip);
   MX_HIP(hipGetLastError());
-  const dim3 grid16{unsigned((int64_t(p.T) + ws::BT16 - 1) / ws::BT16 * p.n_ob), unsigned(r.G), 1u};
+  Scratch parts;
+  if (r.parts > 1) {
+    MX_TRY(parts.alloc(size_t(r.parts) * p.part_stride * 4, s));
+    p.y = parts.as<float>();
+    p.bias = nullptr;
+  }
+  const dim3 grid16{unsigned((int64_t(p.T) + ws::BT16 - 1) / ws::BT16 * p.n_ob), unsigned(r.G), unsigned(r.parts)};
   void (*k16)(fused::Args) = ragged ? ws::wino_ws16_kernel<true, 0> : ws::wino_ws16_kernel<false, 0>;
   hipLaunchKernelGGL(k16, grid16, dim3(512), 0, s, p);
   MX_HIP(hipGetLastError());
-  return MX_OK;
+  if (r.parts == 1) return MX_OK;
+  return conv::conv_sum_splits(p.y, r.parts, p.part_stride, y, bias, p.OH * p.OW, p.Cout, s);
 }
 
 // Launch plan of the Winograd weight gradient: K ranges of output tiles sized
@@ -2180,7 +2236,7 @@ int winograd_describe(const mx_conv2d_desc& d, int phase, bool with_bias, int64_
   if (r.fused) {
     *variant = cat(r.t16 ? "wino_ws16_kernel<" : "wino_ws_kernel<", r.p.C % (2 * fused::BK) ? "ragged" : "even",
                    r.filt ? ",filter>" : ">");
-    *ws_bytes = 0;
+    *ws_bytes = r.parts > 1 ? r.parts * r.p.part_stride * 4 : 0;
   } else {
     // U, V and M are fresh mx_malloc blocks (256-byte aligned).
     const mx_gemm_desc gd = unfused_gemm_desc(r.G, r.p.O, r.p.C, r.chunk * r.p.TH * r.p.TW);
@@ -2218,7 +2274,7 @@ static int winograd_backward_plan(const mx_conv2d_desc& d, int64_t ws_limit, boo
   if (d.ph > 2 || d.pw > 2) return MX_OK;
   MX_TRY(plan_run(dinput_as_forward(d), ws_limit, true, rf));
   MX_TRY(plan_dw_run(d, ws_limit, with_db, rw));
-  if (!rf->fused || !rw->ws || rf->p.T == 0 || rw->p.T == 0) return MX_OK;
+  if (!rf->fused || rf->parts > 1 || !rw->ws || rf->p.T == 0 || rw->p.T == 0) return MX_OK;
   const int64_t cus = cu_count(), n_dx32 = rf->blocks * rf->G, n_dw_all = rw->blocks * rw->ranges;
   bool o = 4 * (n_dx32 + n_dw_all) <= cus ||
            (rf->p.nslab <= 8 && n_dx32 <= cus && 2 * (n_dx32 + n_dw_all) >= 3 * cus);

@@ -301,3 +301,46 @@ def test_forward_weight_order(mx, n, c, h, wd, o, k, stride, dil, groups, shift)
     ref, mag = (F.conv2d(a.double(), b.double(), None, stride, pad, dil, groups)
                 for a, b in ((x, w), (x.abs(), w.abs())))
     assert ((y.cpu().double() - ref).abs() <= (c * k * k / 16 + 8) * 2.0 ** -23 * mag).all()
+
+
+@pytest.mark.parametrize("n,c,hw,o,groups", [
+    (1, 256, (16, 32), 64, 1),     # even slabs, 16-channel parts
+    (1, 145, (23, 24), 70, 1),     # ragged channels, a shorter last part
+    (2, 200, (16, 17), 40, 1),     # odd width, one block of channels
+    (1, 160, (24, 24), 64, 2),
+])
+@pytest.mark.parametrize("flip", [False, True])
+def test_winograd_split_walk(mx, monkeypatch, n, c, hw, o, groups, flip):
+    """The 16-tile Winograd kernel with its channel walk in parts, against
+    float64 and, without scratch, in one pass (C FP32 roundings of the
+    transforms' magnitudes, and seven additions around them)."""
+    g = torch.Generator().manual_seed(c + o)
+    # flip: the input gradient of a layer whose output channels are the walk.
+    ci, co = (o, c) if flip else (c, o)
+    d = mx.conv_desc((n, ci * groups, *hw), (co * groups, ci, 3, 3), (1, 1), (1, 1), (1, 1), groups)
+    w = torch.randn(co * groups, ci, 3, 3, generator=g)
+    x, bias = torch.randn(n, c * groups, *hw, generator=g), torch.randn(o * groups, generator=g)
+    xd, wd, bd = x.cuda(), w.cuda(), bias.cuda()
+    st = torch.cuda.current_stream().cuda_stream
+
+    def run():
+        out = torch.full((n, o * groups, *hw), float("nan"), device="cuda")
+        torch.cuda.synchronize()
+        if flip:
+            mx.conv2d_backward_input(d, xd, wd, out, mx.ALGO_WINOGRAD, st)
+        else:
+            mx.conv2d_forward(d, xd, wd, bd, out, mx.ALGO_WINOGRAD, st)
+        torch.cuda.synchronize()
+        return out.cpu().double()
+
+    wt = w.reshape(groups, c, o, 3, 3).flip(3, 4).transpose(1, 2).reshape(groups * o, c, 3, 3) if flip else w
+    ref = F.conv2d(x.double(), wt.double(), None if flip else bias.double(), padding=1, groups=groups)
+    mag = torch.cat([winograd_magnitude(xs, ws, (1, 1), *hw)
+                     for xs, ws in zip(x.chunk(groups, 1), wt.chunk(groups, 0))], 1) + bias.abs().view(1, -1, 1, 1)
+    phase = mx.MX_CONV_DINPUT if flip else mx.MX_CONV_FORWARD
+    plan = mx.conv2d_plan(d, phase, mx.ALGO_WINOGRAD)
+    assert plan["variant"].startswith("wino_ws16_kernel") and plan["workspace_bytes"] > 0
+    assert ((run() - ref).abs() <= (c + 16) * 2.0 ** -24 * mag).all()
+    monkeypatch.setenv("TORCH_VULKAN_CONV_WORKSPACE_MB", "0")
+    assert mx.conv2d_plan(d, phase, mx.ALGO_WINOGRAD)["workspace_bytes"] == 0
+    assert ((run() - ref).abs() <= (c + 16) * 2.0 ** -24 * mag).all()
