@@ -80,8 +80,9 @@ struct ConvArgs {
 // channel in block): a loader's run of consecutive k (at most kChanBlock) then
 // shares one tap, so one bounds test covers it and its addresses are one
 // channel plane apart, while the taps of one channel block stay within a few
-// slabs (the input lines they share stay in L1).  Other channel counts keep
-// the plain (channel, kh, kw) order.  The weights are packed to match.
+// slabs (the input lines they share stay in L1).  Other channel counts, and
+// forward layers of few positions (plan_forward), keep the plain (channel, kh,
+// kw) order.  The weights are packed to match the blocked one.
 constexpr int kChanBlock = 16;
 __host__ __device__ constexpr bool blocked_channels(int c) { return c % kChanBlock == 0; }
 
