@@ -28,10 +28,9 @@
 // operands; smaller ones run 16- or 32-tile blocks on v_mfma_f32_16x16x4f32.
 //
 // Unfused kernels (few tiles and a channel walk that splitting the 16-tile
-// kernel's does not shorten enough, or MX_WINOGRAD_FUSED=0): the
-// filter, input and output
-// transforms run as separate passes around one batched MFMA GEMM of batch
-// 16*groups over U [16*G][Cout_g][Cin_g], V [16*G][Cin_g][T],
+// kernel's does not shorten enough, or MX_WINOGRAD_FUSED=0): the filter, input
+// and output transforms run as separate passes around one batched MFMA GEMM of
+// batch 16*groups over U [16*G][Cout_g][Cin_g], V [16*G][Cin_g][T],
 // M [16*G][Cout_g][T] with T = N * ceil(OH/2) * ceil(OW/2).
 #include <hip/hip_runtime.h>
 
