@@ -5,13 +5,13 @@
 // FP32 accuracy.  Operands are staged through LDS in double-buffered BK slabs.
 // On the way into LDS each FP32 value is split into three bf16 pieces, and the
 // product runs as six bf16 MFMAs per 16 k (SplitStage, mma_slab_split); tiles
-// whose result is out of the pieces' range run again on FP32 MFMA
-// (tile_product).  Each operand loader chooses its LDS layout: row-major with
-// k contiguous or k-major with rows contiguous, whichever its global reads can
-// fill with wide LDS stores (a row-contiguous operand written row-major would
-// be a strided transpose).  Each wave owns a (BM/WAVES_M) x (BN/WAVES_N)
-// sub-tile built from 32x32 blocks.  Inside a slab lane half h (lane / 32)
-// handles k in [h*BK/2, (h+1)*BK/2) for both operands.
+// whose result is not finite run again on FP32 MFMA (tile_product).  Each
+// operand loader chooses its LDS layout: row-major with k contiguous or k-major
+// with rows contiguous, whichever its global reads can fill with wide LDS
+// stores (a row-contiguous operand written row-major would be a strided
+// transpose).  Each wave owns a (BM/WAVES_M) x (BN/WAVES_N) sub-tile built from
+// 32x32 blocks.  Inside a slab lane half h (lane / 32) handles k in [h*BK/2,
+// (h+1)*BK/2) for both operands.
 //
 // Cfg::OCC is the register budget in waves per SIMD the kernels are compiled
 // for (amdgpu_waves_per_eu): 2 keeps a 128 x 128 tile in 256 registers so two
@@ -175,12 +175,18 @@ struct F32Stage {
   }
 };
 
-// Split stage: each FP32 value as three bf16 pieces, x = hi + mid + lo, every
-// piece the round-to-nearest bf16 of what the pieces before it leave (3 x 8
-// significant bits: the sum is x exactly), in three planes.  The split
-// happens here, on the way into LDS, so each operand value is split once per
-// workgroup and the product loop reads ready bf16 fragments; splitting the
-// fragments after the LDS read costs every wave of a tile row or column the
+// Split stage: each FP32 value as three bf16 pieces, 2^16 x = hi + mid + lo,
+// every piece the round-to-nearest bf16 of what the pieces before it leave (3 x
+// 8 significant bits: the sum is exact), in three planes.  bf16 ends at 2^-133
+// and FP32 at 2^-149; the factor puts FP32's last bit on bf16's (conversions
+// and both matrix instructions keep denormals), without it a value below 2^-110
+// loses bits whatever the factor it meets.  It costs a multiplication per value
+// (1x1 conv 128 -> 512 at 64x28x28 forward + backward 170 -> 173 us, linear
+// 8192 x 4096 x 4096 4144 -> 4119; noting such values instead, three
+// operations a pair, 178 and 4342); the sums carry 2^32 until they are stored.
+// The split happens here, on the way into LDS, so each operand value is split
+// once per workgroup and the product loop reads ready bf16 fragments; splitting
+// the fragments after the LDS read costs every wave of a tile row or column the
 // same work again (256x128 tile, 8192 x 4096 x 4096: 179 TFLOP/s that way).
 // Row-major planes are [k / 8][row][8]: a lane's fragment (8 k of one row) is
 // one 16-byte read and consecutive rows are contiguous; the row index of the
@@ -194,7 +200,10 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-// hi / mid / lo pairs of two values.  The residuals x - piece come from
+// What pieces are scaled by, and back from a product of two.
+constexpr float kPieceScale = 0x1p16f, kProductScale = 0x1p-32f;
+
+// hi / mid / lo pairs of two (scaled) values.  The residuals x - piece come from
 // v_dot2c_f32_bf16 (x + piece0 * -1 + piece1 * 0), which reads the packed pair
 // in place and is exact here; its constants stay in scalar registers because
 // the compiler folds them to an inline constant that the packed operand reads
@@ -224,6 +233,7 @@ struct SplitStage {
   float* p;
   __device__ __forceinline__ uint16_t* at(int elem) const { return reinterpret_cast<uint16_t*>(p) + elem; }
   __device__ __forceinline__ void put4(int elem, f32x4 v) const {
+    v *= kPieceScale;
     const Pieces2 a = split2(v[0], v[1]), b = split2(v[2], v[3]);
     *reinterpret_cast<u32x2*>(at(elem)) = u32x2{a.hi, b.hi};
     *reinterpret_cast<u32x2*>(at(elem + PLANE)) = u32x2{a.mid, b.mid};
@@ -243,7 +253,7 @@ struct SplitStage {
         u32x4 w[3];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const Pieces2 s = split2(v[e + 2 * q], v[e + 2 * q + 1]);
+          const Pieces2 s = split2(v[e + 2 * q] * kPieceScale, v[e + 2 * q + 1] * kPieceScale);
           w[0][q] = s.hi, w[1][q] = s.mid, w[2][q] = s.lo;
         }
         const int elem = row_elem(row, k + e);
@@ -266,7 +276,7 @@ struct SplitStage {
       const float mine = odd ? v[q + 1] : v[q], give = odd ? v[q] : v[q + 1];
       const float got = __builtin_bit_cast(
           float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, give), 0xB1, 0xF, 0xF, true));  // lane ^ 1
-      const Pieces2 s = split2(odd ? got : mine, odd ? mine : got);
+      const Pieces2 s = split2((odd ? got : mine) * kPieceScale, (odd ? mine : got) * kPieceScale);
       const int elem = row_elem(row0 + (q + (odd ? 1 : 0)) * step, k & ~1);
       *reinterpret_cast<uint32_t*>(at(elem)) = s.hi;
       *reinterpret_cast<uint32_t*>(at(elem + PLANE)) = s.mid;
@@ -372,7 +382,7 @@ __device__ __forceinline__ void mma_slab(Acc<C>& acc, const float* As, const flo
 }
 
 // FP32 main loop over nk slabs: the products on v_mfma_f32_32x32x2f32.  It
-// runs where the split loop's result is out of that loop's range (below).
+// runs where the split loop's result is not finite (tile_product).
 // Loaders expose load() (global -> registers, advancing their k cursor by
 // one slab), skip() (one slab on without
 // loading), store(stage) and KMAJOR (whether store() calls col4).  Two LDS
@@ -558,45 +568,43 @@ __device__ __forceinline__ void mainloop_split(Acc<C>& acc, LA& la, LB& lb, int 
 }
 
 // True, for the whole workgroup, when some accumulator of a split product is
-// not to be trusted: not finite (an infinite or huge operand has no finite
-// pieces, and inf * 0 = NaN where FP32 gives inf), or nonzero below 2^-80
-// (operands below 2^-110 lose the low bits of `lo` to bf16's smallest
-// denormal; only a product with a factor above 2^30 can hide them).  An
-// operand below 2^-134 has no nonzero piece and counts as zero.  Uses the
-// first four words of smem, free after the main loop's last barrier.
+// not finite: an infinite operand, or one that the piece scale takes there
+// (from 2^112 up), has no finite pieces, and neither inf - inf nor inf * 0 of
+// pieces is what FP32 gives; sums from 2^96 up overflow with the scale.  Uses
+// the first four words of smem, free after the main loop's last barrier.
 template <class C>
-__device__ __forceinline__ bool acc_out_of_range(const Acc<C>& acc, float* smem) {
-  uint32_t top = 0, low = ~0u;
+__device__ __forceinline__ bool acc_not_finite(const Acc<C>& acc, float* smem) {
+  uint32_t top = 0;
 #pragma unroll
   for (int i = 0; i < C::FM; ++i)
 #pragma unroll
     for (int j = 0; j < C::FN; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const uint32_t mag = __float_as_uint(acc.v[i][j][v]) << 1;
-        top = max(top, mag);
-        low = min(low, mag - 1);  // zero wraps to the top
-      }
-  const bool bad = top >= 0xFF000000u || low < (uint32_t(127 - 80) << 24) - 1;
+      for (int v = 0; v < 16; ++v) top = max(top, __float_as_uint(acc.v[i][j][v]) << 1);
   int* flags = reinterpret_cast<int*>(smem);
-  const bool any = __any(bad);
+  const bool any = __any(top >= 0xFF000000u);
   if ((threadIdx.x & 63) == 0) flags[threadIdx.x >> 6] = any;
   __syncthreads();
   return (flags[0] | flags[1] | flags[2] | flags[3]) != 0;
 }
 
 // The tile's product over nk slabs: the split loop, and again in FP32 where
-// its result is out of the split's range.  init(la, lb) sets up fresh loaders;
-// la ends as the loader of the loop that counted (its row sums are whole).
+// its result is not finite.  init(la, lb) sets up fresh loaders; la ends as the
+// loader of the loop that counted (its row sums are whole).  Returns what the
+// caller multiplies the accumulators by as it stores them (a pass of its own
+// over them spills).
 template <class C, class LA, class LB, class Init>
-__device__ __forceinline__ void tile_product(Acc<C>& acc, LA& la, LB& lb, int nk, float* smem, Init&& init) {
+__device__ __forceinline__ float tile_product(Acc<C>& acc, LA& la, LB& lb, int nk, float* smem, Init&& init) {
   init(la, lb);
   mainloop_split<C>(acc, la, lb, nk, smem);
-  if (acc_out_of_range<C>(acc, smem)) {
+  float scale = kProductScale;
+  if (acc_not_finite<C>(acc, smem)) {
     __syncthreads();  // every wave has read the flags before the stages are written
     init(la, lb);
     mainloop_f32<C>(acc, la, lb, nk, smem);
+    scale = 1.f;
   }
+  return scale;
 }
 
 // 32x32 output layout: lane l, register v -> row 8 * (v / 4) + 4 * (l / 32) + v % 4,

@@ -45,7 +45,7 @@ MX_TILE_KERNEL(C) void conv_dw_kernel(ConvArgs p) {
   LA la;
   LB lb;
   Acc<C> acc;
-  tile_product<C>(acc, la, lb, (k_end - k_begin + C::BK - 1) / C::BK, smem, [&](auto& a, auto& b) {
+  const float scale = tile_product<C>(acc, la, lb, (k_end - k_begin + C::BK - 1) / C::BK, smem, [&](auto& a, auto& b) {
     a.init(p, row0, g, k_begin, k_end);
     b.init(p, col0, g, k_begin, k_end);
   });
@@ -71,7 +71,7 @@ MX_TILE_KERNEL(C) void conv_dw_kernel(ConvArgs p) {
     }
     ccol[j] = n < p.Ncols ? uint32_t(c) * 4u : kOffNone;
   }
-  store_tile<C>(ro, ccol, uint32_t(p.Ncols) * 4u, row0, p.M, [&](int i, int j, int v) { return acc.v[i][j][v]; });
+  store_tile<C>(ro, ccol, uint32_t(p.Ncols) * 4u, row0, p.M, [&](int i, int j, int v) { return acc.v[i][j][v] * scale; });
   if (p.db != nullptr && tn == 0) {
     float* dbd = (p.splits == 1 ? p.db : p.ws_db + int64_t(split) * p.Cout) + g * p.Cout_g;
     const int tid = threadIdx.x;

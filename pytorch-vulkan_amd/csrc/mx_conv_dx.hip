@@ -77,7 +77,7 @@ __device__ __forceinline__ void dx_tile(const ConvArgs& p, int g, int lin, int s
   BufStridedLoader<C::BM, C::BK, MA> la;  // element (ci, k) = wt[g][k][ci]
   LB lb;
   Acc<C> acc;
-  tile_product<C>(acc, la, lb, (k1 - k0 + C::BK - 1) / C::BK, smem, [&](auto& a, auto& b) {
+  const float scale = tile_product<C>(acc, la, lb, (k1 - k0 + C::BK - 1) / C::BK, smem, [&](auto& a, auto& b) {
     a.init(p.wt + int64_t(g) * p.K * p.Cin_g, int64_t(p.K) * p.Cin_g * 4, 1, p.Cin_g, row0, p.M, k0, k1);
     b.init(p, col0, g, k0, k1);
   });
@@ -107,7 +107,7 @@ __device__ __forceinline__ void dx_tile(const ConvArgs& p, int g, int lin, int s
 #pragma unroll
       for (int j = 0; j < C::FN; ++j) {
         if (!ok[j]) continue;
-        *reinterpret_cast<float2*>(dst + cb[j]) = float2{acc.v[i][j][v], 0.f};
+        *reinterpret_cast<float2*>(dst + cb[j]) = float2{acc.v[i][j][v] * scale, 0.f};
         if (row2[j]) *reinterpret_cast<float2*>(dst + cb[j] + p.W) = float2{0.f, 0.f};
       }
     });
@@ -130,7 +130,7 @@ __device__ __forceinline__ void dx_tile(const ConvArgs& p, int g, int lin, int s
     col[j] = cok ? uint32_t((img * p.Cin + g * p.Cin_g) * p.HW + (p.pa + p.sh * i) * p.W + p.pb + p.sw * (q - i * p.Wp)) * 4u
                  : kOffNone;
   }
-  store_tile<C>(ro, col, uint32_t(p.HW) * 4u, row0, p.M, [&](int i, int j, int v) { return acc.v[i][j][v]; });
+  store_tile<C>(ro, col, uint32_t(p.HW) * 4u, row0, p.M, [&](int i, int j, int v) { return acc.v[i][j][v] * scale; });
 }
 
 template <class C, Mode MA, class LB>
@@ -174,6 +174,11 @@ int launch_a(const ConvArgs& p, Mode ma, int bmode, hipStream_t s) {
   return launch_b<C, Mode::RSCALAR>(p, bmode, s);
 }
 
+// Not built, for its registers: the phases' shared launch of 256-row tiles that
+// read both scalar weight rows and gathers in the plain order.
+template <class C, Mode MA>
+constexpr bool dx_phases_built = !(C::BM == 256 && MA == Mode::RSCALAR);
+
 template <class C, Mode MA>
 int launch_set_b(DxPhaseSet set, int bmode, hipStream_t s) {
   int most = 0;
@@ -190,9 +195,11 @@ int launch_set_b(DxPhaseSet set, int bmode, hipStream_t s) {
   else if (blocked_channels(set.q[0].Cout_g))
     hipLaunchKernelGGL((conv_dx_phases_kernel<C, MA, PhaseGatherLoader<C::BN, C::BK, true>>), grid, dim3(kThreads), 0,
                        s, set);
-  else
+  else if constexpr (dx_phases_built<C, MA>)
     hipLaunchKernelGGL((conv_dx_phases_kernel<C, MA, PhaseGatherLoader<C::BN, C::BK, false>>), grid, dim3(kThreads),
                        0, s, set);
+  else
+    for (int i = 0; i < set.n; ++i) MX_TRY((launch_b<C, MA>(set.q[i], bmode, s)));
   MX_HIP(hipGetLastError());
   return MX_OK;
 }

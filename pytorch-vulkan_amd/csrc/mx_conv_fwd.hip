@@ -27,7 +27,7 @@ MX_TILE_KERNEL(C) void conv_fwd_kernel(ConvArgs p) {
   BufStridedLoader<C::BM, C::BK, MA> la;
   LB lb;
   Acc<C> acc;
-  tile_product<C>(acc, la, lb, (k1 - k0 + C::BK - 1) / C::BK, smem, [&](auto& a, auto& b) {
+  const float scale = tile_product<C>(acc, la, lb, (k1 - k0 + C::BK - 1) / C::BK, smem, [&](auto& a, auto& b) {
     a.init(p.wt + int64_t(g) * p.Cout_g * p.ldw, int64_t(p.Cout_g) * p.ldw * 4, p.ldw, 1, row0, p.M, k0, k1);
     b.init(p, col0, g, k0, k1);
   });
@@ -60,7 +60,7 @@ MX_TILE_KERNEL(C) void conv_fwd_kernel(ConvArgs p) {
     col[j] = pos < uint32_t(p.Ncols) ? ((img * p.Cout + g * p.Cout_g) * p.OHOW + (pos - img * p.OHOW)) * 4u : kOffNone;
   }
   store_tile<C>(ro, col, uint32_t(p.OHOW) * 4u, row0, p.M,
-                [&](int i, int j, int v) { return acc.v[i][j][v] + b[i][v >> 2][v & 3]; });
+                [&](int i, int j, int v) { return acc.v[i][j][v] * scale + b[i][v >> 2][v & 3]; });
 }
 
 // Wp[g][co][k] = w[g*Cout_g + co][ci][kh][kw] with k the blocked gathered

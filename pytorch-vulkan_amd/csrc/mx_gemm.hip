@@ -54,7 +54,7 @@ MX_TILE_KERNEL(C) void gemm_kernel(GemmArgs p) {
   StridedLoader<C::BM, C::BK, MA> la;
   StridedLoader<C::BN, C::BK, MB> lb;
   Acc<C> acc;
-  tile_product<C>(acc, la, lb, (k1 - k0 + C::BK - 1) / C::BK, smem, [&](auto& a, auto& b) {
+  const float scale = tile_product<C>(acc, la, lb, (k1 - k0 + C::BK - 1) / C::BK, smem, [&](auto& a, auto& b) {
     a.init(p.a + bz * p.a_sb, p.a_sm, p.a_sk, row0, p.M, k0, k1);
     b.init(p.b + bz * p.b_sb, p.b_sn, p.b_sk, col0, p.N, k0, k1);
   });
@@ -67,7 +67,7 @@ MX_TILE_KERNEL(C) void gemm_kernel(GemmArgs p) {
     }
     float* const part = p.ws + ((int64_t(split) * p.batch + bz) * p.M + row0) * p.N + col0;
     store_tile<C>(buffer_rsrc(part, kBufMaxBytes), col, uint32_t(p.N) * 4u, 0, p.M - row0,
-                  [&](int i, int j, int v) { return acc.v[i][j][v]; });
+                  [&](int i, int j, int v) { return acc.v[i][j][v] * scale; });
     return;
   }
   float* __restrict__ cb = p.c + bz * p.c_sb;
@@ -93,7 +93,7 @@ MX_TILE_KERNEL(C) void gemm_kernel(GemmArgs p) {
       const float* __restrict__ brow = bias + int64_t(row) * p.bias_sm;
 #pragma unroll
       for (int j = 0; j < C::FN; ++j)
-        if (ccol[j] < p.N) crow[ccol[j]] = alpha * acc.v[i][j][v] + beta * brow[int64_t(ccol[j]) * p.bias_sn];
+        if (ccol[j] < p.N) crow[ccol[j]] = alpha * (acc.v[i][j][v] * scale) + beta * brow[int64_t(ccol[j]) * p.bias_sn];
     });
     return;
   }
@@ -103,7 +103,7 @@ MX_TILE_KERNEL(C) void gemm_kernel(GemmArgs p) {
 #pragma unroll
     for (int j = 0; j < C::FN; ++j) col[j] = ccol[j] < p.N ? uint32_t(ccol[j] - col0) * 4u : kOffNone;
     store_tile<C>(buffer_rsrc(cb + int64_t(row0) * p.ldc + col0, kBufMaxBytes), col, uint32_t(p.ldc) * 4u, 0,
-                  p.M - row0, [&](int i, int j, int v) { return alpha * acc.v[i][j][v] + bcol[j]; });
+                  p.M - row0, [&](int i, int j, int v) { return alpha * (acc.v[i][j][v] * scale) + bcol[j]; });
     return;
   }
   for_each_acc_row<C>([&](int r, int i, int v) {
@@ -112,7 +112,7 @@ MX_TILE_KERNEL(C) void gemm_kernel(GemmArgs p) {
     float* __restrict__ crow = cb + int64_t(row) * p.ldc;
 #pragma unroll
     for (int j = 0; j < C::FN; ++j)
-      if (ccol[j] < p.N) crow[ccol[j]] = alpha * acc.v[i][j][v] + bcol[j];
+      if (ccol[j] < p.N) crow[ccol[j]] = alpha * (acc.v[i][j][v] * scale) + bcol[j];
   });
 }
 

@@ -6,9 +6,9 @@ Bound: the pieces restore an operand exactly and the dropped products are below
 2^-24 of a term, so what is left is FP32 accumulation, at most one rounding
 (2^-24 relative to the running sum, itself at most the sum of the terms'
 magnitudes) per 16 terms and product -- bounded here by (K / 16 + 8) * 2^-23 of
-the summed magnitudes.  Operands without pieces (infinite, above the largest
-bf16, below 2^-110) take the FP32 product, checked at K * 2^-24 of the
-magnitudes or by their pattern.
+the summed magnitudes.  Operands without pieces (infinite, or from 2^112 up,
+where the factor that puts FP32's denormals on bf16's overflows) take the FP32
+product, checked at K * 2^-24 of the magnitudes or by their pattern.
 """
 from __future__ import annotations
 
@@ -80,20 +80,38 @@ def test_operands_without_pieces(mx, value, m, n, k):
     assert ((got.double() - ref.double()).abs() <= k * 2.0 ** -23 * mag)[fine].all()
 
 
-@pytest.mark.parametrize("exp_a,exp_b", [(-60, 0), (-118, 0), (-118, 10), (-70, -50), (-128, 20)])
-def test_tiny_operands(mx, exp_a, exp_b):
-    """Operands whose pieces lose bits to bf16's smallest denormal (2^-133) get
-    the FP32 product.  (Operands below 2^-134, FP32 denormals themselves, have no
-    nonzero piece and count as zero.)"""
-    a, b, av, bv = operands("nt", 96, 80, 96, 11)
-    a, b = a.double().mul(2.0 ** exp_a).float(), b.mul(2.0 ** exp_b)
+@pytest.mark.parametrize("layout", ["nt", "tn"])
+@pytest.mark.parametrize("exp_a,exp_b", [(-60, 0), (-118, 0), (-118, 10), (-70, -50), (-128, 20),
+                                         (-118, 40), (-118, 60), (-123, 60), (-126, 90), (-128, 60), (-140, 0),
+                                         (-140, 20), (-140, 120), (60, -123), (20, -140),
+                                         (109, -30), (113, -60), (124, -110), (80, 18)])
+def test_operands_at_both_ends(mx, layout, exp_a, exp_b):
+    """Operands below bf16's smallest denormal (2^-133) or with bits there, and
+    those and results that the pieces' factor takes past FP32's largest."""
+    a, b, av, bv = operands(layout, 96, 80, 96, 11)
+    a, b = a.double().mul(2.0 ** exp_a).float(), b.double().mul(2.0 ** exp_b).float()
     av.copy_(a), bv.copy_(b)
     got = gemm(mx, av, bv).cpu().double()
     ref, mag = a.double() @ b.double(), a.double().abs() @ b.double().abs()
     assert ((got - ref).abs() <= 96 * (2.0 ** -23 * mag + 2.0 ** -149)).all()
 
 
-@pytest.mark.parametrize("case", ["inf", "tiny", "normal"])
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+def test_one_tiny_row(mx, monkeypatch, tile):
+    """A row of tiny operands, and tiny values beside ordinary ones, on every
+    tile: the split product takes them all (no K * 2^-24 of FP32 sums)."""
+    monkeypatch.setenv("MX_GEMM_TILE", str(tile))
+    a, b, av, bv = operands("nt", 300, 260, 100, 13)
+    a[37] = (a[37].double() * 2.0 ** -121).float()
+    a[5:9, 3::7] *= 2.0 ** -120
+    b[:, 77] *= 2.0 ** 80
+    av.copy_(a), bv.copy_(b)
+    got = gemm(mx, av, bv).cpu().double()
+    ref, mag = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    assert ((got - ref).abs() <= (100 / 16 + 8) * 2.0 ** -23 * mag + 2.0 ** -140).all()
+
+
+@pytest.mark.parametrize("case", ["inf", "tiny", "tiny times huge", "normal"])
 @pytest.mark.parametrize("geometry", [((2, 20, 9, 11), 24, 3, 1, 1), ((3, 32, 8, 8), 70, 1, 1, 0),
                                       ((2, 3, 21, 17), 33, 7, 2, 3), ((4, 48, 7, 7), 130, 3, 2, 1)])
 def test_conv_phases(mx, case, geometry):
@@ -105,6 +123,8 @@ def test_conv_phases(mx, case, geometry):
     dy = torch.randn(xs[0], co, d.oh, d.ow, generator=g)
     if case == "tiny":
         dy, x = dy.double().mul(2.0 ** -118).float(), x.double().mul(2.0 ** -118).float()
+    if case == "tiny times huge":  # results of ordinary size from operands whose pieces lose bits
+        dy, x, w = (t.double().mul(2.0 ** e).float() for t, e in ((dy, -124), (x, -124), (w, 100)))
     if case == "inf":
         dy[1, 2, 3, 1] = float("inf")
         x[0, 1, 4, 5] = float("inf")
@@ -113,7 +133,8 @@ def test_conv_phases(mx, case, geometry):
     st, algo = torch.cuda.current_stream().cuda_stream, mx.ALGO_IMPLICIT_GEMM
     mx.conv2d_forward(d, xc, wc, None, y, algo, st)
     mx.conv2d_backward_input(d, dyc, wc, dx, algo, st)
-    scale = 2.0 ** 118 if case == "tiny" else 1.0  # dW of two tiny operands underflows in any FP32 sum
+    # dW of two tiny operands underflows in any FP32 sum
+    scale = {"tiny": 2.0 ** 118, "tiny times huge": 2.0 ** 230}.get(case, 1.0)
     dy_w = (dyc.double() * scale).float()
     mx.conv2d_backward_weight(d, xc, dy_w, dw, db, algo, st)
     torch.cuda.synchronize()
