@@ -938,6 +938,66 @@ constexpr int V_FLOATS = 16 * SK * STILES;  // [coordinate][k][tile], one stage
 // outputs' norm, error 5.9e-7 (FP32 MFMA 7.0e-7); it costs 1% of the time.
 __host__ __device__ inline int negated_from(int ns) { return (5 * ns + 2) / 8; }
 
+// The outputs of one workgroup by the definition, on FP32 MFMA: wave w takes
+// the four outputs of each of its eight tiles (32 columns) for the 64 channels,
+// nine taps of two input channels a step.  16 x 256 x 32^2 with every block
+// here: 647 us (a scalar sum per output took 7048; 75 with none here, 99 on the
+// 16-tile kernel).
+__device__ __forceinline__ void direct_block(const fused::Args& p, int g, int o0, int t0, int wave, int lane) {
+  const int r = lane & 31, h = lane >> 5;
+  const int t = t0 + 8 * wave + (r >> 2);
+  const uint32_t tt = t < p.T ? uint32_t(t) : 0u;
+  const uint32_t img = mfma::fdiv(tt, p.f_thw);
+  const uint32_t pos = tt - img * uint32_t(p.TH * p.TW);
+  const uint32_t ty = mfma::fdiv(pos, p.f_tw), tx = pos - ty * uint32_t(p.TW);
+  const int oy = int(2 * ty) + ((r >> 1) & 1), ox = int(2 * tx) + (r & 1);
+  const bool ok = t < p.T && oy < p.OH && ox < p.OW;
+  const uint32_t plane4 = uint32_t(p.H) * uint32_t(p.W) * 4u;
+  const uint32_t x0 = (img * uint32_t(p.Cin) + uint32_t(g * p.C + h)) * plane4;
+  uint32_t xo[9], wo[2];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) {
+    const int iy = oy - p.ph + k / 3, ix = ox - p.pw + k % 3;
+    const bool in = ok && unsigned(iy) < unsigned(p.H) && unsigned(ix) < unsigned(p.W);
+    xo[k] = in ? x0 + (uint32_t(iy) * uint32_t(p.W) + uint32_t(ix)) * 4u : kOffNone;
+  }
+  const uint32_t w_o = p.flip ? 36u : 36u * uint32_t(p.C), w_c = p.flip ? 36u * uint32_t(p.O) : 36u;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int o = o0 + 32 * i + r;
+    wo[i] = o < p.O ? 36u * uint32_t(g) * uint32_t(p.O) * uint32_t(p.C) + uint32_t(o) * w_o + uint32_t(h) * w_c : kOffNone;
+  }
+  const i32x4 rx = mfma::buffer_rsrc(p.x, p.x_bytes), rw = mfma::buffer_rsrc(p.w, p.w_bytes);
+  const i32x4 ry = mfma::buffer_rsrc(p.y, p.y_bytes);
+  mfma::f32x16 sum[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sum[i][v] = 0.f;
+  for (int c = 0; c < p.C; c += 2) {
+    const bool in = c + h < p.C;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      const float xv = mfma::bload(rx, in ? xo[k] : kOffNone, uint32_t(c) * plane4);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const float wv = mfma::bload(rw, in ? wo[i] : kOffNone, uint32_t(c) * w_c + uint32_t(p.flip ? 8 - k : k) * 4u);
+        sum[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(wv, xv, sum[i], 0, 0, 0);
+      }
+    }
+  }
+  const uint32_t y_plane4 = uint32_t(p.OH) * uint32_t(p.OW) * 4u;
+  const uint32_t y0 = (img * uint32_t(p.Cout) + uint32_t(g * p.O)) * y_plane4 + (uint32_t(oy) * uint32_t(p.OW) + uint32_t(ox)) * 4u;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int o = o0 + 32 * i + 8 * (v >> 2) + 4 * h + (v & 3);
+      const float bb = (p.bias && o < p.O) ? p.bias[g * p.O + o] : 0.f;
+      mfma::bstore(sum[i][v] + bb, ry, ok && o < p.O ? y0 + uint32_t(o) * y_plane4 : kOffNone, 0);
+    }
+}
+
 template <bool RAGGED>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void wino_ws_kernel(fused::Args p) {
   __shared__ __attribute__((aligned(16))) float smem[2 * V_FLOATS];
@@ -976,12 +1036,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     px.fix(rx);
     float d[16], z[16];
     px.patch(d);
+    constexpr float S = mfma::kPieceScale;
 #pragma unroll
     for (int cc = 0; cc < 4; ++cc) {
-      z[0 * 4 + cc] = d[0 * 4 + cc] - d[2 * 4 + cc];
-      z[1 * 4 + cc] = d[1 * 4 + cc] + d[2 * 4 + cc];
-      z[2 * 4 + cc] = d[2 * 4 + cc] - d[1 * 4 + cc];
-      z[3 * 4 + cc] = d[1 * 4 + cc] - d[3 * 4 + cc];
+      const float s1 = d[1 * 4 + cc] * S, s2 = d[2 * 4 + cc] * S;
+      z[0 * 4 + cc] = __builtin_fmaf(d[0 * 4 + cc], S, -s2);
+      z[1 * 4 + cc] = s1 + s2;
+      z[2 * 4 + cc] = s2 - s1;
+      z[3 * 4 + cc] = __builtin_fmaf(-d[3 * 4 + cc], S, s1);
     }
     float* const dst = V + (8 * h + kc) * STILES + lane;
     constexpr int T = SK * STILES;  // one coordinate
@@ -1011,8 +1073,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       a[e][i].lo = __builtin_bit_cast(mfma::bf16x8, mfma::bload4(ru, u_lane + i * 512, at + 2 * u_plane));
     }
   };
-  typedef float f32x16 __attribute__((ext_vector_type(16)));
-  f32x16 acc[2][2][2];  // [coordinate][channel block][tile block]
+  mfma::f32x16 acc[2][2][2];  // [coordinate][channel block][tile block]
 #pragma unroll
   for (int e = 0; e < 2; ++e)
 #pragma unroll
@@ -1081,10 +1142,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   negate();
 
-  // Products that the pieces cannot carry (not finite, or nonzero below
-  // 2^-80: see acc_out_of_range) send the whole workgroup to the direct sum.
+  // Sums that are not finite, or whose output transform need not be (nine of
+  // them, times 2^32), send the whole workgroup to the definition: there an
+  // infinity or a value from 2^112 up, which has no pieces, gives what it
+  // should and only where it should.
   {
-    uint32_t top = 0, low = ~0u;
+    uint32_t top = 0;
 #pragma unroll
     for (int e = 0; e < 2; ++e)
 #pragma unroll
@@ -1092,46 +1155,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            const uint32_t mag = __float_as_uint(acc[e][i][j][v]) << 1;
-            top = max(top, mag);
-            low = min(low, mag - 1);
-          }
-    const bool bad = top >= 0xFF000000u || low < (uint32_t(127 - 80) << 24) - 1;
+          for (int v = 0; v < 16; ++v) top = max(top, __float_as_uint(acc[e][i][j][v]) << 1);
     int* const flags = reinterpret_cast<int*>(smem);
-    const bool any = __any(bad);
+    const bool any = __any(top >= uint32_t(127 + 124) << 24);
     if (lane == 0) flags[wave] = any;
     __syncthreads();
     int all = 0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) all |= flags[i];
-    __syncthreads();
     if (all) {
-      const int t = t0 + (tid & 63);
-      if (t >= p.T) return;
-      const uint32_t img = mfma::fdiv(uint32_t(t), p.f_thw);
-      const uint32_t pos = uint32_t(t) - img * uint32_t(p.TH * p.TW);
-      const uint32_t ty = mfma::fdiv(pos, p.f_tw), tx = pos - ty * uint32_t(p.TW);
-      for (int o = o0 + (tid >> 6); o < min(o0 + SO, p.O); o += 8)
-        for (int q = 0; q < 4; ++q) {
-          const int oy = int(2 * ty) + (q >> 1), ox = int(2 * tx) + (q & 1);
-          if (oy >= p.OH || ox >= p.OW) continue;
-          float sum = 0.f;
-          for (int c = 0; c < p.C; ++c) {
-            const float* const xp = p.x + (int64_t(img) * p.Cin + int64_t(g) * p.C + c) * p.H * p.W;
-            const float* const wk = p.flip ? p.w + ((int64_t(g) * p.C + c) * p.O + o) * 9
-                                           : p.w + ((int64_t(g) * p.O + o) * p.C + c) * 9;
-            for (int k = 0; k < 9; ++k) {
-              const int iy = oy - p.ph + k / 3, ix = ox - p.pw + k % 3;
-              if (unsigned(iy) < unsigned(p.H) && unsigned(ix) < unsigned(p.W))
-                sum += xp[iy * p.W + ix] * wk[p.flip ? 8 - k : k];
-            }
-          }
-          p.y[((int64_t(img) * p.Cout + int64_t(g) * p.O + o) * p.OH + oy) * p.OW + ox] =
-              sum + (p.bias ? p.bias[g * p.O + o] : 0.f);
-        }
+      direct_block(p, g, o0, t0, wave, lane);
       return;
     }
+    __syncthreads();
   }
 
   // Output transform, 32 channels at a time: [coordinate][channel][tile] in
@@ -1174,8 +1210,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const bool ok = o < p.O && tok;
       const float bb = (p.bias && o < p.O) ? p.bias[g * p.O + o] : 0.f;
       const uint32_t off = y_tile + uint32_t(o) * plane4;
-      const float y00 = r0[0] + r0[1] + r0[2] + bb, y01 = r0[1] - r0[2] - r0[3] + bb;
-      const float y10 = r1[0] + r1[1] + r1[2] + bb, y11 = r1[1] - r1[2] - r1[3] + bb;
+      constexpr float S = mfma::kProductScale;
+      const float y00 = (r0[0] + r0[1] + r0[2]) * S + bb, y01 = (r0[1] - r0[2] - r0[3]) * S + bb;
+      const float y10 = (r1[0] + r1[1] + r1[2]) * S + bb, y11 = (r1[1] - r1[2] - r1[3]) * S + bb;
       if (pairs) {
         mfma::bstore2(f32x2{y00, y01}, ry, ok ? off : kOffNone, 0);
         mfma::bstore2(f32x2{y10, y11}, ry, (ok && below) ? off + row4 : kOffNone, 0);
@@ -1204,10 +1241,10 @@ __global__ __launch_bounds__(256) void split_filter_kernel(const float* __restri
   float u[16];
   fused::filter_transform(w, C, O, g, ob + ol, cg * 8 + cl, flip, u);
   const int ns = Cpad / SK, slab = cg >> 1, half = cg & 1;
-  const float sign = slab >= negated_from(ns) ? -1.f : 1.f;
+  const float scale = slab >= negated_from(ns) ? -mfma::kPieceScale : mfma::kPieceScale;
 #pragma unroll
   for (int t = 0; t < 16; t += 2) {
-    const mfma::Pieces2 s = mfma::split2(sign * u[t], sign * u[t + 1]);
+    const mfma::Pieces2 s = mfma::split2(scale * u[t], scale * u[t + 1]);
     const uint32_t piece[3] = {s.hi, s.mid, s.lo};
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
@@ -2053,6 +2090,7 @@ int winograd_run(const mx_conv2d_desc& d, const float* x, const float* w, const 
     MX_TRY(U.alloc(size_t(p.u_bytes), s));
     p.U = U.as<float>();
     p.w = w;
+    p.w_bytes = int64_t(d.cout) * p.C * 9 * 4;
     p.flip = flip ? 1 : 0;
     p.y_even = (reinterpret_cast<uintptr_t>(y) & 7) == 0;
     const dim3 fgrid(unsigned(p.Opad / 32), unsigned(p.Cpad / 8), unsigned(r.G));

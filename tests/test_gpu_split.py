@@ -296,6 +296,48 @@ def test_winograd_split_kernel_infinite_and_tiny(mx, monkeypatch):
     assert ((run(tiny).double() - ref).abs() <= 180 * (2.0 ** -24 * mag + 2.0 ** -149)).all()
 
 
+@pytest.mark.parametrize("n,c,h,wd,o,pad,groups", [
+    (1, 16, 16, 16, 64, (1, 1), 1), (3, 31, 9, 7, 40, (0, 2), 1), (1, 17, 34, 31, 129, (1, 1), 1),
+    (2, 24, 12, 12, 70, (2, 0), 3)])
+@pytest.mark.parametrize("flip", [False, True])
+@pytest.mark.parametrize("case", ["huge weight", "tiny times huge"])
+def test_winograd_split_kernel_range(mx, monkeypatch, n, c, h, wd, o, pad, groups, flip, case):
+    """A weight of 2^113, which has no pieces, in one output channel of every 64:
+    each block takes the definition (9 C roundings of its magnitudes).  Tiny
+    operands times huge ones keep the split product and its bound."""
+    for k, val in (("FUSED", "1"), ("T16", "0"), ("FILTER", "0")):
+        monkeypatch.setenv(f"MX_WINOGRAD_{k}", val)
+    g = torch.Generator().manual_seed(n + c + h + o)
+    ci, co = (o, c) if flip else (c, o)  # flip: the input gradient of a layer o -> c
+    pad_l = (2 - pad[0], 2 - pad[1]) if flip else pad
+    oh, ow = h + 2 * pad[0] - 2, wd + 2 * pad[1] - 2
+    d = mx.conv_desc((n, ci * groups, *((oh, ow) if flip else (h, wd))), (co * groups, ci, 3, 3), (1, 1), pad_l, (1, 1),
+                     groups)
+    x, w = torch.randn(n, c * groups, h, wd, generator=g), torch.randn(co * groups, ci, 3, 3, generator=g)
+    if case == "huge weight":
+        (w[::c, ::64, 1, 1] if flip else w.view(groups, o, c, 3, 3)[:, ::64, 0, 1, 1])[:] = 2.0 ** 113
+        # (flip: output channels are w's second axis, ::c is each group's first filter)
+    else:
+        x, w = (t.double().mul(2.0 ** e).float() for t, e in ((x, -126), (w, 104)))
+    out = torch.full((n, o * groups, oh, ow), float("nan"), device="cuda")
+    xd, wdv, st = x.cuda(), w.cuda(), torch.cuda.current_stream().cuda_stream
+    torch.cuda.synchronize()
+    if flip:
+        mx.conv2d_backward_input(d, xd, wdv, out, mx.ALGO_WINOGRAD, st)
+    else:
+        mx.conv2d_forward(d, xd, wdv, None, out, mx.ALGO_WINOGRAD, st)
+    torch.cuda.synchronize()
+    wt = w.view(groups, c, o, 3, 3).flip(3, 4).transpose(1, 2).reshape(groups * o, c, 3, 3) if flip else w
+    ref = F.conv2d(x.double(), wt.double(), padding=pad, groups=groups)
+    if case == "huge weight":
+        bound = 9 * c * 2.0 ** -24 * F.conv2d(x.double().abs(), wt.double().abs(), padding=pad, groups=groups)
+    else:
+        mag = torch.cat([winograd_magnitude(xs, ws, pad, oh, ow)
+                         for xs, ws in zip(x.chunk(groups, 1), wt.chunk(groups, 0))], 1)
+        bound = (c / 16 + 16) * 2.0 ** -23 * mag
+    assert ((out.cpu().double() - ref).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("n,c,h,wd,o,k,stride,dil,groups,shift", [
     (1, 16, 32, 32, 64, 3, 1, 1, 1, 0),    # 1024 positions: the plain order's last
     (1, 16, 25, 41, 64, 3, 1, 1, 1, 0),    # 1025: the blocked order's first
