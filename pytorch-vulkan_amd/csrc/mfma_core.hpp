@@ -231,9 +231,10 @@ struct SplitStage {
   static constexpr int PLANE = ROWS * BK;  // bf16 elements of one plane
   static constexpr int FLOATS = 3 * PLANE / 2;
   float* p;
+  float scale = kPieceScale;  // negative: the slab is summed negated
   __device__ __forceinline__ uint16_t* at(int elem) const { return reinterpret_cast<uint16_t*>(p) + elem; }
   __device__ __forceinline__ void put4(int elem, f32x4 v) const {
-    v *= kPieceScale;
+    v *= scale;
     const Pieces2 a = split2(v[0], v[1]), b = split2(v[2], v[3]);
     *reinterpret_cast<u32x2*>(at(elem)) = u32x2{a.hi, b.hi};
     *reinterpret_cast<u32x2*>(at(elem + PLANE)) = u32x2{a.mid, b.mid};
@@ -253,7 +254,7 @@ struct SplitStage {
         u32x4 w[3];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const Pieces2 s = split2(v[e + 2 * q] * kPieceScale, v[e + 2 * q + 1] * kPieceScale);
+          const Pieces2 s = split2(v[e + 2 * q] * scale, v[e + 2 * q + 1] * scale);
           w[0][q] = s.hi, w[1][q] = s.mid, w[2][q] = s.lo;
         }
         const int elem = row_elem(row, k + e);
@@ -276,7 +277,7 @@ struct SplitStage {
       const float mine = odd ? v[q + 1] : v[q], give = odd ? v[q] : v[q + 1];
       const float got = __builtin_bit_cast(
           float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, give), 0xB1, 0xF, 0xF, true));  // lane ^ 1
-      const Pieces2 s = split2((odd ? got : mine) * kPieceScale, (odd ? mine : got) * kPieceScale);
+      const Pieces2 s = split2((odd ? got : mine) * scale, (odd ? mine : got) * scale);
       const int elem = row_elem(row0 + (q + (odd ? 1 : 0)) * step, k & ~1);
       *reinterpret_cast<uint32_t*>(at(elem)) = s.hi;
       *reinterpret_cast<uint32_t*>(at(elem + PLANE)) = s.mid;
@@ -420,12 +421,15 @@ __device__ __forceinline__ void mainloop_f32(Acc<C>& acc, LA& la, LB& lb, int nk
 // 6 x 32 cycles; eight v_mfma_f32_32x32x2f32 take 8 x 64.  The error is
 // smaller as well, since 16 products enter one rounding: relative 2-norm
 // against float64 on normal operands, K = 64 / 4096: 1.1e-7 / 0.98e-6 in one
-// accumulator, 0.5e-7 / 0.41e-6 with the five small products in their own,
-// 1.4e-7 / 1.17e-6 on the FP32 instruction.  The bf16 instruction rounds
-// towards minus infinity below the accumulator's last bit, a bias of 1.1e-7 of
-// the result at K = 1568 that the partial sums of a K split would add up;
-// with the small products apart it is 0.07e-7.  So tiles with the registers
-// for it (DUAL) keep two accumulators.
+// accumulator, 0.5e-7 / 0.40e-6 with the five small products in their own,
+// 1.4e-7 / 1.15e-6 on the FP32 instruction.  The bf16 instruction rounds
+// towards minus infinity below the accumulator's last bit.  Tiles with the
+// registers for it (DUAL) keep the small products, which lie there, in their
+// own accumulator: no bias.  In one accumulator it is -2.1e-7 of the result at
+// K = 4096 and -8.4e-6 at 2^18, and the partial sums of a K split add it up
+// (-6.4e-7 of a dW over 16 splits); there the middle half of the slabs is
+// summed negated (mainloop_split): 0.1e-7, 3.8e-7 and 0.4e-7, and the error
+// against float64 at K = 2^18 goes from 1.1e-5 to 0.64e-5 (FP32: 0.92e-5).
 template <class C, bool KMA, bool KMB>
 __device__ __forceinline__ void mma_slab_split(Acc<C>& acc, Acc<C>& small, const float* As, const float* Bs, int wm,
                                                int wn, int lane) {
@@ -515,10 +519,10 @@ __device__ __forceinline__ void mainloop_split(Acc<C>& acc, LA& la, LB& lb, int 
   Acc<C> small;
   if constexpr (C::DUAL) acc_zero<C>(small);
   // Slab in stage `cur`; `na` / `nb` hold the next one and take the one `ahead`.
-  const auto slab = [&](int cur, LA& na, LB& nb) {
+  const auto slab = [&](int cur, LA& na, LB& nb, float scale = kPieceScale) {
     mma_slab_split<C, LA::KMAJOR, LB::KMAJOR>(acc, small, As + cur * C::A_SPLIT, Bs + cur * C::B_SPLIT, wm, wn, lane);
-    na.store(SplitStage<C::BM, C::BK>{As + (cur ^ 1) * C::A_SPLIT});
-    nb.store(SplitStage<C::BN, C::BK>{Bs + (cur ^ 1) * C::B_SPLIT});
+    na.store(SplitStage<C::BM, C::BK>{As + (cur ^ 1) * C::A_SPLIT, C::BM < C::BN ? scale : kPieceScale});
+    nb.store(SplitStage<C::BN, C::BK>{Bs + (cur ^ 1) * C::B_SPLIT, C::BM < C::BN ? kPieceScale : scale});
     if constexpr (C::KH == 8) split_schedule<C, LA::KMAJOR, LB::KMAJOR>();
     na.load();
     nb.load();
@@ -557,7 +561,26 @@ __device__ __forceinline__ void mainloop_split(Acc<C>& acc, LA& la, LB& lb, int 
     la.load();
     lb.load();
     __syncthreads();
-    for (int t = 0; t < nk; ++t) slab(t & 1, la, lb);
+    if constexpr (C::DUAL) {
+      for (int t = 0; t < nk; ++t) slab(t & 1, la, lb);
+    } else {
+      // Slabs [from, to) enter one operand negated and the accumulators change
+      // sign at both ends, so the rounding bias of these slabs meets that of
+      // the others.  A slab's bias goes as the sum's last place: as the square
+      // root of the slabs so far for operands of both signs (5% of the bias is
+      // left), as their number for operands of one (none).  Below 16 slabs it
+      // is 1e-8 of the result.
+      const int from = nk >= 16 ? nk / 4 : -1, to = nk - from;
+      for (int t = 0; t < nk; ++t) {
+        if (t == from || (t == to && from >= 0)) {
+#pragma unroll
+          for (int i = 0; i < C::FM; ++i)
+#pragma unroll
+            for (int j = 0; j < C::FN; ++j) acc.v[i][j] = -acc.v[i][j];
+        }
+        slab(t & 1, la, lb, t + 1 >= from && t + 1 < to && from >= 0 ? -kPieceScale : kPieceScale);
+      }
+    }
   }
   if constexpr (C::DUAL) {
 #pragma unroll

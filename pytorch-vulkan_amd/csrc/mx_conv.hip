@@ -1219,9 +1219,6 @@ std::string dx_variant(const DxPlan& f) {
     // Phases sharing a loader run as one conv_dx_phases_kernel launch.
     int same = 0;
     for (size_t j = 0; j < f.phases.size(); ++j) same += f.phases[j].K != 0 && f.bmodes[j] == f.bmodes[i];
-    // (256-row tiles of scalar weight rows and plain gathers: one launch each.)
-    if (f.gp.tile == conv::TALL && !f.vec_a && f.bmodes[i] == conv::B_GATHER && !conv::blocked_channels(q.Cout_g))
-      same = 1;
     const char* b = f.bmodes[i] == conv::B_VEC ? "PosQuad"
                     : conv::blocked_channels(q.Cout_g) ? "PhaseGather<blocked>" : "PhaseGather";
     std::string n = cat(same > 1 ? "conv_dx_phases_kernel<" : "conv_dx_kernel<", tile_name(f.gp.tile, MX_CONV_DINPUT),

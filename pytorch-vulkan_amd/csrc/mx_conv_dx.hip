@@ -174,11 +174,6 @@ int launch_a(const ConvArgs& p, Mode ma, int bmode, hipStream_t s) {
   return launch_b<C, Mode::RSCALAR>(p, bmode, s);
 }
 
-// Not built, for its registers: the phases' shared launch of 256-row tiles that
-// read both scalar weight rows and gathers in the plain order.
-template <class C, Mode MA>
-constexpr bool dx_phases_built = !(C::BM == 256 && MA == Mode::RSCALAR);
-
 template <class C, Mode MA>
 int launch_set_b(DxPhaseSet set, int bmode, hipStream_t s) {
   int most = 0;
@@ -195,11 +190,9 @@ int launch_set_b(DxPhaseSet set, int bmode, hipStream_t s) {
   else if (blocked_channels(set.q[0].Cout_g))
     hipLaunchKernelGGL((conv_dx_phases_kernel<C, MA, PhaseGatherLoader<C::BN, C::BK, true>>), grid, dim3(kThreads), 0,
                        s, set);
-  else if constexpr (dx_phases_built<C, MA>)
+  else
     hipLaunchKernelGGL((conv_dx_phases_kernel<C, MA, PhaseGatherLoader<C::BN, C::BK, false>>), grid, dim3(kThreads),
                        0, s, set);
-  else
-    for (int i = 0; i < set.n; ++i) MX_TRY((launch_b<C, MA>(set.q[i], bmode, s)));
   MX_HIP(hipGetLastError());
   return MX_OK;
 }

@@ -61,6 +61,48 @@ def test_split_product_is_more_exact_than_fp32_sums(mx):
     assert ((got - ref).norm() / ref.norm()).item() < 2.0 ** -24 * (4096 / 6) ** 0.5
 
 
+@pytest.mark.parametrize("signs", ["both", "one"])
+@pytest.mark.parametrize("tile,m,n,layout", [(0, 256, 256, "nt"), (1, 256, 256, "nn"), (2, 255, 253, "tn")])
+def test_one_accumulator_is_unbiased(mx, monkeypatch, tile, m, n, layout, signs):
+    """Tiles without a second accumulator set, over a long K: the bf16
+    instruction's rounding towards minus infinity leaves a mean error below a
+    tenth of FP32 sums' random one (2^-24 sqrt(K / 6) of the result)."""
+    monkeypatch.setenv("MX_GEMM_TILE", str(tile))
+    k = 32768
+    a, b, av, bv = operands(layout, m, n, k, 17)
+    if signs == "one":
+        av.abs_(), bv.abs_()
+    got, ref = gemm(mx, av, bv).double(), av.double() @ bv.double()
+    error, rms = got - ref, ref.pow(2).mean().sqrt()
+    assert abs((error.mean() / rms).item()) <= 0.1 * 2.0 ** -24 * (k / 6) ** 0.5
+    assert (error.pow(2).mean().sqrt() / rms).item() <= 2.0 ** -24 * (k / 6) ** 0.5
+
+
+@pytest.mark.parametrize("tile,geometry,shift", [  # x shape, output channels, kernel, padding
+    (2, ((4, 16, 111, 111), 128, 3, 1), 0), (4, ((4, 16, 111, 111), 256, 3, 1), 0),  # scalar dy rows, x gather
+    (3, ((16, 256, 56, 56), 64, 1, 0), 1),                                          # scalar dy rows, x in place
+    (0, ((16, 128, 56, 56), 256, 1, 0), 0), (1, ((16, 256, 56, 56), 128, 1, 0), 0)])
+def test_one_accumulator_weight_gradient_is_unbiased(mx, monkeypatch, tile, geometry, shift):
+    """The same for weight gradients: 16 partial sums over 3100 positions each
+    add up their bias, not their random errors."""
+    monkeypatch.setenv("MX_CONV_PLAN", f"{tile},16")
+    xs, co, k, p = geometry
+    g = torch.Generator(device="cuda").manual_seed(tile)
+    x = torch.randn(xs, device="cuda", generator=g)
+    d = mx.conv_desc(xs, (co, xs[1], k, k), (1, 1), (p, p))
+    store = torch.randn(xs[0] * co * d.oh * d.ow + 4, device="cuda", generator=g)
+    dy = store[shift:shift + xs[0] * co * d.oh * d.ow].view(xs[0], co, d.oh, d.ow)
+    dw = torch.empty(co, xs[1], k, k, device="cuda")
+    torch.cuda.synchronize()
+    mx.conv2d_backward_weight(d, x, dy, dw, None, mx.ALGO_IMPLICIT_GEMM, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    ref = sum(dy[i].double().reshape(co, -1) @ F.unfold(x[i:i + 1].double(), k, padding=p)[0].t().contiguous()
+              for i in range(xs[0])).view_as(dw)
+    error, rms, span = dw.double() - ref, ref.pow(2).mean().sqrt(), xs[0] * d.oh * d.ow / 16
+    assert abs((error.mean() / rms).item()) <= 0.1 * 2.0 ** -24 * (span / 6) ** 0.5
+    assert (error.pow(2).mean().sqrt() / rms).item() <= 2.0 ** -24 * (span / 6) ** 0.5
+
+
 @pytest.mark.parametrize("value", [float("inf"), -float("inf"), float("nan"), 3.4028234e38, -3.4e38])
 @pytest.mark.parametrize("m,n,k", [(70, 50, 40), (300, 300, 64)])
 def test_operands_without_pieces(mx, value, m, n, k):
