@@ -21,13 +21,18 @@
 
 namespace mx {
 
-static thread_local std::string g_last_error;
+// Plain storage: a thread's objects with destructors are gone by the time
+// static destructors run, and those still free memory here (the host storages
+// of copies in flight), each call clearing the message first.
+static thread_local char g_last_error[2048];
 
 int set_error(int code, const std::string& msg) {
-  g_last_error = msg;
+  const size_t n = std::min(msg.size(), sizeof g_last_error - 1);
+  std::memcpy(g_last_error, msg.data(), n);
+  g_last_error[n] = 0;
   return code;
 }
-void clear_error() { g_last_error.clear(); }
+void clear_error() { g_last_error[0] = 0; }
 
 static constexpr int kMaxDevices = 64;
 
@@ -160,7 +165,7 @@ using namespace mx;
 
 extern "C" {
 
-const char* mx_last_error(void) { return g_last_error.c_str(); }
+const char* mx_last_error(void) { return g_last_error; }
 int mx_abi_version(void) { return 3; }
 
 int mx_init(int ordinal) {

@@ -340,3 +340,40 @@ def test_implicit_gemm_group_limit(mx):
             mx.conv2d_select(many, phase, mx.ALGO_IMPLICIT_GEMM)
     fine = mx.conv_desc((1, 40000, 4, 4), (20000, 2, 3, 3), (2, 2), (1, 1), (1, 1), 20000)
     assert mx.conv2d_select(fine, mx.MX_CONV_DINPUT, mx.ALGO_IMPLICIT_GEMM) == mx.ALGO_IMPLICIT_GEMM
+
+
+def test_calls_while_the_process_ends_leave_the_heap_alone(tmp_path):
+    """Static destructors free memory through the library after the thread's own
+    objects are gone: a call there, with an earlier error message, must not
+    write to freed memory (seen as an abort at exit)."""
+    import subprocess
+    import torch
+    src, exe = tmp_path / "late.cpp", tmp_path / "late"
+    src.write_text(r"""
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include "mx.h"
+static size_t n = 0;
+static void late() {
+  static char* block[256];  // one of them takes the place of whatever n bytes were freed
+  for (size_t i = 0; i < 256; ++i) std::memset(block[i] = static_cast<char*>(std::malloc(n + i)), 'x', n + i);
+  mx_free(nullptr);
+  for (size_t i = 0; i < 256; ++i)
+    for (size_t k = 0; k < n + i; ++k)
+      if (block[i][k] != 'x') std::_Exit(1);
+  std::puts("unharmed");
+}
+int main() {
+  std::atexit(late);  // after the thread-local destructors
+  mx_memcpy_async(nullptr, nullptr, 4, 99, nullptr);
+  n = std::strlen(mx_last_error()) + 1;
+  return n > 40 ? 0 : 2;
+}
+""")
+    lib = os.path.join(REPO, "pytorch-vulkan_amd", "torch_vulkan")
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    subprocess.run(["g++", f"-I{REPO}/include", str(src), "-o", str(exe), f"{lib}/libmx.so", f"-Wl,-rpath,{lib}",
+                    f"-Wl,-rpath,{torch_lib}", "-Wl,--allow-shlib-undefined"], check=True)
+    run = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert run.returncode == 0 and run.stdout.strip() == "unharmed", (run.returncode, run.stdout, run.stderr)
