@@ -256,10 +256,6 @@ constexpr TileChoice kTiles[] = {{256, 128, 2, 1.81}, {128, 256, 2, 1.75}, {128,
 constexpr int64_t kMaxSplitBytes = int64_t(64) << 20;  // partial products of one call
 constexpr int kSplitBK = 32;                           // K granularity of a split
 constexpr int kMinSplitSpan = 64;                      // shortest K range worth a split
-// Longest K that is split.  No layer comes near it (a weight gradient's K is
-// its batch's positions), and the stream tests take a product of K = 2^19 as
-// work that keeps one workgroup busy for milliseconds.
-constexpr int64_t kMaxSplitK = int64_t(1) << 18;
 
 // Estimated time: a CU holding n tiles runs at rate * occ(n), occ rising from
 // 0.71 with one resident tile to 1 with per_cu; a tile's first loads and its
@@ -384,7 +380,7 @@ int plan_gemm(const mx_gemm_desc* d, const float* a, const float* b, const float
   g->ma = pick_mode(p.a, p.a_sm, p.a_sk, p.a_sb, p.batch, p.M, p.K);
   g->mb = pick_mode(p.b, p.b_sn, p.b_sk, p.b_sb, p.batch, p.N, p.K);
   pick_gemm_tile(d->m, d->n, d->k, d->batch, is_vec(g->ma) && is_vec(g->mb), d->kernel,
-                 split_ok && d->k <= kMaxSplitK && d->n <= kVecStrideMax && d->m * d->n <= INT32_MAX, &g->tile,
+                 split_ok && d->n <= kVecStrideMax && d->m * d->n <= INT32_MAX, &g->tile,
                  &p.splits, &p.kps);
   return MX_OK;
 }

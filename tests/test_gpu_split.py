@@ -204,7 +204,7 @@ def test_conv_phases(mx, case, geometry):
 
 @pytest.mark.parametrize("bias_kind", ["none", "col", "matrix"])
 @pytest.mark.parametrize("m,n,k,batch", [(8, 1000, 2048, None), (1, 37, 1111, None), (65, 130, 4096, None),
-                                         (33, 64, 1500, 3)])
+                                         (33, 64, 1500, 3), (40, 24, (1 << 19) + 6, None)])
 def test_gemm_k_split(mx, m, n, k, batch, bias_kind):
     """Few tiles over a long K: partial products of K ranges, summed with alpha,
     beta and the bias in a second launch."""

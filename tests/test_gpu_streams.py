@@ -17,9 +17,10 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# One 64x64 output tile with a long K: a single workgroup for several
-# milliseconds, so two of them on two streams can only finish early together
-# if the streams really run at the same time.
+# One 64x64 output tile with a long K, in one pass over K (MX_GEMM_TILE=3, the
+# 64x64 tile without K split): a single workgroup for several milliseconds, so
+# two of them on two streams can only finish early together if the streams
+# really run at the same time.
 LONG_K = 1 << 19
 
 
@@ -35,7 +36,9 @@ def long_operands(vk):
     g = torch.Generator().manual_seed(5)
     a = torch.randn(64, LONG_K, generator=g) / 256
     b = torch.randn(LONG_K, 64, generator=g) / 256
-    return a, b, a.to("vulkan"), b.to("vulkan")
+    with pytest.MonkeyPatch.context() as env:
+        env.setenv("MX_GEMM_TILE", "3")
+        yield a, b, a.to("vulkan"), b.to("vulkan")
 
 
 def test_reference_stream_context_events_and_lifetimes(vk):
