@@ -1928,11 +1928,24 @@ double t16_cost(const RunPlan& r, int parts, int slabs) {
   return rounds * (3.0 + 1.25 * slabs);
 }
 
+// The passes in place of a split walk, in us on MI355X, as fitted to 27 layers
+// (within 13%): launches and issue, U, V and M written and read at 5.6 TB/s, the
+// batched GEMM at 222 TFLOP/s.
+double unfused_cost(const RunPlan& r, int64_t images, int64_t passes) {
+  const double c = r.p.C, o = r.p.O, t = double(images) * r.p.TH * r.p.TW, g = r.G;
+  return 5.0 + 18.0 * double(passes) + 64.0 * 2.0 * g * (c * o + c * t + o * t) / 5.6e6 + 32.0 * g * c * o * t / 2.22e8;
+}
+
 // Splits the 16-tile kernel's channel walk where a few workgroups walk long
 // (kMinPart slabs a part and up), the parts' outputs summed by a second launch
-// (6 us with what it costs the host, and their bytes at 3.6 TB/s).
+// (6 us with what it costs the host, and their bytes at 3.6 TB/s).  Returns the
+// cost of what it set, 0 for one part: the rounds and sums above weigh 0.56 in a
+// fit to 32 layers (within 16%), whose other terms are the same for any number
+// of parts: launches, the filter transform (U' written at 2.9 TB/s) and U' read
+// by every block of 16 tiles, from the L2s (23 TB/s) or, past 24 MB, mostly
+// from behind them (15).
 constexpr int kMinPart = 8;
-void split_walk(RunPlan* r, int64_t out_elems, int64_t ws_limit) {
+double split_walk(RunPlan* r, int64_t out_elems, int64_t ws_limit) {
   fused::Args& p = r->p;
   double best = t16_cost(*r, 1, p.nslab);
   for (int want = 2; want <= 8; ++want) {
@@ -1946,6 +1959,9 @@ void split_walk(RunPlan* r, int64_t out_elems, int64_t ws_limit) {
       p.part_stride = out_elems;
     }
   }
+  if (r->parts == 1) return 0.0;
+  const double u = double(p.u_bytes), blocks = double((int64_t(p.T) + ws::BT16 - 1) / ws::BT16);
+  return 9.5 + 0.56 * (best - 6.0) + u / 2.9e6 + blocks * u / (u > 24e6 ? 15e6 : 23e6);
 }
 
 // The cheaper of the 16-tile and the split kernel, in us on MI355X: rounds of
@@ -2008,21 +2024,26 @@ int plan_run(const mx_conv2d_desc& d, int64_t ws_limit, bool dinput, RunPlan* r)
   bool forced = false;
   if (const char* e = std::getenv("MX_WINOGRAD_FUSED"))
     if (e[0] == '0' || e[0] == '1') r->fused = e[0] == '1', forced = true;
-  if (!r->fused && !forced) {
-    // In place of the unfused passes, whose four launches move V and M through
-    // memory.  Measured, unfused / split walk: 256 channels 32^2 28.9 / 20.5 us,
-    // 8 x 16^2 31.6 / 25.5; 512 -> 256 32^2 34.7 / 27.8; 384 -> 128 64^2 39.8 /
-    // 30.3; 512 channels 16 x 8^2 41.5 / 39.4, 8 x 14^2 61.3 / 57.1; 320
-    // channels 2 x 16^2 30.7 / 21.8; 1024 -> 512 24^2 56.3 / 60.3.
-    split_walk(r, d.n * int64_t(p.Cout) * p.OH * p.OW, ws_limit);
-    if (r->parts > 1) r->fused = true;
-  }
   const int64_t u_plain = 16 * int64_t(p.Cout) * p.C * 4;
   const int64_t per_image = 16 * (int64_t(p.Cin) + p.Cout) * p.TH * p.TW * 4;
   const int64_t fit = ws_limit > u_plain ? (ws_limit - u_plain) / per_image : 0;
+  const int64_t passes = fit > 0 ? (d.n + fit - 1) / fit : 0;
+  if (!r->fused && !forced) {
+    // In place of the unfused passes where those cost more or do not fit.
+    // Measured, unfused / split walk: 256 channels 32^2 29.2 / 20.4 us, 8 x 16^2
+    // 32.5 / 26.5; 512 -> 256 32^2 35.4 / 26.9; 384 -> 128 64^2 40.6 / 30.9; 512
+    // channels 16 x 8^2 42.2 / 39.2, 2 x 24^2 49.5 / 46.4, 8 x 14^2 55.8 / 57.5;
+    // 1024 -> 512 16^2 41.1 / 37.5, 24^2 56.1 / 60.1, 8 x 7^2 50.8 / 56.3; 1536
+    // -> 384 28^2 69.2 / 75.9; 768 channels 2 x 14^2 57.3 / 60.4; 4096 -> 128
+    // 14^2 49.1 / 69.7.
+    const double walk = split_walk(r, d.n * int64_t(p.Cout) * p.OH * p.OW, ws_limit);
+    if (r->parts > 1) {
+      r->fused = passes == 0 || walk < unfused_cost(*r, d.n, passes);
+      if (!r->fused) r->parts = 1, p.part_slabs = p.nslab, p.part_stride = 0;
+    }
+  }
   if (!r->fused && fit < 1) r->fused = true;
   if (!r->fused) {
-    const int64_t passes = (d.n + fit - 1) / fit;
     r->chunk = (d.n + passes - 1) / passes;
     r->unfused_bytes = u_plain + per_image * r->chunk;
   }
@@ -2039,7 +2060,7 @@ int plan_run(const mx_conv2d_desc& d, int64_t ws_limit, bool dinput, RunPlan* r)
   r->filt = r->filt && r->fused;
   r->t16 = r->parts > 1 || prefer_t16(*r, dinput);
   if (const char* e = std::getenv("MX_WINOGRAD_T16"))
-    if (e[0] == '0' || e[0] == '1') r->t16 = e[0] == '1', forced = true;
+    if (e[0] == '0' || e[0] == '1') r->t16 = e[0] == '1';
   // The split filter takes half as much again; past the buffer bound the
   // 16-tile kernel runs.
   if (!r->filt && split_filter_bytes(*r) >= mfma::kBufMaxBytes) r->t16 = true;

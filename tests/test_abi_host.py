@@ -342,6 +342,22 @@ def test_implicit_gemm_group_limit(mx):
     assert mx.conv2d_select(fine, mx.MX_CONV_DINPUT, mx.ALGO_IMPLICIT_GEMM) == mx.ALGO_IMPLICIT_GEMM
 
 
+def test_winograd_split_walk_against_the_passes_it_replaces(mx):
+    """Few workgroups on a long channel walk: the split walk where it measured
+    faster than the unfused passes on MI355X, those where they did (us), and the
+    split walk where they do not fit the workspace."""
+    for n, c, hw, o, unfused, walk in [(1, 256, 32, 256, 29.2, 20.4), (16, 512, 8, 512, 42.2, 39.2),
+                                       (1, 1024, 16, 512, 41.1, 37.5), (1, 640, 64, 64, 44.5, 28.5),
+                                       (1, 1024, 24, 512, 56.1, 60.1), (8, 1024, 7, 512, 50.8, 56.3),
+                                       (1, 1536, 28, 384, 69.2, 75.9), (2, 768, 14, 768, 57.3, 60.4),
+                                       (1, 4096, 14, 128, 49.1, 69.7), (8, 512, 14, 512, 55.8, 57.5),
+                                       (1, 2048, 16, 512, None, 66.8)]:
+        d = mx.conv_desc((n, c, hw, hw), (o, c, 3, 3), (1, 1), (1, 1))
+        plan = mx.conv2d_plan(d, mx.MX_CONV_FORWARD, mx.ALGO_WINOGRAD)
+        faster = "wino_ws16_kernel" if unfused is None or walk < unfused else "wino_unfused"
+        assert plan["variant"].startswith(faster), (n, c, hw, o, plan["variant"])
+
+
 def test_calls_while_the_process_ends_leave_the_heap_alone(tmp_path):
     """Static destructors free memory through the library after the thread's own
     objects are gone: a call there, with an earlier error message, must not
