@@ -19,6 +19,7 @@
 #include <mutex>
 #include <numeric>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "mx_conv_common.hpp"
@@ -225,14 +226,15 @@ __global__ __launch_bounds__(256) void conv_depthwise_staged_kernel(DepthwiseArg
 
 // Input gradient: dx[ih][iw] = sum over output channel j of the channel and
 // taps of w * dy[(ih + ph - kh dh) / sh][...] where the division is exact, in
-// (j, kh, kw) order.  The patches hold dy of the m output channels.  UNIT:
-// stride 1.
+// (j, kh, kw) order.  The patches hold dy of the m output channels, zeros where
+// they leave a plane; a tap that reads there adds nothing, which a weight that
+// is not finite has to be kept from (EDGES, a workgroup with such a weight).
+// UNIT: stride 1.
 template <int K, bool UNIT>
 __global__ __launch_bounds__(256) void conv_depthwise_dx_kernel(DepthwiseArgs a) {
   extern __shared__ float patch[];
   const ConvArgs& p = a.p;
   const int KH = K ? K : p.KH, KW = K ? K : p.KW, m = p.Cout_g;
-  constexpr int U = K ? K : 1;
   for (int64_t t = blockIdx.x; t < a.tiles; t += gridDim.x) {
     const int tw = int(t % a.tiles_w), th = int((t / a.tiles_w) % a.tiles_h);
     const int plane0 = int(t / (int64_t(a.tiles_w) * a.tiles_h)) * a.planes;
@@ -244,8 +246,14 @@ __global__ __launch_bounds__(256) void conv_depthwise_dx_kernel(DepthwiseArgs a)
     const int ow0 = UNIT ? left : left >= 0 ? left / p.sw : -((p.sw - 1 - left) / p.sw);
     const float* const dyp = p.dy + int64_t(plane0) * m * p.OHOW;  // planes of dy follow (image, channel, j)
     depthwise_stage(a, patch, dyp, uint32_t(np * m * a.patch), oh0, ow0, p.OH, p.OW);
-    __syncthreads();
-    depthwise_items(a, np, [&](int pl, int row, int col) {
+    int edges = 0;
+    for (int e = threadIdx.x; e < np * m * KH * KW; e += 256) {
+      const uint32_t at = uint32_t(plane0 % p.Cin) * uint32_t(m * KH * KW) + e, n = uint32_t(p.Cout) * uint32_t(KH * KW);
+      edges |= !__builtin_isfinite(p.w[at % n]);
+    }
+    edges = __syncthreads_or(edges);
+    const auto item = [&](int pl, int row, int col, auto EDGES) {
+      constexpr int U = K ? K : 1;
       const uint32_t plane = plane0 + pl, img = fdiv(plane, a.f_cin);
       const int ic = int(plane - img * p.Cin);
       const int y0 = ih0 + row + p.ph - oh0 * p.sh, x0 = iw0 + col + p.pw - ow0 * p.sw;
@@ -265,6 +273,7 @@ __global__ __launch_bounds__(256) void conv_depthwise_dx_kernel(DepthwiseArgs a)
             for (int r = 0; r < kDwRows; ++r) {
               const int ty = y0 + r - kh * p.dh;
               const int qy = UNIT ? ty : int(fdiv(uint32_t(ty), a.f_sh));
+              if (EDGES && (unsigned(oh0 + qy) >= unsigned(p.OH) || unsigned(ow0 + qx) >= unsigned(p.OW))) continue;
               if (UNIT || (xok && qy * p.sh == ty)) acc[r] += src[qy * a.patch_w + qx] * wv;
             }
           }
@@ -273,7 +282,11 @@ __global__ __launch_bounds__(256) void conv_depthwise_dx_kernel(DepthwiseArgs a)
 #pragma unroll
       for (int r = 0; r < kDwRows; ++r)
         if (ih0 + row + r < p.H && iw0 + col < p.W) dst[r * p.W] = acc[r];
-    });
+    };
+    if (edges)
+      depthwise_items(a, np, [&](int pl, int row, int col) { item(pl, row, col, std::true_type{}); });
+    else
+      depthwise_items(a, np, [&](int pl, int row, int col) { item(pl, row, col, std::false_type{}); });
     __syncthreads();
   }
 }

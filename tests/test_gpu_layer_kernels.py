@@ -70,6 +70,43 @@ def test_depthwise_phases(mx, xs, m, k, s, p, dil):
         assert ((got.cpu().double() - ref).abs() <= terms * 2.0 ** -23 * mag + 1e-30).all()
 
 
+def depthwise_dx_by_taps(w, dy, shape, m, s, p, dil):
+    """The input gradient by its definition: a tap that leaves dy adds nothing."""
+    dx = torch.zeros(shape, dtype=torch.float64)
+    wide = dy.double().view(shape[0], shape[1], m, *dy.shape[2:])
+    for j in range(m):
+        for kh in range(w.shape[2]):
+            for kw in range(w.shape[3]):
+                ih = torch.arange(dy.shape[2]) * s[0] - p[0] + kh * dil[0]
+                iw = torch.arange(dy.shape[3]) * s[1] - p[1] + kw * dil[1]
+                rows, cols = (ih >= 0) & (ih < shape[2]), (iw >= 0) & (iw < shape[3])
+                tap = wide[:, :, j][:, :, rows][:, :, :, cols] * w.double().view(shape[1], m, *w.shape[2:])[:, j, kh, kw, None, None]
+                dx[:, :, ih[rows, None], iw[cols]] += tap
+    return dx
+
+
+@pytest.mark.parametrize("xs,m,k,s,p,dil", [DEPTHWISE[i] for i in (1, 2, 3, 5, 6, 7, 9, 10)])
+def test_depthwise_input_gradient_of_weights_not_finite(mx, xs, m, k, s, p, dil):
+    """Infinities and NaN in some filters reach the positions whose taps lie in
+    dy, not the zeros staged around it."""
+    g = torch.Generator().manual_seed(xs[1] + k[1])
+    w = torch.randn(xs[1] * m, 1, *k, generator=g)
+    w[1, 0, 0, 0], w[3, 0, -1, -1], w[-1, 0, 0, -1] = float("inf"), float("nan"), -float("inf")
+    d = mx.conv_desc(xs, tuple(w.shape), s, p, dil, xs[1])
+    dy = torch.randn(xs[0], xs[1] * m, d.oh, d.ow, generator=g)
+    dx = torch.zeros(xs, device="cuda")
+    wc, dyc = w.cuda(), dy.cuda()
+    torch.cuda.synchronize()
+    mx.conv2d_backward_input(d, dyc, wc, dx, mx.ALGO_DIRECT, stream())
+    torch.cuda.synchronize()
+    got, ref = dx.cpu().double(), depthwise_dx_by_taps(w, dy, xs, m, s, p, dil)
+    fine = ref.isfinite()
+    assert fine.any() and not fine.all()
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got[~fine & ~ref.isnan()], ref[~fine & ~ref.isnan()])
+    mag = depthwise_dx_by_taps(w.nan_to_num(0, 0, 0).abs(), dy.abs(), xs, m, s, p, dil)
+    assert ((got - ref).abs() <= (k[0] * k[1] * m + 2) * 2.0 ** -23 * mag + 1e-30)[fine].all()
+
+
 @pytest.mark.parametrize("n,c,h,w", [(1, 3, 1, 1), (2, 5, 7, 7), (64, 17, 6, 6), (65, 3, 5, 4), (130, 2, 3, 3),
                                      (3, 40, 32, 32), (2, 6, 33, 32), (200, 64, 4, 4)])
 @pytest.mark.parametrize("training", [True, False])
