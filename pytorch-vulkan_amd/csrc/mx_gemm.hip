@@ -275,10 +275,20 @@ double tile_cost(const TileChoice& t, int64_t tiles, int64_t cu, int64_t m, int6
 // Cheapest (tile, K split).  Few tiles over a long K leave most of the chip
 // idle (8 x 2048 x 1000: 16 workgroups walking 128 slabs each, 38 us), so K is
 // split where the model finds it faster, the partials summed by a second
-// launch.  `split_ok`: the call may allocate.  MX_GEMM_TILE=<index into
-// kTiles> forces a tile in one pass over K (tests and diagnosis; the 256-wide
-// tiles only for 16-byte operand modes).  `kernel` (mx_gemm_kernel) forces the 64x64 tile or
+// launch.  That launch and the partials' block cost the host 2.5 us (4.8 -> 7.3
+// a call), lost wherever a program issues its calls no faster than they run, so
+// a product that takes less than kMinSplitTime in one pass keeps it: about what
+// a training loop takes to issue one of its calls.  Training passes of a linear
+// layer, split / one pass: 8 x 573 x 466 56.9 / 49.1 us, 256 x 512 x 512 57.8 /
+// 52.6, 8 x 1024 x 1024 54.7 / 56.6, 8 x 2048 x 1000 54.1 / 78.7; forward calls
+// on their own: 8 x 512 x 512 10.0 / 13.5, 8 x 768 x 768 10.0 / 18.9, 8 x 2048 x
+// 1000 11.1 / 45.3.
+// `split_ok`: partials may be used.  MX_GEMM_TILE=<index into kTiles> forces a
+// tile in one pass over K (tests and diagnosis; the 256-wide tiles only for
+// 16-byte operand modes).  `kernel` (mx_gemm_kernel) forces the 64x64 tile or
 // keeps the choice among the large ones.
+constexpr double kMinSplitTime = 14e-6;
+
 void pick_gemm_tile(int64_t m, int64_t n, int64_t k, int64_t batch, bool vec, int kernel, bool split_ok, int* tile,
                     int* splits, int* kps) {
   int first = vec ? 0 : 2, last = 3;
@@ -291,18 +301,30 @@ void pick_gemm_tile(int64_t m, int64_t n, int64_t k, int64_t batch, bool vec, in
       split_ok = false;
     }
   }
-  static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
-  double best = -1;
   const int64_t cu = cu_count();
+  const auto tiles_of = [&](int i) {
+    return ((m + kTiles[i].bm - 1) / kTiles[i].bm) * ((n + kTiles[i].bn - 1) / kTiles[i].bn) * batch;
+  };
+  double best = -1;
+  *splits = 1;
+  *kps = int(k);
   for (int i = first; i <= last; ++i) {
-    const int64_t tiles = ((m + kTiles[i].bm - 1) / kTiles[i].bm) * ((n + kTiles[i].bn - 1) / kTiles[i].bn) * batch;
+    const double cost = tile_cost(kTiles[i], tiles_of(i), cu, m, n, batch, 1, k);
+    if (best < 0 || cost < best) {
+      best = cost;
+      *tile = i;
+    }
+  }
+  if (!split_ok || best < kMinSplitTime) return;
+  static const int kSplits[] = {2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
+  for (int i = first; i <= last; ++i) {
+    const int64_t tiles = tiles_of(i);
     for (const int want : kSplits) {
-      int64_t span = ((k + want - 1) / want + kSplitBK - 1) / kSplitBK * kSplitBK;
-      const int64_t s = (k + span - 1) / span;
-      if (s > 1 && (!split_ok || span < kMinSplitSpan || s * m * n * batch * 4 > kMaxSplitBytes)) break;
-      if (s == 1) span = k;
+      const int64_t span = ((k + want - 1) / want + kSplitBK - 1) / kSplitBK * kSplitBK, s = (k + span - 1) / span;
+      if (s < 2) continue;
+      if (span < kMinSplitSpan || s * m * n * batch * 4 > kMaxSplitBytes) break;
       const double cost = tile_cost(kTiles[i], tiles, cu, m, n, batch, s, span);
-      if (best < 0 || cost < best) {
+      if (cost < best) {
         best = cost;
         *tile = i;
         *splits = int(s);
@@ -417,8 +439,9 @@ extern "C" int mx_gemm_f32(const mx_gemm_desc* d, const float* a, const float* b
   MX_ABI_BEGIN
   hipStream_t s = resolve_stream(stream);
   GemmPlan g;
-  MX_TRY(plan_gemm(d, a, b, bias, c, may_allocate(s), &g));
+  MX_TRY(plan_gemm(d, a, b, bias, c, true, &g));
   if (g.empty) return MX_OK;
+  if (g.p.splits > 1 && !may_allocate(s)) MX_TRY(plan_gemm(d, a, b, bias, c, false, &g));
   MX_REQUIRE(c, MX_ERR_INVALID, "mx_gemm_f32: null output");
   MX_REQUIRE(d->bias_kind == MX_BIAS_NONE || bias, MX_ERR_INVALID, "mx_gemm_f32: null bias");
   GemmArgs& p = g.p;

@@ -393,3 +393,14 @@ int main() {
                     f"-Wl,-rpath,{torch_lib}", "-Wl,--allow-shlib-undefined"], check=True)
     run = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
     assert run.returncode == 0 and run.stdout.strip() == "unharmed", (run.returncode, run.stdout, run.stderr)
+
+
+@pytest.mark.parametrize("m,n,k,split", [(8, 466, 573, False), (64, 512, 512, False), (2, 216, 512, False),
+                                         (256, 512, 512, False), (8, 1000, 2048, True), (8, 1024, 1024, True),
+                                         (64, 64, 1 << 18, True), (8192, 4096, 4096, False)])
+def test_short_products_take_one_launch(mx, m, n, k, split):
+    """K is split where one pass over it is long, not where the second launch
+    costs a program that is bound by issuing its calls."""
+    import torch
+    a, b, c = (torch.empty(s, device="meta") for s in ((m, k), (k, n), (m, n)))
+    assert ("+split" in mx.gemm_variant(mx.gemm_desc(a, b, c))) == split
