@@ -108,7 +108,9 @@ def test_depthwise_input_gradient_of_weights_not_finite(mx, xs, m, k, s, p, dil)
 
 
 @pytest.mark.parametrize("n,c,h,w", [(1, 3, 1, 1), (2, 5, 7, 7), (64, 17, 6, 6), (65, 3, 5, 4), (130, 2, 3, 3),
-                                     (3, 40, 32, 32), (2, 6, 33, 32), (200, 64, 4, 4)])
+                                     (3, 40, 32, 32), (2, 6, 33, 32), (200, 64, 4, 4),
+                                     (1, 3, 60, 70), (2, 5, 61, 67), (5, 2, 160, 160),  # workgroups share a row
+                                     (9, 7, 3, 5), (9, 7, 4, 4), (3, 6, 8, 16), (2, 5, 11, 12)])
 @pytest.mark.parametrize("training", [True, False])
 def test_batch_norm_both_ways(mx, n, c, h, w, training):
     g = torch.Generator().manual_seed(n * c)
