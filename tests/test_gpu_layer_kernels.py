@@ -138,7 +138,11 @@ def test_batch_norm_both_ways(mx, n, c, h, w, training):
 @pytest.mark.parametrize("shape,perm", [((64, 64), (1, 0)), ((65, 130), (1, 0)), ((3, 16, 17), (0, 2, 1)),
                                         ((2, 5, 33, 66), (0, 2, 3, 1)), ((2, 40, 3, 70), (3, 1, 2, 0)),
                                         ((4, 15, 16), (0, 2, 1)), ((1, 7, 1, 129), (3, 0, 2, 1)),
-                                        ((2, 3, 20, 4, 18), (4, 1, 0, 3, 2))])
+                                        ((2, 3, 20, 4, 18), (4, 1, 0, 3, 2)),
+                                        # through LDS: more than 2^19 elements in tiles used enough
+                                        ((731, 1009), (1, 0)), ((9, 16, 4000), (0, 2, 1)), ((3, 4, 330, 198), (0, 2, 3, 1)),
+                                        ((3, 66, 50, 70), (3, 1, 2, 0)), ((513, 64, 16), (0, 2, 1)),
+                                        ((1100, 1, 477), (2, 1, 0))])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.int16])
 def test_permuted_copies(shape, perm, dtype):
     """contiguous() of permuted, broadcast and sliced views, and copies into them."""
