@@ -562,8 +562,9 @@ bool depthwise_staged(const mx_conv2d_desc& d) {
 // Tile of the staged depthwise kernels over planes of h x w values, of which
 // `per_plane` patches each are staged: columns up to 64, rows up to about 1024
 // values (a multiple of an item's rows), then as many planes as make up about
-// 3072 values, all within the LDS budget.  patch_dim(tile extent, axis) gives
-// the patch's rows / columns.  False when not even four rows fit.
+// 3072 values, all within the LDS budget and with two workgroups for every CU.
+// patch_dim(tile extent, axis) gives the patch's rows / columns.  False when not
+// even four rows fit.
 template <class F>
 bool depthwise_tile(DepthwiseArgs* a, int h, int w, int per_plane, F&& patch_dim) {
   a->tile_w = std::min(w, kDwTileW);
@@ -583,7 +584,10 @@ bool depthwise_tile(DepthwiseArgs* a, int h, int w, int per_plane, F&& patch_dim
   a->tiles_h = (h + rows - 1) / rows;
   a->tiles_w = (w + a->tile_w - 1) / a->tile_w;
   a->total_planes = a->p.N * a->p.Cin;
-  a->planes = std::max(1, std::min({3072 / (rows * a->tile_w), kDwLdsFloats / (a->patch * per_plane), a->total_planes}));
+  const int64_t wanted = 2 * cu_count();
+  const int64_t spread = (int64_t(a->total_planes) * a->tiles_h * a->tiles_w + wanted - 1) / wanted;
+  a->planes = int(std::max<int64_t>(1, std::min<int64_t>({3072 / (rows * a->tile_w), kDwLdsFloats / (a->patch * per_plane),
+                                                          a->total_planes, spread})));
   a->tiles = int64_t((a->total_planes + a->planes - 1) / a->planes) * a->tiles_w * a->tiles_h;
   a->f_tw = conv::fast_div(uint32_t(a->tile_w));
   a->f_strips = conv::fast_div(uint32_t(a->strips));
