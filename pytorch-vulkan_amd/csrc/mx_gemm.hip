@@ -253,7 +253,7 @@ struct TileChoice {
 };
 constexpr TileChoice kTiles[] = {{256, 128, 2, 1.81}, {128, 256, 2, 1.75}, {128, 128, 2, 1.70}, {64, 64, 4, 1.36}};
 
-constexpr int64_t kMaxSplitBytes = int64_t(64) << 20;  // partial products of one call
+constexpr int64_t kMaxSplitBytes = int64_t(64) << 20;  // partial products of one call (a caller's budget may hold less)
 constexpr int kSplitBK = 32;                           // K granularity of a split
 constexpr int kMinSplitSpan = 64;                      // shortest K range worth a split
 
@@ -283,13 +283,13 @@ double tile_cost(const TileChoice& t, int64_t tiles, int64_t cu, int64_t m, int6
 // 52.6, 8 x 1024 x 1024 54.7 / 56.6, 8 x 2048 x 1000 54.1 / 78.7; forward calls
 // on their own: 8 x 512 x 512 10.0 / 13.5, 8 x 768 x 768 10.0 / 18.9, 8 x 2048 x
 // 1000 11.1 / 45.3.
-// `split_ok`: partials may be used.  MX_GEMM_TILE=<index into kTiles> forces a
+// `partials`: bytes they may take.  MX_GEMM_TILE=<index into kTiles> forces a
 // tile in one pass over K (tests and diagnosis; the 256-wide tiles only for
 // 16-byte operand modes).  `kernel` (mx_gemm_kernel) forces the 64x64 tile or
 // keeps the choice among the large ones.
 constexpr double kMinSplitTime = 14e-6;
 
-void pick_gemm_tile(int64_t m, int64_t n, int64_t k, int64_t batch, bool vec, int kernel, bool split_ok, int* tile,
+void pick_gemm_tile(int64_t m, int64_t n, int64_t k, int64_t batch, bool vec, int kernel, int64_t partials, int* tile,
                     int* splits, int* kps) {
   int first = vec ? 0 : 2, last = 3;
   if (kernel == MX_GEMM_KERNEL_TILED) first = 3;
@@ -298,7 +298,7 @@ void pick_gemm_tile(int64_t m, int64_t n, int64_t k, int64_t batch, bool vec, in
     const int t = std::atoi(e);
     if (t >= (vec ? 0 : 2) && t < 4) {
       first = last = t;
-      split_ok = false;
+      partials = 0;
     }
   }
   const int64_t cu = cu_count();
@@ -315,14 +315,14 @@ void pick_gemm_tile(int64_t m, int64_t n, int64_t k, int64_t batch, bool vec, in
       *tile = i;
     }
   }
-  if (!split_ok || best < kMinSplitTime) return;
+  if (partials <= 0 || best < kMinSplitTime) return;
   static const int kSplits[] = {2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
   for (int i = first; i <= last; ++i) {
     const int64_t tiles = tiles_of(i);
     for (const int want : kSplits) {
       const int64_t span = ((k + want - 1) / want + kSplitBK - 1) / kSplitBK * kSplitBK, s = (k + span - 1) / span;
       if (s < 2) continue;
-      if (span < kMinSplitSpan || s * m * n * batch * 4 > kMaxSplitBytes) break;
+      if (span < kMinSplitSpan || s * m * n * batch * 4 > partials) break;
       const double cost = tile_cost(kTiles[i], tiles, cu, m, n, batch, s, span);
       if (cost < best) {
         best = cost;
@@ -361,7 +361,7 @@ struct GemmPlan {
   bool empty = false;
 };
 
-int plan_gemm(const mx_gemm_desc* d, const float* a, const float* b, const float* bias, float* c, bool split_ok,
+int plan_gemm(const mx_gemm_desc* d, const float* a, const float* b, const float* bias, float* c, int64_t partials,
               GemmPlan* g) {
   MX_REQUIRE(d, MX_ERR_INVALID, "mx_gemm_f32: null descriptor");
   MX_REQUIRE(d->batch >= 0 && d->m >= 0 && d->n >= 0 && d->k >= 0, MX_ERR_INVALID,
@@ -402,8 +402,7 @@ int plan_gemm(const mx_gemm_desc* d, const float* a, const float* b, const float
   g->ma = pick_mode(p.a, p.a_sm, p.a_sk, p.a_sb, p.batch, p.M, p.K);
   g->mb = pick_mode(p.b, p.b_sn, p.b_sk, p.b_sb, p.batch, p.N, p.K);
   pick_gemm_tile(d->m, d->n, d->k, d->batch, is_vec(g->ma) && is_vec(g->mb), d->kernel,
-                 split_ok && d->n <= kVecStrideMax && d->m * d->n <= INT32_MAX, &g->tile,
-                 &p.splits, &p.kps);
+                 d->n <= kVecStrideMax && d->m * d->n <= INT32_MAX ? partials : 0, &g->tile, &p.splits, &p.kps);
   return MX_OK;
 }
 
@@ -431,17 +430,16 @@ int launch_sum(const GemmArgs& p, hipStream_t s) {
 
 constexpr const char* kTileNames[] = {"256x128x16", "128x256x16", "128x128x16", "64x64x16"};
 
-}  // namespace
-}  // namespace mx
+int64_t partial_bytes(const GemmArgs& p) { return p.splits > 1 ? int64_t(p.splits) * p.batch * p.M * p.N * 4 : 0; }
 
-extern "C" int mx_gemm_f32(const mx_gemm_desc* d, const float* a, const float* b, const float* bias,
-                           float* c, void* stream) {
-  MX_ABI_BEGIN
-  hipStream_t s = resolve_stream(stream);
+}  // namespace
+
+int gemm_within(const mx_gemm_desc* d, const float* a, const float* b, const float* bias, float* c, int64_t partials,
+                hipStream_t s) {
   GemmPlan g;
-  MX_TRY(plan_gemm(d, a, b, bias, c, true, &g));
+  MX_TRY(plan_gemm(d, a, b, bias, c, std::min(partials, kMaxSplitBytes), &g));
   if (g.empty) return MX_OK;
-  if (g.p.splits > 1 && !may_allocate(s)) MX_TRY(plan_gemm(d, a, b, bias, c, false, &g));
+  if (g.p.splits > 1 && !may_allocate(s)) MX_TRY(plan_gemm(d, a, b, bias, c, 0, &g));
   MX_REQUIRE(c, MX_ERR_INVALID, "mx_gemm_f32: null output");
   MX_REQUIRE(d->bias_kind == MX_BIAS_NONE || bias, MX_ERR_INVALID, "mx_gemm_f32: null bias");
   GemmArgs& p = g.p;
@@ -455,11 +453,11 @@ extern "C" int mx_gemm_f32(const mx_gemm_desc* d, const float* a, const float* b
   MX_REQUIRE(a && b, MX_ERR_INVALID, "mx_gemm_f32: null operand");
   Scratch ws;
   if (p.splits > 1) {
-    if (ws.alloc(size_t(p.splits) * p.batch * p.M * p.N * 4, s) == MX_OK) {
+    if (ws.alloc(size_t(partial_bytes(p)), s) == MX_OK) {
       p.ws = ws.as<float>();
     } else {  // no room for partials: one pass over K
       clear_error();
-      MX_TRY(plan_gemm(d, a, b, bias, c, false, &g));
+      MX_TRY(plan_gemm(d, a, b, bias, c, 0, &g));
     }
   }
   switch (g.tile) {
@@ -469,25 +467,41 @@ extern "C" int mx_gemm_f32(const mx_gemm_desc* d, const float* a, const float* b
     default: MX_TRY(launch1<TileSmall>(p, g.ma, g.mb, s));
   }
   return p.splits > 1 ? launch_sum(p, s) : MX_OK;
+}
+
+int gemm_describe(const mx_gemm_desc* d, const float* a, const float* b, int64_t partials, std::string* name,
+                  int64_t* bytes) {
+  GemmPlan g;
+  MX_TRY(plan_gemm(d, a, b, nullptr, nullptr, std::min(partials, kMaxSplitBytes), &g));
+  *bytes = g.empty ? 0 : partial_bytes(g.p);
+  if (g.empty) {
+    *name = "none";
+  } else if (d->k == 0) {
+    *name = "gemm_k0_kernel";
+  } else {
+    const int kind = (d->bias_kind == MX_BIAS_NONE || d->beta == 0.f) ? MX_BIAS_NONE : d->bias_kind;
+    *name = cat("gemm_kernel<", kTileNames[g.tile], ",", mode_name(g.ma), ",", mode_name(g.mb), ">", g.p.splits > 1 ? "+split" : "",
+               kind == MX_BIAS_COL ? "+bias_col" : kind == MX_BIAS_MATRIX ? "+bias_matrix" : "",
+               d->batch > 65535 ? "+batch_chunks" : "");
+  }
+  return MX_OK;
+}
+
+}  // namespace mx
+
+extern "C" int mx_gemm_f32(const mx_gemm_desc* d, const float* a, const float* b, const float* bias,
+                           float* c, void* stream) {
+  MX_ABI_BEGIN
+  return gemm_within(d, a, b, bias, c, kMaxSplitBytes, resolve_stream(stream));
   MX_ABI_END
 }
 
 extern "C" int mx_gemm_variant(const mx_gemm_desc* d, const float* a, const float* b, char* buf, size_t len) {
   MX_ABI_BEGIN
   MX_REQUIRE(buf || !len, MX_ERR_INVALID, "mx_gemm_variant: null buffer");
-  GemmPlan g;
-  MX_TRY(plan_gemm(d, a, b, nullptr, nullptr, true, &g));
   std::string name;
-  if (g.empty) {
-    name = "none";
-  } else if (d->k == 0) {
-    name = "gemm_k0_kernel";
-  } else {
-    const int kind = (d->bias_kind == MX_BIAS_NONE || d->beta == 0.f) ? MX_BIAS_NONE : d->bias_kind;
-    name = cat("gemm_kernel<", kTileNames[g.tile], ",", mode_name(g.ma), ",", mode_name(g.mb), ">", g.p.splits > 1 ? "+split" : "",
-               kind == MX_BIAS_COL ? "+bias_col" : kind == MX_BIAS_MATRIX ? "+bias_matrix" : "",
-               d->batch > 65535 ? "+batch_chunks" : "");
-  }
+  int64_t bytes = 0;
+  MX_TRY(gemm_describe(d, a, b, kMaxSplitBytes, &name, &bytes));
   if (len) {
     std::strncpy(buf, name.c_str(), len - 1);
     buf[len - 1] = 0;

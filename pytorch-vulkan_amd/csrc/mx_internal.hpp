@@ -58,6 +58,13 @@ int upload(const void* host, size_t bytes, hipStream_t s, Scratch& holder);
 // Number of compute units of the current device (cached).
 int cu_count();
 
+// mx_gemm_f32 with at most `partials` bytes of scratch for a K split, and the
+// kernels and scratch of such a call (mx_gemm.hip).
+int gemm_within(const mx_gemm_desc* d, const float* a, const float* b, const float* bias, float* c, int64_t partials,
+                hipStream_t s);
+int gemm_describe(const mx_gemm_desc* d, const float* a, const float* b, int64_t partials, std::string* name,
+                  int64_t* bytes);
+
 }  // namespace mx
 
 #define MX_HIP(expr)                                                                  \

@@ -1818,9 +1818,6 @@ __global__ __launch_bounds__(512) void wino_bwd_kernel(fused::Args pf, fused_dw:
 }
 }  // namespace bwd
 
-int winograd_unfused(const mx_conv2d_desc& d, const float* x, const float* w, const float* bias, float* y,
-                     bool flip, int64_t chunk, hipStream_t s);
-
 }  // namespace
 
 namespace {
@@ -1847,7 +1844,7 @@ mx_gemm_desc unfused_gemm_desc(int G, int Cout_g, int Cin_g, int64_t T) {
 }
 
 int winograd_unfused(const mx_conv2d_desc& d, const float* x, const float* w, const float* bias, float* y,
-                     bool flip, int64_t chunk, hipStream_t s) {
+                     bool flip, int64_t chunk, int64_t partials, hipStream_t s) {
   WinoArgs p{};
   p.flip = flip ? 1 : 0;
   p.w = w;
@@ -1886,7 +1883,7 @@ int winograd_unfused(const mx_conv2d_desc& d, const float* x, const float* w, co
     hipLaunchKernelGGL(wino_input_kernel, dim3(blocks_for(int64_t(p.Cin) * p.T)), dim3(256), 0, s, p);
     MX_HIP(hipGetLastError());
     const mx_gemm_desc gd = unfused_gemm_desc(p.G, p.Cout_g, p.Cin_g, p.T);
-    MX_TRY(mx_gemm_f32(&gd, p.U, p.V, nullptr, p.M, s));
+    MX_TRY(gemm_within(&gd, p.U, p.V, nullptr, p.M, partials, s));
     hipLaunchKernelGGL(wino_output_kernel, dim3(blocks_for(int64_t(p.Cout) * p.T)), dim3(256), 0, s, p);
     MX_HIP(hipGetLastError());
   }
@@ -2081,7 +2078,7 @@ int winograd_run(const mx_conv2d_desc& d, const float* x, const float* w, const 
   MX_TRY(plan_run(d, ws_limit, flip, &r));
   fused::Args& p = r.p;
   if (p.T == 0) return MX_OK;
-  if (!r.fused) return winograd_unfused(d, x, w, bias, y, flip, r.chunk, s);
+  if (!r.fused) return winograd_unfused(d, x, w, bias, y, flip, r.chunk, ws_limit - r.unfused_bytes, s);
   p.bias = bias;
   p.x = x;
   p.y = y;
@@ -2296,13 +2293,15 @@ int winograd_describe(const mx_conv2d_desc& d, int phase, bool with_bias, int64_
                    r.filt ? ",filter>" : ">");
     *ws_bytes = r.parts > 1 ? r.parts * r.p.part_stride * 4 : 0;
   } else {
-    // U, V and M are fresh mx_malloc blocks (256-byte aligned).
+    // U, V and M are fresh mx_malloc blocks (256-byte aligned); the product's
+    // partials take what they leave of the budget.
     const mx_gemm_desc gd = unfused_gemm_desc(r.G, r.p.O, r.p.C, r.chunk * r.p.TH * r.p.TW);
     const float* aligned = reinterpret_cast<const float*>(uintptr_t(256));
-    char gname[96];
-    MX_TRY(mx_gemm_variant(&gd, aligned, aligned, gname, sizeof gname));
+    std::string gname;
+    int64_t partials = 0;
+    MX_TRY(gemm_describe(&gd, aligned, aligned, ws_limit - r.unfused_bytes, &gname, &partials));
     *variant = cat("wino_unfused(", gname, ")", r.chunk < d.n ? "+chunks" : "");
-    *ws_bytes = r.unfused_bytes;
+    *ws_bytes = r.unfused_bytes + partials;
   }
   if (phase == MX_CONV_DINPUT) *variant += "+flip";
   return MX_OK;

@@ -408,6 +408,32 @@ def test_forward_weight_order(mx, n, c, h, wd, o, k, stride, dil, groups, shift)
     assert ((y.cpu().double() - ref).abs() <= (c * k * k / 16 + 8) * 2.0 ** -23 * mag).all()
 
 
+@pytest.mark.parametrize("n,c,hw,o,budget", [(16, 4096, 4, 64, 33), (16, 4096, 4, 64, 64), (1, 4096, 7, 64, 21),
+                                              (2, 4096, 8, 64, 21)])
+def test_winograd_passes_keep_to_the_workspace(mx, monkeypatch, n, c, hw, o, budget):
+    """The passes' batched product splits K within what U, V and M leave of the
+    budget, and the plan names all of it."""
+    monkeypatch.setenv("TORCH_VULKAN_CONV_WORKSPACE_MB", str(budget))
+    g = torch.Generator().manual_seed(c + o)
+    x, w = torch.randn(n, c, hw, hw, generator=g), torch.randn(o, c, 3, 3, generator=g)
+    d = mx.conv_desc(x.shape, w.shape, (1, 1), (1, 1))
+    plan = mx.conv2d_plan(d, mx.MX_CONV_FORWARD, mx.ALGO_WINOGRAD)
+    assert plan["variant"].startswith("wino_unfused") and plan["workspace_bytes"] <= budget << 20
+    xd, wd, y = x.cuda(), w.cuda(), torch.full((n, o, hw, hw), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    stats = mx.MemoryStats()
+    mx.check(mx.lib().mx_empty_cache())
+    mx.check(mx.lib().mx_memory_stats_get(mx.C.byref(stats)))
+    before = stats.reserved_bytes
+    mx.conv2d_forward(d, xd, wd, None, y, mx.ALGO_WINOGRAD, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    mx.check(mx.lib().mx_memory_stats_get(mx.C.byref(stats)))
+    # Blocks above 1 MiB are whole multiples of 2 MiB: U and V here are, M and the partials at most one is not.
+    assert plan["workspace_bytes"] <= stats.reserved_bytes - before < plan["workspace_bytes"] + (2 << 20)
+    ref = F.conv2d(x.double(), w.double(), None, 1, 1)
+    assert ((y.cpu().double() - ref).norm() / ref.norm()).item() < 3e-6
+
+
 @pytest.mark.parametrize("n,c,hw,o,groups", [
     (1, 256, (16, 32), 64, 1),     # even slabs, 16-channel parts
     (1, 145, (23, 24), 70, 1),     # ragged channels, a shorter last part
