@@ -225,17 +225,36 @@ def test_gemm_k_split(mx, m, n, k, batch, bias_kind):
 
 
 def test_gemm_under_capture_takes_no_scratch(mx):
-    """A captured call runs in one pass: replays read and write only the
-    operands, whatever the allocator does between them."""
+    """A captured call runs in one pass: it takes no block from the allocator,
+    and replays write none of those that an eager call's partials came from."""
     a, b = torch.randn(8, 2048, device="cuda"), torch.randn(2048, 1000, device="cuda")
     c, eager = torch.empty(8, 1000, device="cuda"), torch.empty(8, 1000, device="cuda")
     s = torch.cuda.Stream()
-    mx.gemm(a, b, c, stream=s.cuda_stream)  # loads the kernels
+    assert "+split" in mx.gemm_variant(mx.gemm_desc(a, b, c))
     torch.cuda.synchronize()
-    before = mx.memory_stats().device_mallocs if hasattr(mx, "memory_stats") else None
+    mx.check(mx.lib().mx_empty_cache())
+    mx.gemm(a, b, c, stream=s.cuda_stream)  # loads the kernels, leaves the partials' block in the cache
+    torch.cuda.synchronize()
+
+    def blocks():
+        st = mx.MemoryStats()
+        mx.check(mx.lib().mx_memory_stats_get(mx.C.byref(st)))
+        return st.device_mallocs + st.cache_hits, st.cached_blocks
+
+    before = blocks()
+    assert before[1] == 1
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=s):
         mx.gemm(a, b, c, stream=s.cuda_stream)
+    assert blocks() == before
+    # The cached block, whichever number of partials it holds, filled by its next owner.
+    mine = []
+    for splits in range(2, 65):
+        p, size = mx.C.c_void_p(), splits * 8 * 1000 * 4
+        mx.check(mx.lib().mx_malloc(mx.C.byref(p), size, mx.C.c_void_p(s.cuda_stream)))
+        mx.check(mx.lib().mx_fill(p, size // 4, 4, 0x7FC0BEEF, mx.C.c_void_p(s.cuda_stream)))
+        mine.append((p, size))
+    assert blocks()[1] == 0
     for i in range(3):
         a.normal_()
         c.zero_()
@@ -245,7 +264,11 @@ def test_gemm_under_capture_takes_no_scratch(mx):
         mx.gemm(a, b, eager, stream=s.cuda_stream)
         torch.cuda.synchronize()
         assert ((c - eager).norm() / eager.norm()).item() < 2e-6
-    assert before is None or mx.memory_stats().device_mallocs == before
+    for p, size in mine:
+        host = torch.empty(size // 4, dtype=torch.int32)
+        mx.check(mx.lib().mx_memcpy(mx.C.c_void_p(host.data_ptr()), p, size, mx.MX_COPY_D2H, None))
+        assert (host == 0x7FC0BEEF).all()
+        mx.check(mx.lib().mx_free(p))
 
 
 def winograd_magnitude(x, w, pad, oh, ow):
