@@ -635,20 +635,24 @@ int conv_depthwise_forward(const mx_conv2d_desc& d, const float* x, const float*
 
 bool is_depthwise(const mx_conv2d_desc& d) { return d.groups == d.cin && d.groups > 1; }
 
-// Input gradient of a depthwise layer in place of the one-thread-per-value
-// kernel; false where no patch fits (then nothing was launched).
-bool conv_depthwise_dx(const mx_conv2d_desc& d, const ConvArgs& p, hipStream_t s) {
-  DepthwiseArgs a{};
-  a.p = p;
+// Tile of a depthwise layer's input gradient in place of the
+// one-thread-per-value kernel; false where no patch fits.
+bool depthwise_dx_tile(const mx_conv2d_desc& d, DepthwiseArgs* a) {
   const int64_t m = d.cout / d.groups;
   const auto patch_dim = [&](int64_t n, int axis) {
     return (n - 1 + (axis ? (d.kw - 1) * d.dw : (d.kh - 1) * d.dh)) / (axis ? d.sw : d.sh) + 2;
   };
-  if (m > kDwLdsFloats || !depthwise_tile(&a, int(d.h), int(d.w), int(m), patch_dim)) return false;
+  return is_depthwise(d) && m <= kDwLdsFloats && depthwise_tile(a, int(d.h), int(d.w), int(m), patch_dim);
+}
+// Its kernel's template arguments: filter size (0: any) and unit stride.
+int depthwise_dx_k(const mx_conv2d_desc& d) { return d.kh == d.kw && (d.kh == 3 || d.kh == 5) ? int(d.kh) : 0; }
+bool depthwise_dx_unit(const mx_conv2d_desc& d) { return d.sh == 1 && d.sw == 1; }
+
+void conv_depthwise_dx(const mx_conv2d_desc& d, const DepthwiseArgs& a, hipStream_t s) {
   const dim3 grid(unsigned(std::min<int64_t>(a.tiles, 1 << 20)));
-  const size_t lds = depthwise_lds(a, int(m));
-  const int k = d.kh == d.kw && (d.kh == 3 || d.kh == 5) ? int(d.kh) : 0;
-  const bool unit = d.sh == 1 && d.sw == 1;
+  const size_t lds = depthwise_lds(a, int(d.cout / d.groups));
+  const int k = depthwise_dx_k(d);
+  const bool unit = depthwise_dx_unit(d);
 #define MX_DW_DX(K)                                                                                     \
   if (unit)                                                                                             \
     hipLaunchKernelGGL((conv_depthwise_dx_kernel<K, true>), grid, dim3(256), lds, s, a);                \
@@ -662,27 +666,29 @@ bool conv_depthwise_dx(const mx_conv2d_desc& d, const ConvArgs& p, hipStream_t s
     MX_DW_DX(0)
   }
 #undef MX_DW_DX
-  return true;
 }
 
-// Weight gradient (and dBias) of a depthwise layer with 1, 3, 5 or 7 filter
-// columns in place of the one-workgroup-per-weight reduction; false otherwise
-// (also where the walk over a tensor's images would pass a buffer's range).
-bool conv_depthwise_dw(const mx_conv2d_desc& d, const ConvArgs& p, hipStream_t s) {
-  const int64_t step = std::max<int64_t>(1, 1024 / (d.oh * d.ow));
-  if (d.cout > INT32_MAX / 16 || d.kh > 65535 ||
-      (d.n + kDwImages * step) * std::max(d.cin * d.h * d.w, d.cout * d.oh * d.ow) * 4 >= kBufMaxBytes)
-    return false;
+// Whether a depthwise layer's weight gradient (and dBias) runs on its own kernel
+// in place of the one-workgroup-per-weight reduction: 1, 3, 5 or 7 filter
+// columns, and a walk over the tensors' images within a buffer's range.
+int64_t depthwise_dw_step(const mx_conv2d_desc& d) { return std::max<int64_t>(1, 1024 / (d.oh * d.ow)); }
+bool depthwise_dw_fits(const mx_conv2d_desc& d) {
+  return is_depthwise(d) && (d.kw == 1 || d.kw == 3 || d.kw == 5 || d.kw == 7) && d.cout <= INT32_MAX / 16 &&
+         d.kh <= 65535 &&
+         (d.n + kDwImages * depthwise_dw_step(d)) * std::max(d.cin * d.h * d.w, d.cout * d.oh * d.ow) * 4 < kBufMaxBytes;
+}
+
+void conv_depthwise_dw(const mx_conv2d_desc& d, const ConvArgs& p, hipStream_t s) {
+  const int64_t step = depthwise_dw_step(d);
   // As many waves as the positions taken at once fill: 28 x 28 runs on 13,
   // so 576 workgroups (192 channels) are on the chip together.
   const int64_t positions = step * d.oh * d.ow, chunks = (positions + 1023) / 1024;
   const dim3 grid(unsigned(d.cout), unsigned(d.kh)), block(unsigned((positions + 64 * chunks - 1) / (64 * chunks) * 64));
   switch (d.kw) {
-    case 1: hipLaunchKernelGGL(conv_depthwise_dw_kernel<1>, grid, block, 0, s, p, int(step)); return true;
-    case 3: hipLaunchKernelGGL(conv_depthwise_dw_kernel<3>, grid, block, 0, s, p, int(step)); return true;
-    case 5: hipLaunchKernelGGL(conv_depthwise_dw_kernel<5>, grid, block, 0, s, p, int(step)); return true;
-    case 7: hipLaunchKernelGGL(conv_depthwise_dw_kernel<7>, grid, block, 0, s, p, int(step)); return true;
-    default: return false;
+    case 1: hipLaunchKernelGGL(conv_depthwise_dw_kernel<1>, grid, block, 0, s, p, int(step)); break;
+    case 3: hipLaunchKernelGGL(conv_depthwise_dw_kernel<3>, grid, block, 0, s, p, int(step)); break;
+    case 5: hipLaunchKernelGGL(conv_depthwise_dw_kernel<5>, grid, block, 0, s, p, int(step)); break;
+    case 7: hipLaunchKernelGGL(conv_depthwise_dw_kernel<7>, grid, block, 0, s, p, int(step)); break;
   }
 }
 
@@ -1373,6 +1379,11 @@ int describe(const mx_conv2d_desc* desc, int phase, int algo, int with_bias, mx_
     MX_TRY(winograd_describe(d, phase, with_bias != 0, limit, &name, &r.workspace_bytes));
   } else if (chosen == MX_CONV_ALGO_DEPTHWISE) {
     name = depthwise_staged(d) ? "conv_depthwise_kernel<staged>" : "conv_depthwise_kernel<global>";
+  } else if (DepthwiseArgs a{make_args(d)};
+             chosen == MX_CONV_ALGO_DIRECT && phase == MX_CONV_DINPUT && depthwise_dx_tile(d, &a)) {
+    name = cat("conv_depthwise_dx_kernel<", depthwise_dx_k(d), depthwise_dx_unit(d) ? ",unit>" : ">");
+  } else if (chosen == MX_CONV_ALGO_REDUCE && phase == MX_CONV_DWEIGHT && depthwise_dw_fits(d)) {
+    name = cat("conv_depthwise_dw_kernel<", d.kw, ">");  // dBias among it
   } else if (chosen == MX_CONV_ALGO_DIRECT) {
     name = phase == MX_CONV_FORWARD  ? "conv_fwd_direct_kernel"
            : phase == MX_CONV_DINPUT ? "conv_dx_direct_kernel"
@@ -1519,7 +1530,11 @@ int mx_conv2d_backward_input(const mx_conv2d_desc* desc, const float* dy, const 
     p.dy = dy;
     p.w = w;
     p.out = dx;
-    if (!is_depthwise(d) || !conv_depthwise_dx(d, p, s))
+    DepthwiseArgs a{};
+    a.p = p;
+    if (depthwise_dx_tile(d, &a))
+      conv_depthwise_dx(d, a, s);
+    else
       hipLaunchKernelGGL(conv_dx_direct_kernel, dim3(linear_blocks(d.n * d.cin * d.h * d.w)), dim3(256), 0, s, p);
     MX_HIP(hipGetLastError());
     return MX_OK;
@@ -1636,7 +1651,8 @@ int dweight_impl(const mx_conv2d_desc* desc, const float* x, const float* dy, fl
     p.dy = dy;
     p.out = dw;
     p.db = db;
-    if (chosen == MX_CONV_ALGO_REDUCE && is_depthwise(d) && conv_depthwise_dw(d, p, s)) {
+    if (chosen == MX_CONV_ALGO_REDUCE && depthwise_dw_fits(d)) {
+      conv_depthwise_dw(d, p, s);
       MX_HIP(hipGetLastError());
       return MX_OK;
     }

@@ -2289,8 +2289,8 @@ int winograd_describe(const mx_conv2d_desc& d, int phase, bool with_bias, int64_
   RunPlan r;
   MX_TRY(plan_run(phase == MX_CONV_DINPUT ? dinput_as_forward(d) : d, ws_limit, phase == MX_CONV_DINPUT, &r));
   if (r.fused) {
-    *variant = cat(r.t16 ? "wino_ws16_kernel<" : "wino_ws_kernel<", r.p.C % (2 * fused::BK) ? "ragged" : "even",
-                   r.filt ? ",filter>" : ">");
+    *variant = cat(r.t16 ? "wino_ws16_kernel<" : r.filt ? "wino_ws_filter_kernel<" : "wino_ws_kernel<",
+                   r.p.C % (2 * fused::BK) ? "ragged" : "even", r.filt ? ",filter>" : ">", r.parts > 1 ? "+parts" : "");
     *ws_bytes = r.parts > 1 ? r.parts * r.p.part_stride * 4 : 0;
   } else {
     // U, V and M are fresh mx_malloc blocks (256-byte aligned); the product's

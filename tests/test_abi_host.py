@@ -404,3 +404,24 @@ def test_short_products_take_one_launch(mx, m, n, k, split):
     import torch
     a, b, c = (torch.empty(s, device="meta") for s in ((m, k), (k, n), (m, n)))
     assert ("+split" in mx.gemm_variant(mx.gemm_desc(a, b, c))) == split
+
+
+def test_names_of_depthwise_and_winograd_kernels(mx, monkeypatch):
+    """Plans name the kernels that run, apart from those they took the place of."""
+    def variant(xs, cout, k, stride, phase, algo, groups, **kw):
+        d = mx.conv_desc(xs, (cout, xs[1] // groups, k, k), (stride, stride), (k // 2, k // 2), (1, 1), groups)
+        return mx.conv2d_plan(d, phase, algo, **kw)["variant"]
+    dx, dw = mx.MX_CONV_DINPUT, mx.MX_CONV_DWEIGHT
+    assert variant((2, 8, 20, 20), 8, 3, 1, dx, mx.ALGO_DIRECT, 8) == "conv_depthwise_dx_kernel<3,unit>"
+    assert variant((2, 8, 20, 20), 16, 5, 2, dx, mx.ALGO_DIRECT, 8) == "conv_depthwise_dx_kernel<5>"
+    assert variant((2, 8, 20, 20), 8, 7, 1, dx, mx.ALGO_DIRECT, 8) == "conv_depthwise_dx_kernel<0,unit>"
+    assert variant((2, 8, 20, 20), 8, 3, 1, dx, mx.ALGO_DIRECT, 1) == "conv_dx_direct_kernel"
+    assert variant((2, 8, 20, 20), 8, 3, 1, dw, mx.ALGO_REDUCE, 8, with_bias=True) == "conv_depthwise_dw_kernel<3>"
+    assert variant((2, 8, 20, 20), 8, 9, 1, dw, mx.ALGO_REDUCE, 8, with_bias=True) == \
+        "conv_dw_reduce_kernel conv_db_reduce_kernel"
+    assert variant((1, 256, 32, 32), 256, 3, 1, mx.MX_CONV_FORWARD, mx.ALGO_WINOGRAD, 1) == "wino_ws16_kernel<even>+parts"
+    monkeypatch.setenv("MX_WINOGRAD_FUSED", "1")
+    monkeypatch.setenv("MX_WINOGRAD_T16", "0")
+    for filt, name in (("0", "wino_ws_kernel<even>"), ("1", "wino_ws_filter_kernel<even,filter>")):
+        monkeypatch.setenv("MX_WINOGRAD_FILTER", filt)
+        assert variant((2, 32, 8, 8), 32, 3, 1, mx.MX_CONV_FORWARD, mx.ALGO_WINOGRAD, 1) == name
