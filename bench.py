@@ -50,11 +50,21 @@ REPO = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, os.path.join(REPO, "pytorch-vulkan_amd"))
 
 PEAK_FP32_TFLOPS = 157.3
+# FP32 products as six bf16 products of three-piece operands: a sixth of the
+# dense bf16 matrix rate.
+PEAK_SPLIT_TFLOPS = 2500.0 / 6
+SPLIT_KERNELS = ("conv_fwd_kernel", "conv_dx_kernel", "conv_dx_phases_kernel", "conv_dw_kernel", "gemm_kernel",
+                 "wino_ws_kernel")
 PEAK_HBM_GBS = 8000.0
 TRAFFIC_FILE = os.path.join(REPO, "profiles", "traffic_c3.json")
 TRAFFIC_C5_FILE = os.path.join(REPO, "profiles", "traffic_c5.json")
 COPY_FLOATS = 256 * 1024 * 1024  # calibration copy: 1 GiB read, 1 GiB written
 METRIC = "Conv2D fwd+bwd FP32 TFLOP/s & % MFMA peak; fused AdamW GB/s; 1 MI355X"
+
+
+def mfma_peak(kernel):
+    """Peak TFLOP/s of the matrix instruction a kernel's products run on."""
+    return PEAK_SPLIT_TFLOPS if kernel.split("<")[0] in SPLIT_KERNELS else PEAK_FP32_TFLOPS
 
 
 # ------------------------------------------------------------------ workloads
@@ -384,6 +394,7 @@ def c4_kernel_table(tv, step, steps):
             # tile instead of 36).
             row["tflop_s"] = round(v["flops"] / (ms * 1e-3) / 1e12, 3)
             row["executed_tflop_s"] = round(ex / (ms * 1e-3) / 1e12, 3)
+            row["frac_of_peak"] = round(row["executed_tflop_s"] / mfma_peak(name), 4)
             row["frac_of_fp32_peak"] = round(row["executed_tflop_s"] / PEAK_FP32_TFLOPS, 4)
         rows.append((ms, v["flops"], v["samples"], row, ex))
     rows.sort(key=lambda r: -r[0])
@@ -401,7 +412,8 @@ def c4_kernel_table(tv, step, steps):
         res["conv_gemm_executed_tflop_s"] = round(gemm_exec / (gemm_ms * 1e-3) / 1e12, 3)
         res["conv_gemm_frac_of_fp32_peak_executed"] = round(res["conv_gemm_executed_tflop_s"] / PEAK_FP32_TFLOPS, 4)
         res["roofline"] = {"bound": "mfma", "kernel": row["kernel"], "achieved": round(achieved, 3),
-                           "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s", "frac": round(achieved / PEAK_FP32_TFLOPS, 4),
+                           "peak": round(mfma_peak(row["kernel"]), 1), "unit": "TFLOP/s",
+                           "frac": round(achieved / mfma_peak(row["kernel"]), 4),
                            "flops_counted": "executed (Winograd: 16 products per 2x2 tile)",
                            "traffic": None, "launches": n, "avg_launch_us": row["avg_us"],
                            "timing": "HIP events around each call on its stream"}
@@ -979,11 +991,11 @@ def roofline_from(agg, bound, wino_exec_ratio=None):
     avg_us = 1000.0 * ms / n
     if bound == "mfma":
         achieved = flops / n / (avg_us * 1e-6) / 1e12
-        peak, unit = PEAK_FP32_TFLOPS, "TFLOP/s"
+        peak, unit = mfma_peak(label), "TFLOP/s"
     else:
         achieved = nbytes / n / (avg_us * 1e-6) / 1e9
         peak, unit = PEAK_HBM_GBS, "GB/s"
-    out = {"bound": bound, "kernel": label, "achieved": round(achieved, 3), "peak": peak, "unit": unit,
+    out = {"bound": bound, "kernel": label, "achieved": round(achieved, 3), "peak": round(peak, 1), "unit": unit,
            "frac": round(achieved / peak, 4), "traffic": None, "launches": n, "avg_launch_us": round(avg_us, 3)}
     if whole_call:
         out["note"] = ("one Winograd call: its main kernel and the launch beside it (filter transform or "

@@ -32,3 +32,11 @@ def test_roofline_whole_winograd_call_at_executed_flops(bench):
     assert r["achieved"] == pytest.approx(0.5e9 / 40e-6 / 1e12, rel=1e-3)
     assert r["avg_launch_us"] == pytest.approx(40.0)
     assert "Winograd" in r["note"]
+
+
+def test_roofline_divides_by_the_rate_of_the_instruction_used(bench):
+    for kernel, peak in (("conv_dw_kernel<128x128x16>", 2500 / 6), ("gemm_kernel<64x64x16,KVEC,KVEC>", 2500 / 6),
+                         ("wino_ws_kernel", 2500 / 6), ("wino_ws16_kernel", 157.3), ("wino_dw_ws_kernel", 157.3)):
+        r = bench.roofline_from({kernel: (10, 0.30, 1e10, 0)}, "mfma", 0.5)
+        assert r["peak"] == pytest.approx(peak, abs=0.05)
+        assert r["frac"] == pytest.approx(r["achieved"] / peak, rel=1e-3)
