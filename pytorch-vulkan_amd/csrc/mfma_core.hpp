@@ -72,12 +72,9 @@ struct Acc {
 // instruction touches a loaded value before it is stored to LDS one slab
 // later.  (A branch or a select right after the load makes the compiler wait
 // for every load in flight, prefetched slabs included.)
-static __device__ __attribute__((aligned(16))) float kZeroPage[4];  // zero-initialised, never written
+static __device__ float kZeroPage[1];  // zero-initialised, never written
 
 __device__ __forceinline__ float load_or_zero(const float* p, bool ok) { return *(ok ? p : kZeroPage); }
-__device__ __forceinline__ f32x4 load4_or_zero(const float* p, bool ok) {
-  return *reinterpret_cast<const f32x4*>(ok ? p : kZeroPage);
-}
 
 // Raw buffer loads.  An operand tensor becomes one buffer resource (base,
 // byte extent) held in scalar registers; a lane supplies a 32-bit byte offset
@@ -502,12 +499,14 @@ template <class L>
 __device__ __forceinline__ void merge_row_sums(L&, const L&, long) {}
 
 // Split main loop over nk slabs, one barrier per slab: slab t + 1 is split and
-// written to the other stage among slab t's products.  Tiles up to 128x128
-// keep two register sets, even slabs in one and odd slabs in the other, so a
-// load has two slabs of products to land; the larger tiles have registers for
-// one set, and slabs long enough to cover a load.  The loop runs whole pairs
-// of slabs (one exit keeps the accumulators in place): an odd count runs one
-// more, of zeros, since loads past the last slab read zeros.
+// written to the other stage among slab t's products.  DEEP tiles (64x64x16;
+// 128x128 in the convolution forward and input gradient, and in GEMMs that read
+// both operands 16 bytes at a time) keep two register sets, even slabs in one
+// and odd slabs in the other, so a load has two slabs of products to land; the
+// others have registers for one set, or slabs long enough to cover a load.  The
+// DEEP loop runs whole pairs of slabs (one exit keeps the accumulators in
+// place): an odd count runs one more, of zeros, since loads past the last slab
+// read zeros.
 template <class C, class LA, class LB>
 __device__ __forceinline__ void mainloop_split(Acc<C>& acc, LA& la, LB& lb, int nk, float* smem) {
   float* const As = smem;
