@@ -330,6 +330,15 @@ typedef struct mx_gemm_desc {
 
 enum mx_gemm_kernel { MX_GEMM_KERNEL_AUTO = 0, MX_GEMM_KERNEL_TILED = 1, MX_GEMM_KERNEL_REGISTER = 2 };
 
+/* FP32 operands and results.  The products, like those of the implicit-GEMM
+ * convolutions and the larger Winograd layers, are six bf16 products of
+ * operands in three pieces with FP32 sums, which keeps every bit of an operand
+ * (denormals included) and leaves less than 2^-24 of a term out; operands that
+ * are infinite or from 2^112 up, and results from 2^96 up, make their output
+ * tile run again on FP32 matrix instructions.  A product of few tiles over a
+ * long K is split along K, its partials in at most 64 MiB of scratch; a call
+ * whose stream is being captured, or that finds no room, runs in one pass, so
+ * its sums round in another order than the split call's. */
 int mx_gemm_f32(const mx_gemm_desc* desc, const float* a, const float* b, const float* bias,
                 float* c, void* stream);
 

@@ -772,29 +772,24 @@ bool winograd_applicable(const mx_conv2d_desc& d) {
 
 // AUTO's Winograd rule for 3x3 stride-1 layers with at least 32 channels per
 // group on both sides, measured on MI355X per phase against the implicit GEMM
-// (kernel time of each algorithm forced).  On typical layers the fused
-// F(2x2,3x3) forward and input gradient take 0.50-0.89 of the implicit GEMM's
-// time (8x64 channels at 56^2: 17.8 vs 35.6 us; 16x128 at 64^2: 98 vs 184;
-// 16x512 at 8^2: 45.5 vs 60.0).  They lose where their channel walk (input
-// channels for the forward, output channels for the input gradient) is long
-// against the channels they produce, which sets their workgroup count, unless
-// the layer has many positions: 16x1024 at 16^2 to 32 takes 98.5 vs 54.1 us,
-// at 56^2 (8 images) 155 vs 254.  Over 401 layers per phase (batch 1-32,
-// 7^2-56^2, 32-1024 x 32-512 channels) the rule below (Winograd from 16384
-// positions, or from 512 when the walk is at most 4x the channels produced)
-// sums to 2.0% (forward) and 2.4% (input gradient) above the faster algorithm
-// per layer, a cut at 1024 positions to 6.7% and 4.6%.  The weight gradient's
-// break-even follows the layer's work, not its positions: in two sweeps (342
-// and 401 layers: batch 1-32, 7^2-56^2, 32-1024 input x 32-512 output
-// channels, kernel time of each algorithm forced) it wins from
-// 2^25 multiply-adds per filter tap (positions x input channels per group x
-// output channels; 16x512 at 8^2 to 512: 46 vs 73 us) and loses below
-// (8x32 at 16^2 to 64: 11.8 vs 10.5 us); summed over each sweep it costs
-// 0.7-0.8% more than the faster algorithm per layer, a 2048-position cut
-// 8-15% more.  This replaces the reference heuristic for these layers (its
-// Winograd is a grouped-layer forward rule, csrc/ops/convolution.cpp:454-460,
-// kept below); every other layer, and padding beyond 2, keeps the
-// reference's choices.
+// (kernel time of each algorithm forced) over 401 layers (batch 1-32, 7^2-56^2,
+// 32-1024 x 32-512 channels) and 70 random ones outside them.  Forward and input
+// gradient: Winograd from 16384 positions, or from 512 when the channel walk
+// (input channels for the forward, output channels for the input gradient) is at
+// most 4x the channels produced, which set the workgroup count.  Weight gradient:
+// its break-even follows the layer's work, so Winograd from 2^25 multiply-adds
+// per filter tap (positions x input channels per group x output channels).
+// The lines were drawn while both ran FP32 MFMA, where the rule summed to 2.0%,
+// 2.4% and 0.7% above the faster algorithm per layer (forward, input gradient,
+// weight gradient; random layers 1.4, 1.3 and 0.3).  With the split product and
+// walks in parts it is 5.9%, 5.4% and 1.0% (3.9, 3.4 and 4.1): long walks now
+// reach further down with Winograd (implicit GEMM / Winograd, forward: 16 x 1024
+// at 28^2 to 64 126 / 81 us, 8 x 1024 at 28^2 to 128 113 / 80; input gradient 16
+// x 64 at 28^2 to 512 70 / 51), and weight gradients of more work are faster as
+// implicit GEMMs (24 x 768 at 10 x 8 to 768 163 / 198).  This replaces the
+// reference heuristic for these layers (its Winograd is a grouped-layer forward
+// rule, csrc/ops/convolution.cpp:454-460, kept below); every other layer, and
+// padding beyond 2, keeps the reference's choices.
 bool winograd_auto(const mx_conv2d_desc& d, int phase) {
   if (!winograd_applicable(d) || d.ph > 2 || d.pw > 2 || d.cin / d.groups < 32 || d.cout / d.groups < 32)
     return false;
