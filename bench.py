@@ -423,8 +423,8 @@ def c4_kernel_table(tv, step, steps):
 def run_streams(torch, reps=5):
     """Copy / compute overlap on the "vulkan" device: a 256 MiB upload from
     page-locked host memory (non_blocking) on a copy stream beside two one-tile
-    GEMMs (64x64 output, K = 2^19: one workgroup for milliseconds) on a
-    compute stream, then two such GEMMs on two streams.  Each figure is the
+    GEMMs (64x64 output, K = 2^19 in one pass, MX_GEMM_TILE=3: one workgroup
+    for milliseconds) on a compute stream, then two such GEMMs on two streams.  Each figure is the
     best of `reps` runs timed on the host between device synchronisations."""
     import torch_vulkan as tv
 
@@ -456,10 +456,14 @@ def run_streams(torch, reps=5):
             with tv.stream(s):
                 a @ b
 
-    t_copy = timed(upload)
-    t_gemm = timed(lambda: gemms((s1, s1)))
-    t_both = timed(lambda: (upload(), gemms((s1, s1))))
-    t_two = timed(lambda: gemms((s1, s2)))
+    os.environ["MX_GEMM_TILE"] = "3"
+    try:
+        t_copy = timed(upload)
+        t_gemm = timed(lambda: gemms((s1, s1)))
+        t_both = timed(lambda: (upload(), gemms((s1, s1))))
+        t_two = timed(lambda: gemms((s1, s2)))
+    finally:
+        os.environ.pop("MX_GEMM_TILE", None)
     out = {"workload": "stream overlap: 256 MiB non_blocking upload from pinned memory on a copy stream beside "
                        "two one-tile GEMMs (64x64, K=2^19) on a compute stream; then the two GEMMs on two streams",
            "copy_ms": round(t_copy, 3), "h2d_gb_s": round(4 * (64 << 20) / (t_copy * 1e-3) / 1e9, 1),
