@@ -282,7 +282,8 @@ double tile_cost(const TileChoice& t, int64_t tiles, int64_t cu, int64_t m, int6
 // layer, split / one pass: 8 x 573 x 466 56.9 / 49.1 us, 256 x 512 x 512 57.8 /
 // 52.6, 8 x 1024 x 1024 54.7 / 56.6, 8 x 2048 x 1000 54.1 / 78.7; forward calls
 // on their own: 8 x 512 x 512 10.0 / 13.5, 8 x 768 x 768 10.0 / 18.9, 8 x 2048 x
-// 1000 11.1 / 45.3.
+// 1000 11.1 / 45.3.  Operands read as scalars take longer than the model has it:
+// 10 x 694 x 378, 13.9 us of it, runs for 23.5 us in one pass, 9.3 split.
 // `partials`: bytes they may take.  MX_GEMM_TILE=<index into kTiles> forces a
 // tile in one pass over K (tests and diagnosis; the 256-wide tiles only for
 // 16-byte operand modes).  `kernel` (mx_gemm_kernel) forces the 64x64 tile or
@@ -315,7 +316,7 @@ void pick_gemm_tile(int64_t m, int64_t n, int64_t k, int64_t batch, bool vec, in
       *tile = i;
     }
   }
-  if (partials <= 0 || best < kMinSplitTime) return;
+  if (partials <= 0 || best * (vec ? 1.0 : 1.1) < kMinSplitTime) return;
   static const int kSplits[] = {2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
   for (int i = first; i <= last; ++i) {
     const int64_t tiles = tiles_of(i);

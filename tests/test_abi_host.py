@@ -397,6 +397,7 @@ int main() {
 
 @pytest.mark.parametrize("m,n,k,split", [(8, 466, 573, False), (64, 512, 512, False), (2, 216, 512, False),
                                          (256, 512, 512, False), (8, 1000, 2048, True), (8, 1024, 1024, True),
+                                         (10, 378, 694, True), (10, 376, 692, False),
                                          (64, 64, 1 << 18, True), (8192, 4096, 4096, False)])
 def test_short_products_take_one_launch(mx, m, n, k, split):
     """K is split where one pass over it is long, not where the second launch
