@@ -54,7 +54,7 @@ MX_TILE_KERNEL(C) void gemm_kernel(GemmArgs p) {
   StridedLoader<C::BM, C::BK, MA> la;
   StridedLoader<C::BN, C::BK, MB> lb;
   Acc<C> acc;
-  const float scale = tile_product<C>(acc, la, lb, (k1 - k0 + C::BK - 1) / C::BK, smem, [&](auto& a, auto& b) {
+  const float scale = tile_product<C, true>(acc, la, lb, (k1 - k0 + C::BK - 1) / C::BK, smem, [&](auto& a, auto& b) {
     a.init(p.a + bz * p.a_sb, p.a_sm, p.a_sk, row0, p.M, k0, k1);
     b.init(p.b + bz * p.b_sb, p.b_sn, p.b_sk, col0, p.N, k0, k1);
   });
